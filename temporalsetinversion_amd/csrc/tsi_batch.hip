@@ -572,7 +572,9 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             J.t.visits = b->visits_d + njobs;
             J.t.shading = s.p.shading;
             J.t.grad = s.a.grad;
-            J.blocks_x = (r.width + 15u) / 16u;
+            J.t.mask = reinterpret_cast<const uint32_t *>(s.a.grad) + 3;
+            J.t.mask_stride = 4u;
+            J.blocks_x = (r.width + kTraceTile - 1u) / kTraceTile;
             b->job_of[i] = int32_t(njobs);
             s.w = r.width;
             s.h = r.height;
@@ -608,7 +610,7 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             const bool cin = (jb[j].t.shading & TSI_SHADE_CINEMATIC) != 0;
             uint32_t &acc = cin ? bcin : bplain;
             jb[j].block0 = acc;
-            acc += jb[j].blocks_x * ((jb[j].t.height + 15u) / 16u);
+            acc += jb[j].blocks_x * ((jb[j].t.height + kTraceTile - 1u) / kTraceTile);
             nplain += cin ? 0u : 1u;
         }
         HIP_OK(hipMemcpyAsync(b->jobs_d, b->jobs_h, njobs * sizeof(TraceJob), hipMemcpyHostToDevice, b->stream));

@@ -317,7 +317,20 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         if (ok) a.st[C] = make_float4(f, time, terr, __uint_as_float(cmeta));
         // dx/dy/dz: written by the reverse pass; zeroed when the node is allocated, so a
         // reused node never shows a previous occupant's values.
-        if (ok && (isnew || (REV && guard && td))) a.grad[C] = gradv;
+        // (the fourth word is the node's surface mask, which its own group keeps)
+        if (ok && isnew) a.grad[C] = gradv;
+        else if (REV && ok && guard && td) {
+            float *gd = reinterpret_cast<float *>(&a.grad[C]);
+            gd[0] = gradv.x;
+            gd[1] = gradv.y;
+            gd[2] = gradv.z;
+        }
+        // the parent's surface mask: which of its children a ray stops at (f <= 0)
+        {
+            const uint64_t surface = ballot(ok && f <= 0.0f);
+            if (ok && o == 0)
+                reinterpret_cast<uint32_t *>(&a.grad[P])[3] = uint32_t(surface >> (lane & 56u)) & 0xFFu;
+        }
 
         // ---- compaction of the outputs ----
         const bool next_fwd_only = !a.swept && !a.force_deriv &&

@@ -4,7 +4,8 @@
 //   st[n]   = {f, t, time_err, meta}   meta bit31 = fast, bits 0-30 = child block + 1 (0: leaf)
 //   blo[n]  = {x.lo, y.lo, z.lo, 0}    box
 //   bhi[n]  = {x.hi, y.hi, z.hi, 0}
-//   grad[n] = {dx, dy, dz, 0}          sensitivity midpoints (compute.wgsl:3967-3969)
+//   grad[n] = {dx, dy, dz, mask}       sensitivity midpoints (compute.wgsl:3967-3969); mask: bit o =
+//                                      child o has f <= 0 (a surface or inside: where rays stop)
 // Children of a node are one block of 8 consecutive nodes (child index x + 2y + 4z, the
 // numbering of compute.wgsl:3576 and 4295).  Node 0 is the root; block 0 holds only it.
 #pragma once
@@ -108,6 +109,8 @@ struct TraceArgs {
     unsigned long long *visits;
     uint32_t shading;           // TSI_SHADE_* (normal_viz, gradient normals, cinematic)
     const float4 *grad;         // the nodes' dx, dy, dz (gradient normals)
+    const uint32_t *mask;       // the nodes' surface masks (grad[n].w), mask_stride words apart
+    uint32_t mask_stride;
 };
 
 

@@ -42,18 +42,19 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
                  const hipEvent_t *e_level);
 int launch_reset(const KArgs &a, const float box[6], uint64_t nodes, hipStream_t s);
 int launch_enqueue_root(const KArgs &a, hipStream_t s);
+constexpr uint32_t kTraceTile = 16;   // a batched trace block's pixels: kTraceTile x kTraceTile
 // blocks > 0 (with next_quad, a counter zeroed on `s` before): the persistent form on that many
-// blocks (k_trace_quads); else one 16x16-pixel block per tile (k_trace)
+// blocks (k_trace_quads); else one block per tile (k_trace)
 int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blocks = 0, uint32_t *next_quad = nullptr);
-int launch_snapshot(const KArgs &a, float4 *s_st, float4 *s_blo, float4 *s_bhi, float4 *s_grad, uint64_t nodes,
-                    uint32_t grid, hipStream_t s);
+int launch_snapshot(const KArgs &a, float4 *s_st, float4 *s_blo, float4 *s_bhi, float4 *s_grad, uint32_t *s_mask,
+                    uint64_t nodes, uint32_t grid, hipStream_t s);
 int launch_rgba8(const float4 *in, uchar4 *out, uint32_t n, hipStream_t s);
 
 // One frame of a batched trace (k_trace_batch): the session's nodes and the frame's arguments.
 struct TraceJob {
     const float4 *st, *blo, *bhi, *grad;
     TraceArgs t;
-    uint32_t blocks_x;  // ceil(width / 16): 16x16-pixel blocks per row
+    uint32_t blocks_x;  // ceil(width / kTraceTile): blocks per row
     uint32_t block0;    // the frame's first block in the launch
 };
 // (cinematic: every job's session shades with TSI_SHADE_CINEMATIC; no job mixes the two)

@@ -139,6 +139,7 @@ struct tsi_ctx {
         unsigned long long *visits_h = nullptr;
         hipStream_t stream = nullptr;
         float4 *st = nullptr, *blo = nullptr, *bhi = nullptr;   // snapshot, voxel_capacity nodes
+        uint32_t *mask = nullptr;                               // surface masks
         float4 *grad = nullptr;                                 // gradient normals only
         float4 *rgba = nullptr;                                 // the frame it writes
         float *depth = nullptr;
@@ -375,7 +376,7 @@ void release(tsi_ctx *c) {
         for (hipEvent_t *e : {&t.begin, &t.end, &t.snap})
             if (*e) { hipEventDestroy(*e); *e = nullptr; }
         if (t.visits_h) { hipHostFree(t.visits_h); t.visits_h = nullptr; }
-        dfree(t.st); dfree(t.blo); dfree(t.bhi); dfree(t.grad); dfree(t.rgba); dfree(t.depth); dfree(t.visits);
+        dfree(t.st); dfree(t.blo); dfree(t.bhi); dfree(t.mask); dfree(t.grad); dfree(t.rgba); dfree(t.depth); dfree(t.visits);
         if (t.stream) { hipStreamDestroy(t.stream); t.stream = nullptr; }
     }
     dfree(c->st); dfree(c->blo); dfree(c->bhi); dfree(c->grad);
@@ -847,8 +848,15 @@ int harvest_all(tsi_ctx *c) {
 
 }  // namespace
 
-int tsi_trace_async(tsi_ctx *c) {
-    if (!c) return TSI_E_ARG;
+}  // extern "C"
+
+namespace {
+
+// Starts the trace of the current octree in the next trace slot.  overlap: over a device-side
+// snapshot of the nodes in use, on the slot's stream, beside the frames queued after it.  Without
+// it (the caller waits for the trace before it queues anything else) the octree itself is traced,
+// on the main stream, and always by the full launch: nothing runs beside it.
+int start_trace(tsi_ctx *c, bool overlap) {
     const uint32_t W = c->u.resolution[0], H = c->u.resolution[1];
     if (W == 0 || H == 0) return TSI_E_ARG;
     int rc;
@@ -864,22 +872,34 @@ int tsi_trace_async(tsi_ctx *c) {
         if ((rc = dmalloc(&ts.rgba, px)) || (rc = dmalloc(&ts.depth, px))) return rc;
         ts.px = px;
     }
-    if (!ts.st) {
-        if ((rc = dmalloc(&ts.st, c->nodes)) || (rc = dmalloc(&ts.blo, c->nodes)) || (rc = dmalloc(&ts.bhi, c->nodes))) {
-            dfree(ts.st); dfree(ts.blo); dfree(ts.bhi);
-            return rc;
-        }
-    }
     KArgs a = make_args(c);
-    // snapshot of the nodes in use, in stream order after the last set inversion
     const bool gradient_normals = (c->p.shading & (TSI_SHADE_NORMALS | TSI_SHADE_CINEMATIC)) && (c->p.shading & TSI_SHADE_GRADIENT);
-    if (gradient_normals && !ts.grad && (rc = dmalloc(&ts.grad, c->nodes))) return rc;
-    if (launch_snapshot(a, ts.st, ts.blo, ts.bhi, gradient_normals ? ts.grad : nullptr, c->nodes, c->grid_misc,
-                        c->stream) != 0)
-        return TSI_E_HIP;
-    HIP_OK(hipEventRecord(ts.snap, c->stream));
-    HIP_OK(hipStreamWaitEvent(ts.stream, ts.snap, 0));
+    const float4 *grad = gradient_normals ? c->grad : nullptr;
+    hipStream_t s = c->stream;
+    if (overlap) {
+        if (!ts.st) {
+            if ((rc = dmalloc(&ts.st, c->nodes)) || (rc = dmalloc(&ts.blo, c->nodes)) || (rc = dmalloc(&ts.bhi, c->nodes)) ||
+                (rc = dmalloc(&ts.mask, c->nodes))) {
+                dfree(ts.st); dfree(ts.blo); dfree(ts.bhi); dfree(ts.mask);
+                return rc;
+            }
+        }
+        // snapshot of the nodes in use, in stream order after the last set inversion
+        if (gradient_normals && !ts.grad && (rc = dmalloc(&ts.grad, c->nodes))) return rc;
+        if (launch_snapshot(a, ts.st, ts.blo, ts.bhi, gradient_normals ? ts.grad : nullptr, ts.mask, c->nodes,
+                            c->grid_misc, c->stream) != 0)
+            return TSI_E_HIP;
+        HIP_OK(hipEventRecord(ts.snap, c->stream));
+        HIP_OK(hipStreamWaitEvent(ts.stream, ts.snap, 0));
+        a.st = ts.st;
+        a.blo = ts.blo;
+        a.bhi = ts.bhi;
+        grad = ts.grad;
+        s = ts.stream;
+    }
     TraceArgs t{};
+    t.mask = overlap ? ts.mask : reinterpret_cast<const uint32_t *>(c->grad) + 3;
+    t.mask_stride = overlap ? 1u : 4u;
     std::memcpy(t.view, c->u.view, sizeof t.view);
     t.width = W;
     t.height = H;
@@ -889,16 +909,13 @@ int tsi_trace_async(tsi_ctx *c) {
     t.depth = ts.depth;
     t.visits = ts.visits;
     t.shading = c->p.shading;
-    t.grad = ts.grad;
-    a.st = ts.st;
-    a.blo = ts.blo;
-    a.bhi = ts.bhi;
-    HIP_OK(hipMemsetAsync(ts.visits, 0, 2 * sizeof(unsigned long long), ts.stream));
-    HIP_OK(hipEventRecord(ts.begin, ts.stream));
+    t.grad = grad;
+    HIP_OK(hipMemsetAsync(ts.visits, 0, 2 * sizeof(unsigned long long), s));
+    HIP_OK(hipEventRecord(ts.begin, s));
     uint32_t blocks = 0;
     if (c->trace_blocks_env >= 0) {
         blocks = uint32_t(c->trace_blocks_env) * uint32_t(c->num_cu);
-    } else if (c->last_si_ms > 0.0f && c->last_trace_ms > 0.0f) {
+    } else if (overlap && c->last_si_ms > 0.0f && c->last_trace_ms > 0.0f) {
         // the persistent form's expected time, from the last trace in either form (+/-10 %
         // hysteresis around the switch)
         const float tp = c->last_trace_persistent ? c->last_trace_ms : 1.15f * c->last_trace_ms;
@@ -907,13 +924,21 @@ int tsi_trace_async(tsi_ctx *c) {
         blocks = c->trace_persistent ? uint32_t(c->num_cu) : 0u;
     }
     ts.persistent = blocks != 0;
-    if (launch_trace(a, t, ts.stream, blocks, reinterpret_cast<uint32_t *>(ts.visits + 1)) != 0)
-        return TSI_E_HIP;
-    HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, sizeof(unsigned long long), hipMemcpyDeviceToHost, ts.stream));
-    HIP_OK(hipEventRecord(ts.end, ts.stream));
+    if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + 1)) != 0) return TSI_E_HIP;
+    HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    HIP_OK(hipEventRecord(ts.end, s));
     c->last_tslot = k;
     c->t_issued += 1;
     return TSI_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int tsi_trace_async(tsi_ctx *c) {
+    if (!c) return TSI_E_ARG;
+    return start_trace(c, true);
 }
 
 int tsi_trace_wait(tsi_ctx *c, float *rgba_out, float *depth_out) {
@@ -929,7 +954,8 @@ int tsi_trace_wait(tsi_ctx *c, float *rgba_out, float *depth_out) {
 }
 
 int tsi_trace(tsi_ctx *c, float *rgba_out, float *depth_out) {
-    int rc = tsi_trace_async(c);
+    if (!c) return TSI_E_ARG;
+    int rc = start_trace(c, false);
     if (rc) return rc;
     return tsi_trace_wait(c, rgba_out, depth_out);
 }
