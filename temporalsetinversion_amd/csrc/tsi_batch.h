@@ -32,6 +32,9 @@
 namespace tsi {
 
 constexpr uint32_t kBatchMaxSessions = 1024;
+// A phase's units are dealt to this many queues (unit u to queue u mod kClaimQueues), each claimed from
+// by the blocks of its group: one counter serves 83 claims per us over the chip (see kTallySlots).
+constexpr uint32_t kClaimQueues = 32;
 enum : uint32_t { kErrBarrier = 4u };   // a grid barrier timed out (the run is abandoned)
 
 struct BatchSession {
@@ -50,7 +53,8 @@ struct BatchCtl {
     uint32_t bar_count[16];               // grid barrier: arrivals since the run began
     uint32_t bar_gen[16];                 // barriers completed
     uint32_t error[16];                   // kErrBarrier
-    uint32_t claim[kMaxLevels + 4];       // work-queue heads, one per level phase
+    // work-queue heads per level phase, kClaimQueues of them, each in a line of its own
+    uint32_t claim[kMaxLevels + 4][kClaimQueues][32];
 };
 
 struct BatchArgs {
@@ -118,7 +122,7 @@ TSI_DI void batch_units(const BatchSession &S, int d, uint32_t &nr, uint32_t &nf
 
 // One dealloc unit: group g of the cascade's list `step` (dealloc_step's loop body).
 template <class KA>
-TSI_DI uint64_t dealloc_group(const KA &a, int step, uint32_t g) {
+TSI_DI uint32_t dealloc_group(const KA &a, int step, uint32_t g) {
     Counters *cnt = a.cnt;
     const uint32_t count = min(cnt->dlist_count[step], a.dlist_cap);
     const uint32_t *in = a.dlists[step & 1];
@@ -131,7 +135,7 @@ TSI_DI uint64_t dealloc_group(const KA &a, int step, uint32_t g) {
     const uint32_t m = active ? meta_of(a.st[blk * 8u + o]) & kChildMask : 0u;
     wave_append(m != 0, m - 1u, out, &cnt->dlist_count[step + 1], a.dlist_cap, &cnt->frame_error, kErrQueue);
     wave_append(active && o == 0, blk, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
-    return (active && o == 0) ? 1u : 0u;
+    return popc64(ballot(active && o == 0));
 }
 
 // The persistent kernel's body.  Tapes::group<REV>(tape, a, level, time, g, count, stk, tally)
@@ -174,13 +178,14 @@ TSI_DI void batch_run(const BatchArgs &b) {
 
     const uint32_t lane = lane_id();
     const uint32_t wpb = blockDim.x >> 6;   // wavefronts per block
-    const uint32_t nwaves = nb * wpb;
     const uint32_t bwave = __builtin_amdgcn_readfirstlane(blockIdx.x * wpb + (tid >> 6));
     float2 *stk = b.stack + size_t(bwave) * b.stack_len * 64u;
     const uint32_t cu = b.claim_units;
-    // the first round's units go to the blocks in turn (wavefront w of block i takes slot
-    // w * nb + i), so that a phase of a few units runs on as many CUs
-    const uint32_t slot = __builtin_amdgcn_readfirstlane((tid >> 6) * nb + blockIdx.x);
+    // the block's queue, and the wavefront's place among the queue's: in the first round units go to
+    // the queue's blocks in turn, so that a phase of a few units runs on as many CUs
+    const uint32_t nq = min(kClaimQueues, nb), q = blockIdx.x % nq;
+    const uint32_t qblocks = (nb - q + nq - 1u) / nq, qwaves = qblocks * wpb;
+    const uint32_t slot = __builtin_amdgcn_readfirstlane((tid >> 6) * qblocks + blockIdx.x / nq);
 
     for (int d = b.first_phase; d < b.phases; ++d) {
         // ---- the phase's unit table (every block builds the same one) ----
@@ -206,12 +211,15 @@ TSI_DI void batch_run(const BatchArgs &b) {
         }
         const uint32_t total = pre[m];
 
-        // ---- units: in the first round wavefront slot i takes unit i; then wavefronts claim cu
-        //      units at a time from the phase's counter, which hands out units from nwaves on
-        //      (a phase of no more units than wavefronts takes no atomic) ----
-        for (uint32_t base = slot, take = 1u; base < total; take = cu) {
-            const uint32_t end = min(base + take, total);
-            for (uint32_t u = base; u < end; ++u) {
+        // ---- the queue's units (q, q + nq, q + 2 nq, ..): in the first round wavefront slot i takes
+        //      unit i of the queue; then wavefronts claim cu units at a time from the queue's counter,
+        //      which hands out units from qwaves on (a queue of no more units than wavefronts takes no
+        //      atomic) ----
+        const uint32_t qlen = total > q ? (total - q + nq - 1u) / nq : 0u;
+        for (uint32_t base = slot, take = 1u; base < qlen; take = cu) {
+            const uint32_t end = min(base + take, qlen);
+            for (uint32_t i = base; i < end; ++i) {
+                const uint32_t u = q + nq * i;
                 // segment j with pre[j] <= u < pre[j + 1]
                 uint32_t lo = 0, hi = m;
                 while (hi - lo > 1u) {
@@ -235,12 +243,12 @@ TSI_DI void batch_run(const BatchArgs &b) {
                     Tapes::template group<false>(tape, a, d, time, g, list_entries(a, d, 0), stk, tl);
                 else
                     tl.freed = dealloc_group(a, d, g);
-                flush_tally(a.cnt, tl);
+                flush_tally(a.tally, tl);
             }
-            if (nwaves >= total) break;
+            if (qwaves >= qlen) break;
             uint32_t next = 0;
-            if (lane == 0) next = atomicAdd(&b.ctl->claim[d + 1], cu);
-            base = __builtin_amdgcn_readfirstlane(bcast(next, 0)) + nwaves;
+            if (lane == 0) next = atomicAdd(&b.ctl->claim[d + 1][q][0], cu);
+            base = __builtin_amdgcn_readfirstlane(bcast(next, 0)) + qwaves;
         }
         if (!grid_sync(b, gen)) return;
     }
@@ -250,11 +258,15 @@ TSI_DI void batch_run(const BatchArgs &b) {
     if (!grid_sync(b, gen)) return;
     // commit, the frame's counters for the host, and buf_main: the root re-enqueued for the
     // session's next frame (compute.wgsl:4690-4707)
-    for (uint32_t s = blockIdx.x * blockDim.x + tid; s < ns; s += nb * blockDim.x) {
+    // (a wavefront per session)
+    for (uint32_t s = blockIdx.x * wpb + (tid >> 6); s < ns; s += nb * wpb) {
         const KArgs &a = b.sess[s].a;
         frame_commit(a);
-        b.out[s] = *a.cnt;
-        a.cnt->root_pending = 1u;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the lanes' writes, for the copy below
+        const uint32_t *from = reinterpret_cast<const uint32_t *>(a.cnt);
+        uint32_t *to = reinterpret_cast<uint32_t *>(b.out + s);
+        for (uint32_t i = lane; i < uint32_t(sizeof(Counters) / 4); i += 64u) to[i] = from[i];
+        if (lane == 0) a.cnt->root_pending = 1u;
     }
 }
 

@@ -129,6 +129,7 @@ struct tsi_batch {
     Counters *out_d = nullptr, *out_h = nullptr;
     TraceJob *jobs_d = nullptr, *jobs_h = nullptr;
     unsigned long long *visits_d = nullptr, *visits_h = nullptr;
+    uint64_t *tally = nullptr;                  // each session's statistics (KArgs::tally)
     char *arena = nullptr;
     uint64_t arena_bytes = 0, arena_used = 0;
     std::map<uint64_t, uint64_t> free_ranges;   // offset -> bytes
@@ -182,7 +183,7 @@ void release(tsi_batch *b) {
     if (b->mod) hipModuleUnload(b->mod);
     b->mod = nullptr;
     dfree(b->stack); dfree(b->sess_d); dfree(b->ctl); dfree(b->out_d); dfree(b->jobs_d);
-    dfree(b->visits_d); dfree(b->arena);
+    dfree(b->visits_d); dfree(b->tally); dfree(b->arena);
     hfree(b->sess_h); hfree(b->out_h); hfree(b->jobs_h); hfree(b->visits_h);
     for (auto &e : b->ev)
         if (e) { hipEventDestroy(e); e = nullptr; }
@@ -235,6 +236,7 @@ void session_args(const tsi_batch *b, Session &s, const Layout &L) {
     a.pending_free = reinterpret_cast<uint32_t *>(base + L.pending);
     a.free_stack = reinterpret_cast<uint32_t *>(base + L.free_stack);
     a.cnt = reinterpret_cast<Counters *>(base + L.cnt);
+    a.tally = b->tally + size_t(&s - b->sessions.data()) * kTallySlots * kTallyStride;
     a.stack = nullptr;
     const Lowered &low = b->low[s.tape];
     a.nfwd = low.nfwd;
@@ -384,9 +386,11 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
         if ((rc = dmalloc(&b->stack, stack_elems)) || (rc = dmalloc(&b->sess_d, C.max_sessions)) ||
             (rc = dmalloc(&b->ctl, 1)) ||
             (rc = dmalloc(&b->out_d, C.max_sessions)) || (rc = dmalloc(&b->jobs_d, C.max_sessions)) ||
-            (rc = dmalloc(&b->visits_d, C.max_sessions)) || (rc = hmalloc(&b->sess_h, C.max_sessions)) ||
+            (rc = dmalloc(&b->visits_d, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)) ||
+            (rc = dmalloc(&b->tally, size_t(C.max_sessions) * kTallySlots * kTallyStride)) ||
+            (rc = hmalloc(&b->sess_h, C.max_sessions)) ||
             (rc = hmalloc(&b->out_h, C.max_sessions)) || (rc = hmalloc(&b->jobs_h, C.max_sessions)) ||
-            (rc = hmalloc(&b->visits_h, C.max_sessions)))
+            (rc = hmalloc(&b->visits_h, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)))
             break;
         uint64_t arena = C.arena_bytes;
         if (arena == 0) {
@@ -569,7 +573,8 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             J.t.zdist = tsi_camera_zdist(r.height);
             J.t.rgba = s.rgba;
             J.t.depth = s.depth;
-            J.t.visits = b->visits_d + njobs;
+            J.t.visits = b->visits_d + size_t(njobs) * kBatchVisitSlots * kTallyStride;
+            J.t.visit_slots = kBatchVisitSlots;
             J.t.shading = s.p.shading;
             J.t.grad = s.a.grad;
             J.t.mask = reinterpret_cast<const uint32_t *>(s.a.grad) + 3;
@@ -614,12 +619,13 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             nplain += cin ? 0u : 1u;
         }
         HIP_OK(hipMemcpyAsync(b->jobs_d, b->jobs_h, njobs * sizeof(TraceJob), hipMemcpyHostToDevice, b->stream));
-        if (launch_fill_u32(reinterpret_cast<uint32_t *>(b->visits_d), 0u, 2u * njobs, b->stream)) return TSI_E_HIP;
+        if (launch_fill_u32(reinterpret_cast<uint32_t *>(b->visits_d), 0u, 2u * njobs * kBatchVisitSlots * kTallyStride, b->stream)) return TSI_E_HIP;
         HIP_OK(hipEventRecord(b->ev[2], b->stream));
         if (nplain && launch_trace_batch(b->jobs_d, nplain, bplain, false, b->stream)) return TSI_E_HIP;
         if (nplain < njobs && launch_trace_batch(b->jobs_d + nplain, njobs - nplain, bcin, true, b->stream))
             return TSI_E_HIP;
-        HIP_OK(hipMemcpyAsync(b->visits_h, b->visits_d, njobs * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+        HIP_OK(hipMemcpyAsync(b->visits_h, b->visits_d,
+                              size_t(njobs) * kBatchVisitSlots * kTallyStride * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                               b->stream));
     }
     HIP_OK(hipMemcpyAsync(b->out_h, b->out_d, n * sizeof(Counters), hipMemcpyDeviceToHost, b->stream));
@@ -673,7 +679,9 @@ int tsi_batch_wait(tsi_batch *b, tsi_frame_result *results, double *set_ms, doub
         r.stats.allocated_nodes = h.stats[kStatLive] * 8u;
         r.stats.eval_launches = 1;
         r.stats.eval_kernel_ms = sms;
-        if (b->job_of[i] >= 0) r.node_visits = b->visits_h[b->job_of[i]];
+        if (b->job_of[i] >= 0)
+            for (uint32_t k = 0; k < kBatchVisitSlots; ++k)
+                r.node_visits += b->visits_h[(size_t(b->job_of[i]) * kBatchVisitSlots + k) * kTallyStride];
     }
     return ctl.error[0] ? TSI_E_HIP : TSI_OK;
 }

@@ -32,15 +32,15 @@ namespace tsi {
 // One step of the dealloc cascade (compute.wgsl:3533-3543) over list `step` (buffer step & 1):
 // every node of a freed block that has children passes its child block on to list step + 1,
 // and the block goes to the pending free list.  A wavefront takes 8 blocks (lane = 8 * block
-// slot + node).  Returns this lane's count of freed blocks.
-TSI_DI uint64_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t nwaves) {
+// slot + node).  Returns the wavefront's count of freed blocks.
+TSI_DI uint32_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t nwaves) {
     Counters *cnt = a.cnt;
     const uint32_t count = min(cnt->dlist_count[step], a.dlist_cap);
     const uint32_t *in = a.dlists[step & 1];
     uint32_t *out = a.dlists[(step + 1) & 1];
     const uint32_t lane = lane_id();
     const uint32_t o = lane & 7u;
-    uint64_t freed = 0;
+    uint32_t freed = 0;
     for (uint32_t g = wave; g * 8u < count; g += nwaves) {
         const uint32_t idx = g * 8u + (lane >> 3);
         const bool active = idx < count;
@@ -48,15 +48,16 @@ TSI_DI uint64_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t n
         const uint32_t m = active ? meta_of(a.st[b * 8u + o]) & kChildMask : 0u;
         wave_append(m != 0, m - 1u, out, &cnt->dlist_count[step + 1], a.dlist_cap, &cnt->frame_error, kErrQueue);
         wave_append(active && o == 0, b, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
-        freed += (active && o == 0) ? 1 : 0;
+        freed += popc64(ballot(active && o == 0));
     }
     return freed;
 }
 
-// Per-lane tallies of the cells a wavefront processed, summed over the wavefront and added to
-// the counters once (flush_tally).
+// A wavefront's tallies of the cells it processed: counts of its lanes (uniform, from ballots) and
+// per-lane sums of work; added to the frame's statistics once (flush_tally).
 struct LevelTally {
-    uint64_t cells = 0, rev = 0, par = 0, enq = 0, rev_ops = 0, fwd_ops = 0, pruned = 0, freed = 0, spec = 0;
+    uint32_t cells = 0, rev = 0, par = 0, enq = 0, freed = 0, spec = 0;
+    uint64_t rev_ops = 0, fwd_ops = 0, pruned = 0;
 };
 
 // Frontier entries of one list at a level (a list that overflowed, flagged by wave_append,
@@ -124,7 +125,7 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             if (o == 0) atomicOr(&cnt->frame_error, kErrPool);
         }
         if (!sp && isnew && ok && o == 0) a.st[P].w = __uint_as_float((pmeta & kFastBit) | (blk + 1u));
-        if (!sp) tl.par += (active && o == 0) ? 1 : 0;
+        if (!sp) tl.par += popc64(ballot(active && o == 0));
 
         const uint32_t C = ok && !(sp && isnew) ? blk * 8u + o : 0u;
         float4 cst = make_float4(1.0f, 0.0f, 0.0f, 0.0f);   // mallocV (compute.wgsl:3437-3449)
@@ -335,10 +336,9 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         // ---- compaction of the outputs ----
         const bool next_fwd_only = !a.swept && !a.force_deriv &&
                                    ((cmeta & kChildMask) == 0 || (cmeta & kFastBit) || width / 2.0f <= eps);
-        const uint32_t at_f = wave_append(enq && next_fwd_only, C, next_f, &cnt->list_count[level + 1][0],
-                                          a.list_cap, &cnt->frame_error, kErrQueue);
-        const uint32_t at_r = wave_append(enq && !next_fwd_only, C, next_r, &cnt->list_count[level + 1][1],
-                                          a.list_cap, &cnt->frame_error, kErrQueue);
+        uint32_t at_f, at_r;
+        wave_append2(enq && next_fwd_only, enq && !next_fwd_only, C, next_f, next_r, cnt->list_count[level + 1],
+                     a.list_cap, &cnt->frame_error, kErrQueue, at_f, at_r);
         // dropped blocks are freed by the next level's forward-only kernel (the dealloc step
         // below), their descendants by the levels after it
         wave_append(drop_children, old_child - 1u, a.dlists[(level + 1) & 1], &cnt->dlist_count[level + 1], a.dlist_cap,
@@ -358,29 +358,31 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             if (!valid) rec = nullptr;
             if (ballot(rec != nullptr) != 0) E.liveness(a, rec);
         }
-        tl.cells += guard ? 1 : 0;
-        tl.spec += have ? 1 : 0;
-        tl.rev += (guard && td) ? 1 : 0;
-        tl.enq += enq ? 1 : 0;
+        tl.cells += popc64(ballot(guard));
+        tl.spec += popc64(ballot(have));
+        tl.rev += popc64(ballot(guard && td));
+        tl.enq += popc64(ballot(enq));
     }
 }
 
-// Adds a wavefront's tallies to the counters: one atomic per statistic.
-TSI_DI void flush_tally(Counters *cnt, const LevelTally &t) {
-    const uint64_t n_cells = wave_sum64(t.cells), n_rev = wave_sum64(t.rev), n_par = wave_sum64(t.par),
-                   n_enq = wave_sum64(t.enq), rev_ops = wave_sum64(t.rev_ops), fwd_ops = wave_sum64(t.fwd_ops),
-                   n_pruned = wave_sum64(t.pruned), n_freed = wave_sum64(t.freed), n_spec = wave_sum64(t.spec);
-    if (lane_id() == 0) {
-        if (n_cells) atomicAdd((unsigned long long *)&cnt->stats[kStatCells], (unsigned long long)n_cells);
-        if (n_rev) atomicAdd((unsigned long long *)&cnt->stats[kStatRevCells], (unsigned long long)n_rev);
-        if (n_par) atomicAdd((unsigned long long *)&cnt->stats[kStatParents], (unsigned long long)n_par);
-        if (n_enq) atomicAdd((unsigned long long *)&cnt->stats[kStatEnqueued], (unsigned long long)n_enq);
-        if (rev_ops) atomicAdd((unsigned long long *)&cnt->stats[kStatRevOps], (unsigned long long)rev_ops);
-        if (fwd_ops) atomicAdd((unsigned long long *)&cnt->stats[kStatFwdOps], (unsigned long long)fwd_ops);
-        if (n_pruned) atomicAdd((unsigned long long *)&cnt->stats[kStatPruned], (unsigned long long)n_pruned);
-        if (n_freed) atomicAdd((unsigned long long *)&cnt->stats[kStatDeallocs], (unsigned long long)n_freed);
-        if (n_spec) atomicAdd((unsigned long long *)&cnt->stats[kStatSpec], (unsigned long long)n_spec);
-    }
+// Adds a wavefront's tallies to the block's slot of the frame's statistics: one atomic instruction,
+// lane k adding statistic k.
+TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t) {
+    const uint64_t rev_ops = wave_sum64(t.rev_ops), fwd_ops = wave_sum64(t.fwd_ops), pruned = wave_sum64(t.pruned);
+    const uint32_t k = lane_id();
+    uint64_t v = 0;
+    v = k == kStatCells ? t.cells : v;
+    v = k == kStatRevCells ? t.rev : v;
+    v = k == kStatParents ? t.par : v;
+    v = k == kStatEnqueued ? t.enq : v;
+    v = k == kStatRevOps ? rev_ops : v;
+    v = k == kStatDeallocs ? t.freed : v;
+    v = k == kStatFwdOps ? fwd_ops : v;
+    v = k == kStatPruned ? pruned : v;
+    v = k == kStatSpec ? t.spec : v;
+    if (v)
+        atomicAdd(reinterpret_cast<unsigned long long *>(tally + (blockIdx.x % kTallySlots) * kTallyStride + k),
+                  (unsigned long long)v);
 }
 
 // One level of one frontier list: wavefront `wave` of `nwaves` strides over the list; `bwave`
@@ -406,7 +408,7 @@ TSI_DI void eval_level(const KArgs &a, int level, float time, uint32_t wave_, ui
     //      descendants (forward-only kernel; the reverse kernel of the level does not touch the
     //      list, which the previous level's kernels finished) ----
     if (!REV && level > 0) tl.freed = dealloc_step(a, level, wave, nwaves);
-    flush_tally(a.cnt, tl);
+    flush_tally(a.tally, tl);
 }
 
 // The speculative pass's parents (KArgs::spec_*): every node at depth < spec_levels as the frame
@@ -461,7 +463,7 @@ TSI_DI void frame_begin(const KArgs &a, uint32_t t, uint32_t nt) {
         c->list_count[i][1] = 0;
         c->dlist_count[i] = 0;
     }
-    for (uint32_t i = t; i < uint32_t(kNumStats); i += nt) c->stats[i] = 0;
+    for (uint32_t i = t; i < kTallySlots * kTallyStride; i += nt) a.tally[i] = 0;
     for (uint32_t i = t; i < uint32_t(kMaxLevels + 2); i += nt) c->pool_used[i] = 0;
     if (t == 0) {
         c->alloc_tickets = 0;
@@ -492,9 +494,17 @@ TSI_DI void frame_end(const KArgs &a, uint32_t t, uint32_t nt) {
     for (uint32_t i = t; i < P && base + i < a.nblocks; i += nt) a.free_stack[base + i] = a.pending_free[i];
 }
 
-// After frame_end has finished everywhere: the allocator's new state (one thread).
+// After frame_end has finished everywhere: the frame's statistics, summed over the tally's slots, and
+// the allocator's new state (one wavefront; lane k sums statistic k).
 TSI_DI void frame_commit(const KArgs &a) {
     Counters *cnt = a.cnt;
+    const uint32_t k = lane_id();
+    if (k < uint32_t(kNumStats) && k != uint32_t(kStatLive)) {
+        uint64_t v = 0;
+        for (uint32_t i = 0; i < kTallySlots; ++i) v += a.tally[i * kTallyStride + k];
+        cnt->stats[k] = v;
+    }
+    if (k != 0) return;
     const uint32_t T = cnt->alloc_tickets, F = cnt->free_top, P = min(cnt->pending, a.nblocks);
     const uint32_t used = T < F ? T : F;
     uint32_t bump = cnt->bump + (T > F ? T - F : 0u);

@@ -138,8 +138,9 @@ __global__ void __launch_bounds__(256) k_prune(KArgs a, int level, int which) {
 __global__ void __launch_bounds__(256) k_dealloc(KArgs a, int step) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
-    uint64_t freed = wave_sum64(dealloc_step(a, step, wave, nwaves));
-    if (lane_id() == 0 && freed) atomicAdd((unsigned long long *)&a.cnt->stats[kStatDeallocs], (unsigned long long)freed);
+    LevelTally tl;
+    tl.freed = dealloc_step(a, step, wave, nwaves);
+    if (tl.freed) flush_tally(a.tally, tl);
 }
 
 // Free-list merge and counter commit at the end of a frame (frame_end / frame_commit, tsi_eval.h).
@@ -220,7 +221,7 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
             return -1;
         hipEventRecord(sp->done, sp->stream);
     }
-    hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(256), 0, s, a);
     if (sp) hipStreamWaitEvent(s, sp->done, 0);
     if (e_eval0) hipEventRecord(e_eval0, s);
     for (int d = 0; d < fl.levels; ++d) {
@@ -255,7 +256,7 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
     for (int c = fl.levels; c <= fl.levels + 1; ++c)
         hipLaunchKernelGGL(k_dealloc, dim3(fl.grid_misc), dim3(256), 0, s, a, c);
     hipLaunchKernelGGL(k_frame_end, dim3(fl.grid_misc), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_frame_commit, dim3(1), dim3(1), 0, s, a);
+    hipLaunchKernelGGL(k_frame_commit, dim3(1), dim3(64), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

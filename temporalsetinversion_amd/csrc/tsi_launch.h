@@ -43,7 +43,9 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
 int launch_reset(const KArgs &a, const float box[6], uint64_t nodes, hipStream_t s);
 int launch_enqueue_root(const KArgs &a, hipStream_t s);
 constexpr uint32_t kTraceTile = 16;   // a batched trace block's pixels: kTraceTile x kTraceTile
-// blocks > 0 (with next_quad, a counter zeroed on `s` before): the persistent form on that many
+// claim counters of the persistent trace, each in a line of its own (2 * kTallyStride uint32 apart)
+constexpr uint32_t kTraceQueues = 8;
+// blocks > 0 (with next_quad, kTraceQueues counters zeroed on `s` before): the persistent form on that many
 // blocks (k_trace_quads); else one block per tile (k_trace)
 int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blocks = 0, uint32_t *next_quad = nullptr);
 int launch_snapshot(const KArgs &a, float4 *s_st, float4 *s_blo, float4 *s_bhi, float4 *s_grad, uint32_t *s_mask,

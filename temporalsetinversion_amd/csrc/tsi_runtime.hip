@@ -57,6 +57,10 @@ int scratch_setup(int device, uchar4 **out) {
 
 }  // namespace
 
+// A trace slot's counters: the node visits (TraceArgs::visits), then the persistent trace's claims.
+constexpr size_t kVisitBytes = size_t(tsi::kVisitSlots) * tsi::kTallyStride * sizeof(unsigned long long);
+constexpr size_t kTraceCounters = size_t(tsi::kVisitSlots + tsi::kTraceQueues) * tsi::kTallyStride;
+
 struct tsi_ctx {
     tsi_params p{};
     int device = 0;
@@ -71,6 +75,7 @@ struct tsi_ctx {
     uint32_t *dlists[2] = {nullptr, nullptr};
     uint32_t *pending = nullptr, *free_stack = nullptr;
     Counters *cnt = nullptr;
+    uint64_t *tally = nullptr;          // KArgs::tally
     float2 *stack = nullptr;
     size_t stack_bytes = 0;
     FwdIns *fprog = nullptr;
@@ -199,6 +204,7 @@ KArgs make_args(const tsi_ctx *c) {
     a.pending_free = c->pending;
     a.free_stack = c->free_stack;
     a.cnt = c->cnt;
+    a.tally = c->tally;
     a.stack = c->stack;
     a.fprog = c->fprog;
     a.rprog = c->rprog;
@@ -382,7 +388,7 @@ void release(tsi_ctx *c) {
     dfree(c->st); dfree(c->blo); dfree(c->bhi); dfree(c->grad);
     for (auto &l : c->lists) for (auto &x : l) dfree(x);
     dfree(c->dlists[0]); dfree(c->dlists[1]);
-    dfree(c->pending); dfree(c->free_stack); dfree(c->cnt); dfree(c->stack);
+    dfree(c->pending); dfree(c->free_stack); dfree(c->cnt); dfree(c->tally); dfree(c->stack);
     dfree(c->spec_list); dfree(c->spec_cnt); dfree(c->spec_res); dfree(c->spec_stack);
     if (c->spec_ready) { hipEventDestroy(c->spec_ready); c->spec_ready = nullptr; }
     if (c->spec_stream) { hipStreamDestroy(c->spec_stream); c->spec_stream = nullptr; }
@@ -525,7 +531,7 @@ int tsi_create(const tsi_params *params, tsi_ctx **out) {
         }
         for (auto &t : c->tslot) {
             for (hipEvent_t *e : {&t.begin, &t.end}) evok = evok && hipEventCreate(e) == hipSuccess;
-            evok = evok && hipHostMalloc((void **)&t.visits_h, sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess;
+            evok = evok && hipHostMalloc((void **)&t.visits_h, kVisitBytes, hipHostMallocDefault) == hipSuccess;
         }
         if (!evok) { rc = TSI_E_HIP; break; }
         uint64_t nodes = params->voxel_capacity ? params->voxel_capacity : (uint64_t(1) << 24);
@@ -563,10 +569,10 @@ int tsi_create(const tsi_params *params, tsi_ctx **out) {
             break;
         if ((rc = dmalloc(&c->dlists[0], c->dlist_cap)) || (rc = dmalloc(&c->dlists[1], c->dlist_cap)) ||
             (rc = dmalloc(&c->pending, c->nblocks)) || (rc = dmalloc(&c->free_stack, c->nblocks)) ||
-            (rc = dmalloc(&c->cnt, 1)))
+            (rc = dmalloc(&c->cnt, 1)) || (rc = dmalloc(&c->tally, size_t(kTallySlots) * kTallyStride)))
             break;
         for (auto &t : c->tslot)
-            if (!rc) rc = dmalloc(&t.visits, 2);   // the visit count, then the persistent trace's quad counter
+            if (!rc) rc = dmalloc(&t.visits, kTraceCounters);
         if (rc) break;
         if (hipMemsetAsync(c->cnt, 0, sizeof(Counters), c->stream) != hipSuccess) { rc = TSI_E_HIP; break; }
         // level kernels stride over their frontier; 4 blocks (16 wavefronts) per CU for both lists
@@ -830,11 +836,13 @@ int harvest_trace(tsi_ctx *c) {
     HIP_OK(hipEventSynchronize(t.end));
     float tms = 0.0f;
     hipEventElapsedTime(&tms, t.begin, t.end);
-    c->last_visits = *t.visits_h;
+    uint64_t visits = 0;
+    for (uint32_t k = 0; k < kVisitSlots; ++k) visits += t.visits_h[k * kTallyStride];
+    c->last_visits = visits;
     c->last_trace_ms = tms;
     c->last_trace_persistent = t.persistent;
     c->trace_ms_total += tms;
-    c->trace_visits_total += *t.visits_h;
+    c->trace_visits_total += visits;
     c->trace_count += 1;
     return TSI_OK;
 }
@@ -910,7 +918,8 @@ int start_trace(tsi_ctx *c, bool overlap) {
     t.visits = ts.visits;
     t.shading = c->p.shading;
     t.grad = grad;
-    HIP_OK(hipMemsetAsync(ts.visits, 0, 2 * sizeof(unsigned long long), s));
+    t.visit_slots = kVisitSlots;
+    HIP_OK(hipMemsetAsync(ts.visits, 0, kTraceCounters * sizeof(unsigned long long), s));
     HIP_OK(hipEventRecord(ts.begin, s));
     uint32_t blocks = 0;
     if (c->trace_blocks_env >= 0) {
@@ -924,8 +933,8 @@ int start_trace(tsi_ctx *c, bool overlap) {
         blocks = c->trace_persistent ? uint32_t(c->num_cu) : 0u;
     }
     ts.persistent = blocks != 0;
-    if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + 1)) != 0) return TSI_E_HIP;
-    HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + kVisitSlots * kTallyStride)) != 0) return TSI_E_HIP;
+    HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, kVisitBytes, hipMemcpyDeviceToHost, s));
     HIP_OK(hipEventRecord(ts.end, s));
     c->last_tslot = k;
     c->t_issued += 1;

@@ -842,7 +842,8 @@ TSI_DI void shade_tile(const KArgs &a, const TraceArgs &t, uint32_t x0, uint32_t
 template <class G>
 TSI_DI void add_visits(const TraceArgs &t, uint32_t visits) {
     const uint64_t v = wave_sum64(G::counts() ? visits : 0u);
-    if (lane_id() == 0 && v) atomicAdd((unsigned long long *)t.visits, (unsigned long long)v);
+    const uint32_t slot = (blockIdx.x + blockIdx.y * 5u) & (t.visit_slots - 1u);
+    if (lane_id() == 0 && v) atomicAdd((unsigned long long *)t.visits + slot * kTallyStride, (unsigned long long)v);
 }
 
 }  // namespace
@@ -860,7 +861,7 @@ __global__ void __launch_bounds__(256) k_trace(KArgs a, TraceArgs t) {
 }
 
 // The same pixels on a grid of a few blocks per CU: each wavefront claims 8x8-pixel quadrants
-// (row-major over the frame) from a counter until none is left.  A full launch keeps every CU's
+// (row-major over the frame, dealt to kTraceQueues counters) until none is left.  A full launch keeps every CU's
 // wave slots filled with trace wavefronts while any block is pending, so the next frame's level
 // kernels, launched beside it, wait for slots; this leaves the CUs most of their slots.  Each pixel
 // is shaded by the same code as in k_trace: the frame is the same.
@@ -868,11 +869,12 @@ template <bool CIN>
 __global__ void __launch_bounds__(256) k_trace_quads(KArgs a, TraceArgs t, uint32_t *next_quad, uint32_t quads_x,
                                                      uint32_t nquads) {
     __shared__ uint2 stack_lds[kStackDepth * 256u];
+    const uint32_t queue = blockIdx.x % kTraceQueues;
     uint32_t visits = 0;
     for (;;) {
         uint32_t q = 0;
-        if (lane_id() == 0) q = atomicAdd(next_quad, 1u);
-        q = __builtin_amdgcn_readfirstlane(q);
+        if (lane_id() == 0) q = atomicAdd(next_quad + queue * 2u * kTallyStride, 1u);
+        q = __builtin_amdgcn_readfirstlane(q) * kTraceQueues + queue;
         if (q >= nquads) break;
         shade_tile<LaneG, CIN>(a, t, (q % quads_x) * 8u, (q / quads_x) * 8u, LaneG::Stack{stack_lds + threadIdx.x}, visits);
     }
@@ -912,6 +914,7 @@ __global__ void __launch_bounds__(256) k_trace_batch(const TraceJob *jobs, uint3
     t.grad = J.t.grad;
     t.mask = J.t.mask;
     t.mask_stride = J.t.mask_stride;
+    t.visit_slots = J.t.visit_slots;
     const uint32_t local = blk - J.block0;
     const uint32_t w = threadIdx.x >> 6;
     uint32_t visits = 0;
@@ -937,7 +940,7 @@ int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blo
     const bool cin = (t.shading & TSI_SHADE_CINEMATIC) != 0;
     if (blocks && next_quad) {   // persistent: `blocks` blocks, *next_quad zeroed on the stream before
         const uint32_t qx = (t.width + 7u) / 8u, nq = qx * ((t.height + 7u) / 8u);
-        const uint32_t nb = std::min(blocks, (nq + 3u) / 4u);
+        const uint32_t nb = std::min(blocks, std::max(kTraceQueues, (nq + 3u) / 4u));   // (a block for every queue)
         if (cin) hipLaunchKernelGGL(k_trace_quads<true>, dim3(nb), dim3(256), 0, s, a, t, next_quad, qx, nq);
         else hipLaunchKernelGGL(k_trace_quads<false>, dim3(nb), dim3(256), 0, s, a, t, next_quad, qx, nq);
         return hipGetLastError() == hipSuccess ? 0 : -1;

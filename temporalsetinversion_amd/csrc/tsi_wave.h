@@ -33,6 +33,30 @@ TSI_DI uint32_t wave_append(bool p, uint32_t value, uint32_t *list, uint32_t *cn
     return at;
 }
 
+// Appends to two lists at once: lanes with pf to list_f, lanes with pr to list_r (never both), their
+// counts side by side at cnt[0 .. 1] (8-byte aligned): one atomic per wavefront for the two.
+TSI_DI void wave_append2(bool pf, bool pr, uint32_t value, uint32_t *list_f, uint32_t *list_r, uint32_t *cnt,
+                         uint32_t cap, uint32_t *err, uint32_t errbit, uint32_t &at_f, uint32_t &at_r) {
+    const uint64_t mf = ballot(pf), mr = ballot(pr);
+    at_f = at_r = 0xFFFFFFFFu;
+    if ((mf | mr) == 0) return;
+    unsigned long long base = 0;
+    if (lane_id() == 0)
+        base = atomicAdd(reinterpret_cast<unsigned long long *>(cnt),
+                         (unsigned long long)popc64(mf) | ((unsigned long long)popc64(mr) << 32));
+    const uint32_t bf = bcast(uint32_t(base), 0), br = bcast(uint32_t(base >> 32), 0);
+    if (pf || pr) {
+        const uint32_t at = pf ? bf + rank_in(mf) : br + rank_in(mr);
+        uint32_t *list = pf ? list_f : list_r;
+        if (at < cap) {
+            list[at] = value;
+            if (pf) at_f = at; else at_r = at;
+        } else {
+            atomicOr(err, errbit);
+        }
+    }
+}
+
 TSI_DI uint64_t wave_sum64(uint64_t v) {
     for (int off = 32; off > 0; off >>= 1) {
         uint32_t lo = uint32_t(v), hi = uint32_t(v >> 32);
