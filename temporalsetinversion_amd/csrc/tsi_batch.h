@@ -60,7 +60,7 @@ struct BatchCtl {
 struct BatchArgs {
     const BatchSession *sess;
     BatchCtl *ctl;
-    Counters *out;          // each session's counters after the frame (read back by the host)
+    CounterHead *out;          // each session's counters after the frame (read back by the host)
     float2 *stack;          // saved-operand stacks, stack_len rows x 64 lanes per wavefront
     uint32_t stack_len;
     uint32_t nsess;
@@ -117,14 +117,14 @@ TSI_DI void batch_units(const BatchSession &S, int d, uint32_t &nr, uint32_t &nf
         nr = (list_entries(S.a, d, 1) + 7u) / 8u;
         nf = (list_entries(S.a, d, 0) + 7u) / 8u;
     }
-    if (d >= 1) nd = (min(S.a.cnt->dlist_count[d], S.a.dlist_cap) + 7u) / 8u;
+    if (d >= 1) nd = (min(S.a.cnt->level[d].dlist, S.a.dlist_cap) + 7u) / 8u;
 }
 
 // One dealloc unit: group g of the cascade's list `step` (dealloc_step's loop body).
 template <class KA>
 TSI_DI uint32_t dealloc_group(const KA &a, int step, uint32_t g) {
     Counters *cnt = a.cnt;
-    const uint32_t count = min(cnt->dlist_count[step], a.dlist_cap);
+    const uint32_t count = min(cnt->level[step].dlist, a.dlist_cap);
     const uint32_t *in = a.dlists[step & 1];
     uint32_t *out = a.dlists[(step + 1) & 1];
     const uint32_t lane = lane_id();
@@ -133,7 +133,7 @@ TSI_DI uint32_t dealloc_group(const KA &a, int step, uint32_t g) {
     const bool active = idx < count;
     const uint32_t blk = active ? in[idx] : 0u;
     const uint32_t m = active ? meta_of(a.st[blk * 8u + o]) & kChildMask : 0u;
-    wave_append(m != 0, m - 1u, out, &cnt->dlist_count[step + 1], a.dlist_cap, &cnt->frame_error, kErrQueue);
+    wave_append(m != 0, m - 1u, out, &cnt->level[step + 1].dlist, a.dlist_cap, &cnt->frame_error, kErrQueue);
     wave_append(active && o == 0, blk, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
     return popc64(ballot(active && o == 0));
 }
@@ -265,7 +265,7 @@ TSI_DI void batch_run(const BatchArgs &b) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the lanes' writes, for the copy below
         const uint32_t *from = reinterpret_cast<const uint32_t *>(a.cnt);
         uint32_t *to = reinterpret_cast<uint32_t *>(b.out + s);
-        for (uint32_t i = lane; i < uint32_t(sizeof(Counters) / 4); i += 64u) to[i] = from[i];
+        for (uint32_t i = lane; i < uint32_t(sizeof(CounterHead) / 4); i += 64u) to[i] = from[i];
         if (lane == 0) a.cnt->root_pending = 1u;
     }
 }

@@ -126,7 +126,7 @@ struct tsi_batch {
     float2 *stack = nullptr;
     BatchSession *sess_d = nullptr, *sess_h = nullptr;
     BatchCtl *ctl = nullptr;
-    Counters *out_d = nullptr, *out_h = nullptr;
+    CounterHead *out_d = nullptr, *out_h = nullptr;
     TraceJob *jobs_d = nullptr, *jobs_h = nullptr;
     unsigned long long *visits_d = nullptr, *visits_h = nullptr;
     uint64_t *tally = nullptr;                  // each session's statistics (KArgs::tally)
@@ -628,7 +628,7 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
                               size_t(njobs) * kBatchVisitSlots * kTallyStride * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                               b->stream));
     }
-    HIP_OK(hipMemcpyAsync(b->out_h, b->out_d, n * sizeof(Counters), hipMemcpyDeviceToHost, b->stream));
+    HIP_OK(hipMemcpyAsync(b->out_h, b->out_d, n * sizeof(CounterHead), hipMemcpyDeviceToHost, b->stream));
     HIP_OK(hipEventRecord(b->ev[3], b->stream));
     b->pending = true;
     return TSI_OK;
@@ -658,7 +658,7 @@ int tsi_batch_wait(tsi_batch *b, tsi_frame_result *results, double *set_ms, doub
     const uint32_t n = uint32_t(b->reqs.size());
     for (uint32_t j = 0; j < n; ++j) {
         const uint32_t i = b->order[j];
-        const Counters &h = b->out_h[j];
+        const CounterHead &h = b->out_h[j];
         if (!results) continue;
         tsi_frame_result &r = results[i];
         std::memset(&r, 0, sizeof r);

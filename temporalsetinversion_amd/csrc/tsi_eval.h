@@ -6,11 +6,12 @@
 //
 // Engine (evaluation of the tape for the wavefront's 64 cells):
 //   Engine(a, wave, lane)
-//   select(a, which, g, pruned_ok, prec_in, rec_idx, need_choices)  program for group g
+//   select(a, which, g, pruned_ok, prec_in, rec_idx, need_choices, act)  program for group g
 //                                   (pruned_ok: every parent has a liveness record and the
 //                                   group's cells lie inside their parents; the lane's parent
 //                                   record is prec_in + rec_idx; need_choices: some cell may
-//                                   write a liveness record its children can use)
+//                                   write a liveness record its children can use; act: the
+//                                   lane's cell is evaluated)
 //   forward<PUSH>(a, x, y, z, t, stk, field, Rlo, Rhi) -> algorithmic f32 ops; PUSH saves the
 //                                   operands the reverse rules need on the wavefront's stack
 //                                   (stk: uniform base, row r of lane l at stk[64 r + l])
@@ -18,7 +19,13 @@
 //   (Rlo/Rhi: a register file the engine may use between the two calls)
 //   records()                      records run per forward pass
 //   choices_recorded()             the forward pass recorded the MIN/MAX choices
-//   liveness(a, rec)               the cell's liveness record (kPrune engines)
+//   hold_choices()                 keeps them: the next forward pass records none (kSkip)
+//   liveness(a, rec, cap)          the cell's liveness record (kPrune engines), word w at
+//                                   rec[w cap]
+//   kSkip                          records serve to skip parts of the full tape whose outcome the
+//                                   parents decided (results and counts are the full tape's): the
+//                                   speculative pass leaves records too, and a cell's t-window is
+//                                   compared with its record's (equal: kExactT; else inside)
 #pragma once
 #include "tsi_wave.h"
 
@@ -35,7 +42,7 @@ namespace tsi {
 // slot + node).  Returns the wavefront's count of freed blocks.
 TSI_DI uint32_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t nwaves) {
     Counters *cnt = a.cnt;
-    const uint32_t count = min(cnt->dlist_count[step], a.dlist_cap);
+    const uint32_t count = min(cnt->level[step].dlist, a.dlist_cap);
     const uint32_t *in = a.dlists[step & 1];
     uint32_t *out = a.dlists[(step + 1) & 1];
     const uint32_t lane = lane_id();
@@ -46,12 +53,15 @@ TSI_DI uint32_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t n
         const bool active = idx < count;
         const uint32_t b = active ? in[idx] : 0u;
         const uint32_t m = active ? meta_of(a.st[b * 8u + o]) & kChildMask : 0u;
-        wave_append(m != 0, m - 1u, out, &cnt->dlist_count[step + 1], a.dlist_cap, &cnt->frame_error, kErrQueue);
+        wave_append(m != 0, m - 1u, out, &cnt->level[step + 1].dlist, a.dlist_cap, &cnt->frame_error, kErrQueue);
         wave_append(active && o == 0, b, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
         freed += popc64(ballot(active && o == 0));
     }
     return freed;
 }
+
+// Levels from which a launch claims its blocks ahead: above, a level has at most 8^4 / 8 groups.
+static constexpr int kClaimLevel = 5;
 
 // A wavefront's tallies of the cells it processed: counts of its lanes (uniform, from ballots) and
 // per-lane sums of work; added to the frame's statistics once (flush_tally).
@@ -65,7 +75,7 @@ struct LevelTally {
 // the kernel only reads; its fields are then scalar loads).
 template <class KA>
 TSI_DI uint32_t list_entries(const KA &a, int level, int which) {
-    return min(a.cnt->list_count[level][which], a.list_cap);
+    return min(a.cnt->level[level].list[which], a.list_cap);
 }
 
 // Group g (entries 8g .. 8g + 7) of one frontier list at one level: 8 parents x 8 child octants
@@ -76,7 +86,7 @@ TSI_DI uint32_t list_entries(const KA &a, int level, int which) {
 // a leaf as new cells), and only its SpecCell record and the parent's tag are written.
 template <bool REV, class Engine, class KA>
 TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t count, float2 *stk, Engine &E,
-                       Slots &Rlo, Slots &Rhi, LevelTally &tl, bool spec = false) {
+                       Slots &Rlo, Slots &Rhi, LevelTally &tl, bool spec = false, uint32_t *tickets = nullptr) {
     const int which = REV ? 1 : 0;
     const bool sp = REV && spec;
     Counters *cnt = a.cnt;
@@ -102,14 +112,20 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         const bool isnew = active && (pmeta & kChildMask) == 0;
         const bool pfast = (pmeta & kFastBit) != 0;
 
-        // ---- allocate child blocks for new parents: one atomic per wavefront ----
+        // ---- allocate child blocks for new parents (tickets: claimed by the caller, else one
+        //      atomic per group) ----
         uint32_t blk = (pmeta & kChildMask) - 1u;
         {
             const uint64_t req = sp ? 0u : ballot(isnew && o == 0);
             if (req) {
                 uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(&cnt->alloc_tickets, popc64(req));
-                base = bcast(base, 0);
+                if (tickets) {   // claimed ahead (eval_level)
+                    base = *tickets;
+                    *tickets += popc64(req);
+                } else {
+                    if (lane == 0) base = atomicAdd(&cnt->alloc_tickets, popc64(req));
+                    base = bcast(base, 0);
+                }
                 uint32_t tk = base + rank_in(req);
                 tk = bcast(tk, int(lane & ~7u));
                 if (isnew) {
@@ -168,11 +184,13 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         //      else the full tape ----
         // every parent of the group has a record (capacities are multiples of 8)
         bool pruned_ok = false;
+        float wlo = 0.0f, whi = 0.0f;
         const uint32_t rec_idx = active ? pidx : g * 8u;
         if (prune && level > 0 && g * 8u + 8u <= a.prune_cap) {
-            const float wlo = __uint_as_float(prec_in[rec_idx]);
-            const float whi = __uint_as_float(prec_in[a.prune_cap + rec_idx]);
-            const bool inside = targ.lo >= wlo && targ.hi <= whi && cx.lo >= plo.x && cx.hi <= phi.x &&
+            wlo = __uint_as_float(prec_in[rec_idx]);
+            whi = __uint_as_float(prec_in[a.prune_cap + rec_idx]);
+            const bool tin = Engine::kExactT ? targ.lo == wlo && targ.hi == whi : targ.lo >= wlo && targ.hi <= whi;
+            const bool inside = tin && cx.lo >= plo.x && cx.hi <= phi.x &&
                                 cy.lo >= plo.y && cy.hi <= phi.y && cz.lo >= plo.z && cz.hi <= phi.z;
             pruned_ok = ballot(guard && !inside) == 0;
         }
@@ -184,7 +202,7 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         // that is not known yet.
         bool kids_ok = false;
         if (prune) {
-            kids_ok = a.swept || (cmeta & kChildMask) == 0 || width / 2.0f <= eps;
+            kids_ok = Engine::kSkip || a.swept || (cmeta & kChildMask) == 0 || width / 2.0f <= eps;
             if (guard && !kids_ok) {
                 const uint32_t cb = ((cmeta & kChildMask) - 1u) * 8u;
                 float tmin = a.st[cb].y;
@@ -193,7 +211,23 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             }
         }
         const bool need_choices = prune && ballot(guard && kids_ok && leaf_w > eps) != 0;
-        E.select(a, which, g, pruned_ok, prec_in, rec_idx, need_choices);
+        E.select(a, which, g, pruned_ok, prec_in, rec_idx, need_choices, guard);
+        // kSkip: the record's t-window, wide enough for this cell's children.  They start at their
+        // own last evaluation, all 8 at the same time; where that lies before this cell's window (a
+        // degenerate one, mostly: the parent was fast), the decisions are taken from a forward pass
+        // of their own over the wider window, if the parents' records cover it (then it costs little;
+        // without it nearly every group of an animated csg frame's level 8 ran the whole tape).
+        Iv rwin = targ;
+        bool widen = false;
+        if (Engine::kSkip && pruned_ok && need_choices) {
+            if (guard && leaf_w > eps && (cmeta & kChildMask) != 0) {
+                const float tc = a.st[((cmeta & kChildMask) - 1u) * 8u].y;
+                rwin.lo = fminf(targ.lo, tc);
+            }
+            const bool in = Engine::kExactT ? rwin.lo == wlo && rwin.hi == whi : rwin.lo >= wlo && rwin.hi <= whi;
+            widen = ballot(guard && rwin.lo != targ.lo) != 0 && ballot(guard && !in) == 0;
+            if (!widen) rwin = targ;
+        }
 
         // ---- this cell's speculative results: the frame-start pass evaluated it (its parent
         //      carries this frame's tag) from the same inputs ----
@@ -217,6 +251,10 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         uint32_t fcv = 0;
         const uint64_t need_eval = ballot(guard && !have);
         if (need_eval) {
+            if (widen) {
+                E.template forward<REV>(a, cx, cy, cz, rwin, stk, field, Rlo, Rhi);
+                E.hold_choices();
+            }
             fcv = E.template forward<REV>(a, cx, cy, cz, targ, stk, field, Rlo, Rhi);
             if (guard && !have && !sp) {
                 tl.fwd_ops += fcv;
@@ -241,6 +279,10 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             }
             if (sp) {
                 // the record of the speculative pass, and the parent's tag for this frame
+                if (Engine::kSkip && E.choices_recorded()) {
+                    const uint32_t cell = (g * 8u + ps) * 8u + o;
+                    E.liveness(a, ok ? a.spec_rec + cell : nullptr, a.spec_cap * 8u);
+                }
                 if (ok) {
                     SpecCell r;
                     r.field_lo = field.lo;
@@ -337,11 +379,11 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
         const bool next_fwd_only = !a.swept && !a.force_deriv &&
                                    ((cmeta & kChildMask) == 0 || (cmeta & kFastBit) || width / 2.0f <= eps);
         uint32_t at_f, at_r;
-        wave_append2(enq && next_fwd_only, enq && !next_fwd_only, C, next_f, next_r, cnt->list_count[level + 1],
+        wave_append2(enq && next_fwd_only, enq && !next_fwd_only, C, next_f, next_r, cnt->level[level + 1].list,
                      a.list_cap, &cnt->frame_error, kErrQueue, at_f, at_r);
         // dropped blocks are freed by the next level's forward-only kernel (the dealloc step
         // below), their descendants by the levels after it
-        wave_append(drop_children, old_child - 1u, a.dlists[(level + 1) & 1], &cnt->dlist_count[level + 1], a.dlist_cap,
+        wave_append(drop_children, old_child - 1u, a.dlists[(level + 1) & 1], &cnt->level[level + 1].dlist, a.dlist_cap,
                     &cnt->frame_error, kErrQueue);
 
         // ---- liveness of the enqueued cells, for their children's pruned programs ----
@@ -350,13 +392,21 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             uint32_t *rec = nullptr;
             if (at_f < a.prune_cap) rec = prec_f + at_f;
             if (at_r < a.prune_cap) rec = prec_r + at_r;
-            const bool valid = kids_ok && E.choices_recorded();
+            // (a group the speculative pass evaluated as a whole ran no forward pass: its records)
+            const bool ran = E.choices_recorded();
+            const bool valid = kids_ok && (ran || (Engine::kSkip && have));
             if (rec) {
-                rec[0] = valid ? __float_as_uint(targ.lo) : 0x7f800000u;
-                rec[a.prune_cap] = valid ? __float_as_uint(targ.hi) : 0xff800000u;
+                const Iv win = ran ? rwin : targ;
+                rec[0] = valid ? __float_as_uint(win.lo) : 0x7f800000u;
+                rec[a.prune_cap] = valid ? __float_as_uint(win.hi) : 0xff800000u;
             }
             if (!valid) rec = nullptr;
-            if (ballot(rec != nullptr) != 0) E.liveness(a, rec);
+            if (ran) {
+                if (ballot(rec != nullptr) != 0) E.liveness(a, rec, a.prune_cap);
+            } else if (Engine::kSkip && rec) {
+                const uint32_t *from = a.spec_rec + (size_t(__float_as_uint(plo.w)) * 8u + o);
+                for (uint32_t w = 2; w < Engine::kRecWords; ++w) rec[size_t(w) * a.prune_cap] = from[size_t(w) * (a.spec_cap * 8u)];
+            }
         }
         tl.cells += popc64(ballot(guard));
         tl.spec += popc64(ballot(have));
@@ -385,6 +435,29 @@ TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t) {
                   (unsigned long long)v);
 }
 
+// Tickets for the new parents (entries without children) of this wavefront's groups: a look ahead
+// over its entries, 8 groups at a time, the block's wavefronts summed in LDS, one atomic per block.
+// Every wavefront of the block calls it.  Returns the wavefront's first ticket.
+// A node is listed once per frame and gets its children from its own group alone, so what the
+// look-ahead sees is what the groups will see.
+TSI_DI uint32_t claim_tickets(const KArgs &a, const uint32_t *list, uint32_t count, uint32_t wave, uint32_t nwaves) {
+    __shared__ uint32_t need[5];   // per wavefront, and the block's first ticket
+    const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
+    uint32_t n = 0;
+    for (uint32_t g0 = wave; g0 * 8u < count; g0 += 8u * nwaves) {
+        const uint32_t idx = (g0 + (lane >> 3) * nwaves) * 8u + (lane & 7u);
+        const bool active = idx < count;
+        n += popc64(ballot(active && (meta_of(a.st[active ? list[idx] : 0u]) & kChildMask) == 0));
+    }
+    if (lane == 0) need[w] = n;
+    __syncthreads();
+    const uint32_t n0 = need[0], n1 = need[1], n2 = need[2], n3 = need[3];
+    if (threadIdx.x == 0) need[4] = n0 + n1 + n2 + n3 ? atomicAdd(&a.cnt->alloc_tickets, n0 + n1 + n2 + n3) : 0u;
+    __syncthreads();
+    const uint32_t t = need[4] + (w > 0 ? n0 : 0u) + (w > 1 ? n1 : 0u) + (w > 2 ? n2 : 0u);
+    return __builtin_amdgcn_readfirstlane(t);
+}
+
 // One level of one frontier list: wavefront `wave` of `nwaves` strides over the list; `bwave`
 // indexes the wavefront's own buffers (saved-operand stack, choice rows), unique in the launch.
 // level -1 (reverse list): the speculative pass over the candidate parents (eval_group).
@@ -402,8 +475,14 @@ TSI_DI void eval_level(const KArgs &a, int level, float time, uint32_t wave_, ui
     // array, so that it is promoted to VGPRs; unused by straight-line engines)
     Slots Rlo, Rhi;
     LevelTally tl;
+    // the blocks of all new parents of the block's groups, claimed with one atomic: at 12 ns each
+    // chip-wide, one per group held the level up by a quarter of a millisecond on a frontier of
+    // 20 270 groups
+    uint32_t tickets = 0;
+    if (!sp && level >= kClaimLevel) tickets = claim_tickets(a, a.lists[level & 1][REV ? 1 : 0], count, wave, nwaves);
     for (uint32_t g = wave; g * 8u < count; g += nwaves)
-        eval_group<REV, Engine>(a, level, time, g, count, stk, E, Rlo, Rhi, tl, sp);
+        eval_group<REV, Engine>(a, level, time, g, count, stk, E, Rlo, Rhi, tl, sp,
+                                !sp && level >= kClaimLevel ? &tickets : nullptr);
     // ---- the dealloc cascade's step for the blocks dropped by the previous level and their
     //      descendants (forward-only kernel; the reverse kernel of the level does not touch the
     //      list, which the previous level's kernels finished) ----
@@ -459,12 +538,12 @@ TSI_DI void spec_gather(const KA &a, uint32_t t, uint32_t nt) {
 TSI_DI void frame_begin(const KArgs &a, uint32_t t, uint32_t nt) {
     Counters *c = a.cnt;
     for (uint32_t i = t; i < uint32_t(kMaxLevels + 2); i += nt) {
-        c->list_count[i][0] = 0;
-        c->list_count[i][1] = 0;
-        c->dlist_count[i] = 0;
+        c->level[i].list[0] = 0;
+        c->level[i].list[1] = 0;
+        c->level[i].dlist = 0;
+        c->level[i].pool_used = 0;
     }
     for (uint32_t i = t; i < kTallySlots * kTallyStride; i += nt) a.tally[i] = 0;
-    for (uint32_t i = t; i < uint32_t(kMaxLevels + 2); i += nt) c->pool_used[i] = 0;
     if (t == 0) {
         c->alloc_tickets = 0;
         c->pending = 0;
@@ -480,7 +559,7 @@ TSI_DI void frame_begin(const KArgs &a, uint32_t t, uint32_t nt) {
                                   ((meta & kChildMask) == 0 || (meta & kFastBit) || w <= a.epsilon);
             const int which = fwd_only ? 0 : 1;
             a.lists[0][which][0] = 0u;
-            c->list_count[0][which] = 1;
+            c->level[0].list[which] = 1;
         }
     }
 }
@@ -528,9 +607,9 @@ TSI_DI void eval_level(const KArgs &a, int level, float time) {
 // launches wrote.
 TSI_DI uint32_t level_split(const KArgs &a, int level, uint32_t blocks) {
     const Counters *cnt = a.cnt;
-    uint32_t cf = min(cnt->list_count[level][0], a.list_cap);
-    if (level > 0) cf = max(cf, min(cnt->dlist_count[level], a.dlist_cap));
-    const uint32_t cr = min(cnt->list_count[level][1], a.list_cap);
+    uint32_t cf = min(cnt->level[level].list[0], a.list_cap);
+    if (level > 0) cf = max(cf, min(cnt->level[level].dlist, a.dlist_cap));
+    const uint32_t cr = min(cnt->level[level].list[1], a.list_cap);
     const uint32_t bf = (cf + 31u) / 32u, br = (cr + 31u) / 32u;   // 8 entries per wavefront
     if (bf + br <= blocks) return bf;
     if (bf == 0u) return 0u;

@@ -344,7 +344,9 @@ TSI_DI void live_walk(const FwdIns *prog, uint32_t n, uint32_t out_slot, const C
 
 // ---- the interpreter as an evaluation engine of eval_level --------------------------------
 struct InterpEngine {
-    static constexpr bool kPrune = true;
+    static constexpr bool kPrune = true, kSkip = false, kExactT = false;
+    static constexpr uint32_t kRecWords = 0;
+    TSI_DI void hold_choices() {}
     const FwdIns *fprog;
     const RevIns *rprog;
     uint32_t n;          // records of the current program
@@ -359,7 +361,7 @@ struct InterpEngine {
         ch.n = 0u;
     }
 
-    TSI_DI void select(const KArgs &a, int which, uint32_t g, bool pruned_ok, const uint32_t *, uint32_t, bool) {
+    TSI_DI void select(const KArgs &a, int which, uint32_t g, bool pruned_ok, const uint32_t *, uint32_t, bool, bool) {
         fprog = a.fprog;
         rprog = a.rprog;
         n = a.nfwd;
@@ -398,7 +400,7 @@ struct InterpEngine {
     TSI_DI uint32_t records() const { return n; }
     TSI_DI bool choices_recorded() const { return choices; }
 
-    TSI_DI void liveness(const KArgs &a, uint32_t *rec) { live_walk(fprog, n, a.out_slot, ch, a.nchunks, rec, a.prune_cap); }
+    TSI_DI void liveness(const KArgs &a, uint32_t *rec, uint32_t) { live_walk(fprog, n, a.out_slot, ch, a.nchunks, rec, a.prune_cap); }
 };
 
 }  // namespace tsi

@@ -18,6 +18,7 @@
 #include <unistd.h>
 #include <utime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -189,6 +190,21 @@ bool is_minmax_form(uint32_t form) {
 // forms whose reverse rule needs only a decision (compute.wgsl 2640 ABS_I_RR, 2884-2903 MIN/MAX)
 bool is_code_form(uint32_t form) { return is_minmax_form(form) || form == F_ABS; }
 
+// forms whose reverse rule gives [0, 0] for a sensitivity of [0, 0] whatever the operands are
+bool zero_product(uint32_t form) {
+    return is_code_form(form) || form == F_ADD_RR || form == F_ADD_RL || form == F_SUB_RR || form == F_SUB_RL ||
+           form == F_SUB_LR || form == F_NEG || form == F_RET || form == F_MUL_RL || form == F_DIV_RL ||
+           form == F_MUL_RR || form == F_SQR || form == F_SQRT || form == F_DIV_RR || form == F_DIV_LR ||
+           form == F_MOD_RL;
+}
+
+// the rule's operands are all single-use (the reference's short-circuit applies)
+bool single_use(const RevIns &rv, uint32_t side) {
+    if (side == 1) return (rv.flags & R_U1_A) != 0;
+    if (side == 2) return (rv.flags & R_U1_B) != 0;
+    return (rv.flags & R_U1_A) && (rv.flags & R_U1_B);
+}
+
 // operand values the reverse rule of a form reads (rev_form_t in tsi_rules.h): x = the first
 // register operand (the register of a literal-then-register form), y = the second
 void rev_needs(uint32_t form, bool &x, bool &y) {
@@ -309,12 +325,269 @@ JitLayout jit_layout(const std::vector<FwdIns> &fwd, const Lowered &L, bool prun
     return y;
 }
 
+// ---- chains of unions (JitChain) ----
+namespace {
+
+// Segments the chain needs at least ($TSI_JIT_CHAIN, default 16; 0 turns chains off).  A union of 8
+// spheres takes the same time in a straight line (a 64 x 64 pass 229 us, 6 levels of 256 x 256 2.98
+// ms, either way); 64 smooth-min capsules at 512^3 take 350 us a frame instead of 385, 257 segments
+// at 1024^3 0.81 ms instead of 1.37.
+uint32_t chain_min_segments() {
+    static const uint32_t m = [] {
+        const char *e = std::getenv("TSI_JIT_CHAIN");
+        const long v = e ? std::strtol(e, nullptr, 10) : 16;
+        return v >= 0 && v <= 4096 ? uint32_t(v) : 16u;
+    }();
+    return m;
+}
+
+}  // namespace
+
+JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
+                   const std::vector<RevIns> &rev, const Lowered &L) {
+    JitChain C;
+    const uint32_t min_segs = chain_min_segments();
+    if (min_segs == 0 || n < 24) return C;
+    auto side = [&](uint32_t j) { return side_of(tape[j]); };
+    auto form = [&](uint32_t j) { return j < 4 ? uint32_t(F_COUNT) : uint32_t(fwd[j - 4].form); };
+    auto left = [&](uint32_t j) { return larg_of(tape[j]); };
+    auto right = [&](uint32_t j) { return rarg_of(tape[j]); };
+    std::vector<std::vector<uint32_t>> users(n);
+    std::vector<uint32_t> deps(n, 0);   // inputs a record depends on (bits x, y, z, t)
+    for (uint32_t k = 0; k < 4; ++k) deps[k] = 1u << k;
+    std::vector<char> used(n, 0);
+    used[n - 1] = 1;
+    for (uint32_t j = n; j-- > 4;)
+        if (used[j]) {
+            if (side(j) == 0 || side(j) == 1) used[left(j)] = 1;
+            if (side(j) == 0 || side(j) == 2) used[right(j)] = 1;
+        }
+    for (uint32_t j = 4; j < n; ++j) {
+        if (side(j) == 0 || side(j) == 1) { deps[j] |= deps[left(j)]; if (used[j]) users[left(j)].push_back(j); }
+        if (side(j) == 0 || side(j) == 2) { deps[j] |= deps[right(j)]; if (used[j]) users[right(j)].push_back(j); }
+    }
+    // every form inclusion-monotone in binary32 (a sub-interval's value lies in the interval's), but
+    // for the transcendental ones, which get checks of their own
+    std::vector<uint32_t> trans;
+    for (uint32_t j = 4; j < n; ++j) {
+        if (!used[j] || (side(j) == 0 && left(j) == right(j))) return C;
+        switch (form(j)) {
+        case F_ADD_RR: case F_ADD_RL: case F_SUB_RR: case F_SUB_RL: case F_SUB_LR: case F_MUL_RR: case F_MUL_RL:
+        case F_DIV_RL: case F_SQR: case F_SQRT: case F_MIN_RR: case F_MIN_RL: case F_MAX_RR: case F_MAX_RL: case F_NEG:
+        case F_ABS: case F_RET: case F_FLOOR: case F_ZERO:
+            break;
+        case F_SIN: case F_COS: case F_EXP: case F_LOG: trans.push_back(j); break;
+        default: return C;
+        }
+    }
+    // ---- the links, from the top ----
+    std::vector<uint32_t> links(n, 0);   // links from a record down, at most
+    for (uint32_t k = 4; k < n; ++k) {
+        if (form(k) == F_MIN_RR || form(k) == F_MAX_RR) links[k] = 1u + std::max(links[left(k)], links[right(k)]);
+        else if (form(k) == F_SUB_RR) links[k] = links[left(k)];
+    }
+    if (form(n - 1) != F_RET || side(n - 1) != 1) return C;
+    // dominated by c among the records below the chain's current top: every user is
+    auto single_user = [&](uint32_t k, uint32_t c) { return users[k].size() == 1 && users[k][0] == c; };
+    std::vector<JitChain::Segment> segs;   // from the top
+    double growth = 0.0;                   // log2 bound of the sensitivities' growth along the chain
+    uint32_t cur = left(n - 1);
+    if (cur < 4 || !single_user(cur, n - 1)) return C;
+    for (;;) {
+        JitChain::Segment S;
+        S.o = cur;
+        uint32_t m = cur;
+        if (form(cur) == F_SUB_RR) {
+            // min(a, b) - c * max(k - |..|, 0)^2: with the maximum decided for 0, min(a, b)
+            const uint32_t A = left(cur);
+            uint32_t B = right(cur);
+            if (A < 4 || B < 4 || form(A) != F_MIN_RR || !single_user(A, cur) || !single_user(B, cur)) break;
+            std::vector<uint32_t> thr{cur, A};   // records a decided link passes a sensitivity through
+            double c = 1.0;
+            uint32_t above = cur;
+            while (B >= 4 && form(B) == F_MUL_RL && single_user(B, above)) {
+                const float l = tape[B].literal;
+                if (!(l >= 0x1p-10f && l <= 0x1p20f)) break;
+                c *= double(l);
+                thr.push_back(B);
+                above = B;
+                B = left(B);
+            }
+            if (B < 4 || form(B) != F_SQR || !single_user(B, above)) break;
+            thr.push_back(B);
+            const uint32_t M = left(B);
+            if (M < 4 || form(M) != F_MAX_RL || tape[M].literal != 0.0f || std::signbit(tape[M].literal)) break;
+            bool only_b = true;
+            for (uint32_t u : users[M]) only_b = only_b && u == B;
+            if (!only_b) break;
+            const uint32_t X = left(M);
+            if (X < 4 || form(X) != F_SUB_LR || !(std::fabs(tape[X].literal) <= 0x1p20f) || right(X) < 4 ||
+                form(right(X)) != F_ABS)
+                break;
+            m = A;
+            S.lit = int(M);
+            for (uint32_t k : thr) S.through += single_use(rev[(n - 1) - k], side(k)) ? rev[(n - 1) - k].cost : 0u;
+            growth += std::log2(1.0 + 2.0 * c * std::fabs(double(tape[X].literal)));   // |h| <= k
+        } else if (form(cur) == F_MIN_RR || form(cur) == F_MAX_RR) {
+            S.through = single_use(rev[(n - 1) - cur], side(cur)) ? rev[(n - 1) - cur].cost : 0u;
+        } else {
+            break;
+        }
+        S.choice = m;
+        S.is_min = form(m) == F_MIN_RR;
+        if (left(m) == right(m) || left(m) < 4 || right(m) < 4) break;
+        // the chain goes on in the operand with more links below it
+        const uint32_t l = left(m), r = right(m);
+        S.p_left = links[l] >= links[r];
+        S.p = S.p_left ? l : r;
+        S.w = S.p_left ? r : l;
+        // the chain operand is read by the decision (and a smooth minimum's difference) alone, so the
+        // segment's own operand does not depend on it
+        if (S.lit < 0) {
+            if (!single_user(S.p, m)) break;
+        } else {
+            const uint32_t X = left(uint32_t(S.lit)), ab = right(X), d = left(ab);
+            if (!single_user(X, uint32_t(S.lit)) || !single_user(ab, X) || d < 4 || form(d) != F_SUB_RR ||
+                !single_user(d, ab) || !((left(d) == l && right(d) == r) || (left(d) == r && right(d) == l)) ||
+                users[S.p].size() != 2 || !((users[S.p][0] == m && users[S.p][1] == d) ||
+                                            (users[S.p][0] == d && users[S.p][1] == m)))
+                break;
+        }
+        segs.push_back(S);
+        cur = S.p;
+        if (segs.size() > 4000) break;
+    }
+    if (segs.size() < min_segs || growth > 100.0) return C;
+    // ---- each record's segment: the one of all its users ----
+    // (base first: chain numbers from the bottom)
+    const uint32_t count = uint32_t(segs.size());
+    auto assign = [&](uint32_t from) {   // the links segs[0 .. count - from), numbered from count - from down to 1
+        std::vector<int> seg(n, -1), chain_of(n, -1);
+        for (uint32_t i = 0; i < count - from; ++i) chain_of[segs[i].o] = int(count - from - i);
+        chain_of[segs[count - from - 1].p] = 0;
+        for (uint32_t k = n; k-- > 4;) {
+            if (chain_of[k] >= 0) { seg[k] = chain_of[k]; continue; }
+            int s = -2;
+            for (uint32_t u : users[k]) s = s == -2 ? seg[u] : (s == seg[u] ? s : -1);
+            seg[k] = s < 0 ? -1 : s;
+        }
+        return seg;
+    };
+    // The chain ends above the first link that does not fit: globals, then the segments one after the
+    // other, each from its first record to its chain record, then the RET; every record of a segment
+    // (the base's too) of a rule that gives [0, 0] for a zero sensitivity, or skipped then.
+    uint32_t from = 0;
+    std::vector<int> seg;
+    for (;; ++from) {
+        if (count - from < min_segs) return C;
+        seg = assign(from);
+        bool good = true;
+        int at = -1;
+        for (uint32_t k = 4; k + 1 < n && good; ++k) {
+            good = seg[k] == at || (seg[k] == at + 1 && (at < 0 || seg[k - 1] == at));
+            if (good && seg[k] != at) good = at < 0 || k - 1 == (at == 0 ? segs[count - from - 1].p : segs[count - from - at].o);
+            at = seg[k];
+            if (seg[k] >= 0)
+                good = good && (zero_product(form(k)) || single_use(rev[(n - 1) - k], side(k)));
+        }
+        for (uint32_t i = 0; i < count - from && good; ++i) {
+            const JitChain::Segment &S = segs[i];
+            const int id = int(count - from - i);
+            for (uint32_t u : users[S.p]) good = good && seg[u] == id;
+            good = good && seg[S.choice] == id && (S.lit < 0 || seg[S.lit] == id);
+        }
+        if (good && at == int(count - from)) break;
+    }
+    // ---- the transcendental records ----
+    for (uint32_t j : trans) {
+        if (seg[j] >= 0) {
+            if (deps[j] & 7u) return C;   // of the position, in a segment: no check reaches it
+            C.exact_t = true;
+        } else {
+            C.x_records.push_back(j);
+        }
+    }
+    if (C.x_records.size() > 8) return C;
+    JitChain::Segment base;
+    base.o = segs[count - from - 1].p;
+    C.segs.push_back(base);
+    for (uint32_t i = count - from; i-- > 0;) C.segs.push_back(segs[i]);
+    for (JitChain::Segment &S : C.segs) S.lo = n;
+    for (uint32_t k = n; k-- > 4;)
+        if (seg[k] >= 0) C.segs[size_t(seg[k])].lo = k;
+    // ---- classes: segments of the same structure ----
+    std::map<std::string, uint32_t> known;
+    for (uint32_t i = 0; i < C.segs.size(); ++i) {
+        JitChain::Segment &S = C.segs[i];
+        std::string key = i == 0 ? "base" : "link";
+        auto tok = [&](uint32_t k) {
+            if (i > 0 && k == S.p) return std::string("p");
+            return seg[k] == int(i) ? "t" + std::to_string(k - S.lo) : "v" + std::to_string(k);
+        };
+        for (uint32_t j = S.lo; j <= S.o; ++j) {
+            key += ";" + std::to_string(form(j)) + "," + std::to_string(side(j));
+            if (side(j) == 0 || side(j) == 1) key += "," + tok(left(j));
+            if (side(j) == 0 || side(j) == 2) key += "," + tok(right(j));
+            key += "," + std::to_string(unsigned(rev[(n - 1) - j].cost)) + (single_use(rev[(n - 1) - j], side(j)) ? "u" : "");
+        }
+        if (i > 0) key += ";" + std::to_string(S.choice - S.lo) + "," + std::to_string(S.lit < 0 ? -1 : S.lit - int(S.lo)) + (S.p_left ? "l" : "r");
+        const auto it = known.find(key);
+        if (it == known.end()) {
+            S.cls = uint32_t(known.size());
+            known[key] = S.cls;
+            JitChain::Class K;
+            K.rep = i;
+            K.lit.assign(S.o - S.lo + 1, -1);
+            C.classes.push_back(K);
+        } else {
+            S.cls = it->second;
+            const JitChain::Segment &R = C.segs[C.classes[S.cls].rep];
+            for (uint32_t j = S.lo; j <= S.o; ++j)
+                if (std::memcmp(&tape[j].literal, &tape[R.lo + (j - S.lo)].literal, 4) != 0) C.classes[S.cls].lit[j - S.lo] = 1;
+        }
+    }
+    C.lit_words = 1;   // [0]: the class
+    for (JitChain::Class &K : C.classes) {
+        uint32_t w = 1;
+        for (int &l : K.lit)
+            if (l >= 0) l = int(w++);
+        C.lit_words = std::max(C.lit_words, w);
+    }
+    // ---- rows of the globals that segments and rules read ----
+    C.row.assign(n, -1);
+    std::vector<char> need(n, 0);
+    for (uint32_t j = 4; j < n; ++j) {
+        const bool l = side(j) == 0 || side(j) == 1, r = side(j) == 0 || side(j) == 2;
+        bool nx = false, ny = false;
+        rev_needs(form(j), nx, ny);
+        if (is_code_form(form(j))) nx = ny = true;
+        if (seg[j] >= 0) nx = ny = true;
+        if (nx && l && seg[left(j)] < 0) need[left(j)] = 1;
+        if ((side(j) == 2 ? nx : ny) && r && seg[right(j)] < 0) need[right(j)] = 1;
+    }
+    for (uint32_t k = 0; k < n; ++k)
+        if (need[k]) C.row[k] = int(C.rows++);
+    // what the kernels hold per wavefront: a mask word per lane, the rows of the allocated stack
+    if (C.classes.size() > 32 || C.lit_words > 32 || C.segs.size() > 2048 || C.rows + C.segs.size() > L.stack) {
+        C.segs.clear();
+        return C;
+    }
+    C.seg = seg;
+    C.words = uint32_t(C.segs.size() + 31) / 32;
+    C.col_words = 2u * uint32_t(C.x_records.size()) + C.words + 1u;
+    C.record_words = 2u + C.col_words;
+    return C;
+}
+
 std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
                        const std::vector<RevIns> &rev, const Lowered &L, bool rev_kernel, bool prune,
-                       const JitDomain *domain, bool skip, uint32_t group) {
+                       const JitDomain *domain, bool skip, uint32_t group, const JitChain *chain) {
     std::string o;
     o.reserve(size_t(n) * 500u);
     const JitLayout Y = jit_layout(fwd, L, prune, group);
+    const bool ch = !prune && chain && chain->ok();
+    const JitChain none;
+    const JitChain &CH = ch ? *chain : none;
     const uint32_t G = Y.group, RW = Y.region_words, MW = Y.mode_words;
     auto region_of = [&](uint32_t j) { return (j - 4) / G; };
     // MIN/MAX index of record j (records in order)
@@ -368,7 +641,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
     o += "static constexpr uint32_t kTapeRecords = " + std::to_string(L.nfwd) + "u;\n";
     o += "static constexpr uint32_t kRegionWords = " + std::to_string(RW) + "u, kModeWords = " + std::to_string(MW) +
          "u;\n";
-    o += "struct RegionMask { uint32_t w[" + std::to_string(RW) + "]; };\n";
+    o += ch ? std::string("struct RegionMask { uint32_t w, top; };   // w: word k in lane k\n")
+            : "struct RegionMask { uint32_t w[" + std::to_string(RW) + "]; };\n";
     // fix() with its bounds in scalar registers: a 4-byte encoding per use instead of an
     // 8-byte one with a literal (the tape functions' code is streamed from L2 by every wave)
     o += "struct FixK { float lo, hi; };\n"
@@ -380,7 +654,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
          "    if (__builtin_constant_p(x.lo) && __builtin_constant_p(x.hi)) return fix(x);\n"
          "    return I(wmax(x.lo, k.lo), wmin(x.hi, k.hi));\n}\n";
     o += "TSI_DI uint32_t abs_code(Iv x) { return I_CONTAINS_ZERO(x) ? 3u : (x.hi < 0.0f ? 2u : 1u); }\n";
-    o += "struct FwdOut { Iv field; uint32_t cost, records; };\n";
+    o += ch ? "struct FwdOut { Iv field; uint32_t cost, records, live, rows; };\n"
+            : "struct FwdOut { Iv field; uint32_t cost, records; };\n";
     // Unpruned modules (lean): the saved-operand stack as global memory, so that global loads are
     // counted one by one (vmcnt) and the next region's loads stay in flight while this region
     // waits for its own (through a generic pointer they are flat loads, after which only a wait
@@ -526,6 +801,311 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         return std::string(is_min ? "min_choice(" : "max_choice(") + l + ", " + rhs + ")";
     };
 
+    // ---- a chain's tape functions (JitChain): globals in a straight line, a loop over segments ----
+    // Segment table: per segment lit_words words, [0] its class, then the literals its class does not
+    // share.  The next segment's entry is in flight (scalar loads) while a segment runs.
+    auto chain_names = [&](uint32_t c) {   // name of operand k in the body of class c
+        const JitChain::Segment &R = CH.segs[CH.classes[c].rep];
+        const bool base = CH.classes[c].rep == 0;
+        return [R, base](uint32_t k) {
+            if (!base && k == R.p) return std::string("p");
+            return "v" + std::to_string(k);
+        };
+    };
+    auto chain_lit = [&](uint32_t c, uint32_t j) {
+        const JitChain::Class &C = CH.classes[c];
+        const int w = C.lit[j - CH.segs[C.rep].lo];
+        return w < 0 ? lit(tape[j].literal) : "__uint_as_float(c_.v[" + std::to_string(w) + "])";
+    };
+    // the forward expression of record j of class c (that of a global: c < 0)
+    auto chain_fwd = [&](int c, uint32_t j, const std::string &l, const std::string &r) {
+        const uint32_t form = fwd[j - 4].form;
+        bool f = ff[j], z = form == F_SQRT && side_of(tape[j]) == 1 && pz[larg_of(tape[j])];
+        std::string lt = lit(tape[j].literal);
+        if (c >= 0) {
+            const uint32_t at = j - CH.segs[CH.classes[size_t(c)].rep].lo;
+            for (const JitChain::Segment &S : CH.segs)
+                if (S.cls == uint32_t(c)) {
+                    f = f && ff[S.lo + at];
+                    z = z && pz[larg_of(tape[S.lo + at])];
+                }
+            lt = chain_lit(uint32_t(c), j);
+        }
+        const std::string e = z ? "SQRT_NN(" + l + ")"
+                                : "fwd_form_t<true>(" + std::to_string(form) + "u, " + l + ", " + r + ", " + lt + ")";
+        return std::make_pair(f ? e : "fixk(" + e + ", K)", f);
+    };
+    // one reverse rule: record j, sensitivity s (name), operand names a / b, the derivatives from the
+    // operands' values; add(k, product, zero test or empty) receives the contributions
+    auto chain_rule = [&](int c, uint32_t j, const std::string &s, const std::string &a, const std::string &b, bool f_,
+                          uint64_t &static_ops, const std::function<void(bool, const std::string &, const std::string &)> &add) {
+        const auto &g = tape[j];
+        const uint32_t side = side_of(g), form = fwd[j - 4].form;
+        const RevIns &rv = rev[(n - 1) - j];
+        const std::string J = "_" + std::to_string(j);
+        const std::string lt = c >= 0 ? chain_lit(uint32_t(c), j) : lit(g.literal);
+        std::string rule = "rev_form_t<true>(" + std::to_string(form) + "u, " + (side == 0 || side == 1 ? a : b) + ", " +
+                           (side == 0 ? b : "ZI") + ", " + lt + ")";
+        if (form == F_SQRT && side == 1 && f_) rule = "Iv2{sqrt_rr_of_value(v" + std::to_string(j) + "), ZI}";
+        const bool code = is_code_form(form);
+        if (code) {
+            const std::string kc = "kc" + J;
+            const bool rl = form == F_MIN_RL || form == F_MAX_RL;
+            o += "        const uint32_t " + kc + " = " + code_expr(j, a, rl ? "I_FROM(" + lt + ")" : b) + ";\n";
+            if (form == F_ABS)
+                rule = "Iv2{sel(" + kc + " == 3u, I(-1.0f, 1.0f), sel(" + kc + " == 2u, I_FROM(-1.0f), ONE)), ZI}";
+            else if (rl)
+                rule = "Iv2{sel((" + kc + " & 1u) != 0u, ONE, ZI), ZI}";
+            else
+                rule = "Iv2{sel((" + kc + " & 1u) != 0u, ONE, ZI), sel((" + kc + " & 2u) != 0u, ONE, ZI)}";
+        }
+        o += "        const Iv2 d" + J + " = " + rule + ";\n";
+        // fix of the derivative: as in the straight-line pass (emit_reverse)
+        auto d = [&](const char *x) {
+            const std::string e = "d" + J + "." + x;
+            const uint32_t other = x[0] == 'a' ? rarg_of(g) : larg_of(g);
+            if (code || (form == F_MUL_RR && other >= 4u)) return e;
+            if (domain && (form == F_MUL_RR || (form == F_SQR && f_))) return e;
+            return "fixk(" + e + ", K)";
+        };
+        const bool u1 = single_use(rv, side);
+        const std::string z = "z" + J;
+        if (u1) {
+            o += "        const bool " + z + " = " + (j == n - 1 ? std::string("false") : "(" + s + ".lo == 0.0f && " + s + ".hi == 0.0f)") +
+                 ";\n        ops += " + z + " ? 0u : " + std::to_string(unsigned(rv.cost)) + "u;\n";
+        } else if (c < 0) {   // (a segment's: counted for all segments at once)
+            static_ops += rv.cost;
+        }
+        const std::string zt = u1 && !zero_product(form) ? z : std::string();
+        // both products before either is added (an operand may be both)
+        if (side == 0) {
+            o += "        const Iv na" + J + " = MUL_II(" + d("a") + ", " + s + "), nb" + J + " = MUL_II(" + d("b") + ", " + s + ");\n";
+            add(true, "na" + J, zt);
+            add(false, "nb" + J, zt);
+        } else {
+            add(side == 1, "MUL_II(" + d("a") + ", " + s + ")", zt);
+        }
+    };
+    auto emit_chain = [&]() {
+        const uint32_t NL = CH.lit_words, NS = uint32_t(CH.segs.size()), X = uint32_t(CH.x_records.size()), W = CH.words;
+        auto row = [&](uint32_t k) { return "(stk + " + std::to_string(64u * k) + "u)[lane]"; };
+        // ---- tables ----
+        o += "struct SegEntry { uint32_t v[" + std::to_string(NL) + "]; };\nstatic __constant__ const uint32_t kSegTab[" +
+             std::to_string(NS * NL) + "] = {\n";
+        for (const JitChain::Segment &S : CH.segs) {
+            std::vector<uint32_t> e(NL, 0u);
+            e[0] = S.cls;
+            const JitChain::Class &C = CH.classes[S.cls];
+            for (uint32_t j = S.lo; j <= S.o; ++j)
+                if (C.lit[j - S.lo] >= 0) std::memcpy(&e[size_t(C.lit[j - S.lo])], &tape[j].literal, 4);
+            for (uint32_t x : e) o += std::to_string(x) + "u,";
+            o += "\n";
+        }
+        o += "};\nTSI_DI SegEntry seg_entry(uint32_t i) {\n    SegEntry e;\n    const uint32_t *t = kSegTab + size_t(i) * " +
+             std::to_string(NL) + "u;\n    for (uint32_t k = 0; k < " + std::to_string(NL) + "u; ++k) e.v[k] = t[k];\n    return e;\n}\n";
+        if (rev_kernel) {   // ops a sensitivity passes through in decided segments, summed from the base up
+            o += "static __constant__ const uint32_t kThrough[" + std::to_string(NS + 1) + "] = {0u,";
+            uint32_t t = 0;
+            for (const JitChain::Segment &S : CH.segs) o += std::to_string(t += S.through) + "u,";
+            o += "};\n";
+        }
+        o += "// the words of a mask of all segments, word w in lane w\nTSI_DI uint32_t all_segments(uint32_t lane) {\n    return lane < " +
+             std::to_string(NS / 32) + "u ? 0xFFFFFFFFu : (lane == " + std::to_string(NS / 32) + "u ? " +
+             std::to_string((1ull << (NS % 32)) - 1ull) + "u : 0u);\n}\n\n";
+        // ---- forward ----
+        o += "template <bool PUSH>\n__device__ __noinline__ FwdOut tape_forward(Iv v0, Iv v1, Iv v2, Iv v3, float2 *stk_, uint32_t lane, "
+             "const uint32_t *lrec, uint32_t cap, uint32_t *cols, RegionMask mask, bool act) {\n"
+             "    gfloat2 *stk = (gfloat2 *)stk_;\n    const Iv ZI = I_FROM(0.0f);\n    const FixK K = fix_consts();\n";
+        for (uint32_t k = 0; k + 1 < n; ++k) {
+            if (k >= 4 && CH.seg[k] >= 0) break;
+            if (k >= 4) {
+                const uint32_t side = side_of(tape[k]);
+                const std::string l = (side == 0 || side == 1) ? V(larg_of(tape[k])) : "ZI";
+                const std::string r = (side == 0 || side == 2) ? V(rarg_of(tape[k])) : "ZI";
+                o += "    const Iv " + V(k) + " = " + chain_fwd(-1, k, l, r).first + ";\n";
+            }
+            if (CH.row[k] >= 0) o += "    if (PUSH) " + row(uint32_t(CH.row[k])) + " = make_float2(" + V(k) + ".lo, " + V(k) + ".hi);\n";
+        }
+        uint64_t outside_cost = 0;
+        uint32_t outside = 0;
+        for (uint32_t j = 4; j < n; ++j)
+            if (CH.seg[j] < 0) { outside_cost += fwd[j - 4].cost; outside += 1; }
+        o += "    bool skipping = __builtin_amdgcn_readfirstlane(uint32_t(lrec != nullptr)) != 0u;\n";
+        if (X) {
+            o += "    if (skipping) {\n        bool in = true;\n";
+            for (uint32_t i = 0; i < X; ++i) {
+                const std::string v = V(CH.x_records[i]);
+                o += "        in = in && " + v + ".lo >= __uint_as_float(lrec[size_t(" + std::to_string(2 + 2 * i) + "u) * cap]) && " + v +
+                     ".hi <= __uint_as_float(lrec[size_t(" + std::to_string(3 + 2 * i) + "u) * cap]);\n";
+            }
+            o += "        skipping = __builtin_amdgcn_ballot_w64(act && !in) == 0;\n    }\n    if (cols) {\n";
+            for (uint32_t i = 0; i < X; ++i) {
+                const std::string v = V(CH.x_records[i]);
+                o += "        cols[" + std::to_string(2 * i * 64u) + "u] = __float_as_uint(" + v + ".lo);\n        cols[" +
+                     std::to_string((2 * i + 1) * 64u) + "u] = __float_as_uint(" + v + ".hi);\n";
+            }
+            o += "    }\n";
+        }
+        o += "    const uint32_t mw = skipping ? mask.w : all_segments(lane);\n"
+             "    const uint32_t top = skipping ? mask.top : 0u;\n"
+             "    uint32_t tp = 0u, live = 0u, rows = " + std::to_string(CH.rows) + "u;\n"
+             "    uint32_t cost = " + std::to_string(outside_cost) + "u, records = " + std::to_string(outside) + "u;   // of what runs\n"
+             "    Iv cur = I_FROM(__uint_as_float(0x7f800000u));   // (a base that no cell needs)\n"
+             "#pragma unroll 1\n    for (uint32_t w = 0; w < " + std::to_string(W) + "u; ++w) {\n"
+             "        uint32_t m = uint32_t(__builtin_amdgcn_readlane(int(mw), int(w)));\n"
+             "        uint32_t np = 0u, lw = 0u;\n        if (m) {\n"
+             "            uint32_t b = uint32_t(__builtin_ctz(m));\n            SegEntry c_ = seg_entry(w * 32u + b);\n"
+             "#pragma unroll 1\n            for (;;) {\n                m &= m - 1u;\n"
+             "                const uint32_t nb = m ? uint32_t(__builtin_ctz(m)) : b;\n"
+             "                // (this entry is there before the next one's loads go out: scalar loads return in any\n"
+             "                // order, and a wait after them would be a wait for both)\n"
+             "                uint32_t cls = c_.v[0], ni = w * 32u + nb;\n"
+             "                asm volatile(\"\" : \"+s\"(cls), \"+s\"(ni));\n"
+             "                const SegEntry next = seg_entry(ni);\n"
+             "                const uint32_t i = w * 32u + b;\n                bool dp = false, dw = false;\n                Iv pin = cur;\n"
+             "                switch (cls) {\n";
+        for (uint32_t c = 0; c < CH.classes.size(); ++c) {
+            const JitChain::Segment &R = CH.segs[CH.classes[c].rep];
+            const bool base = CH.classes[c].rep == 0;
+            const auto nm = chain_names(c);
+            o += "                case " + std::to_string(c) + "u: {\n";
+            if (!base) {
+                const std::string inf = R.is_min ? "0x7f800000u" : "0xff800000u";
+                // (the value of a chain operand that the segment's own operand always wins over)
+                o += "        const Iv p = sel(top == i, I_FROM(__uint_as_float(" + inf + ")), cur);\n        pin = p;\n";
+            }
+            for (uint32_t j = R.lo; j <= R.o; ++j) {
+                const uint32_t side = side_of(tape[j]);
+                const std::string l = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
+                const std::string r = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
+                o += "        const Iv " + V(j) + " = " + chain_fwd(int(c), j, l, r).first + ";\n";
+            }
+            if (!base) {
+                const std::string l = nm(larg_of(tape[R.choice])), r = nm(rarg_of(tape[R.choice]));
+                const std::string lt = l + ".hi < " + r + ".lo", gt = r + ".hi < " + l + ".lo";
+                const std::string lw = R.is_min ? lt : gt, rw = R.is_min ? gt : lt;
+                std::string z;
+                if (R.lit >= 0) z = " && " + nm(larg_of(tape[uint32_t(R.lit)])) + ".hi < 0.0f";
+                o += "        dp = " + (R.p_left ? lw : rw) + z + ";\n        dw = " + (R.p_left ? rw : lw) + z + ";\n";
+            }
+            uint64_t cost = 0;
+            for (uint32_t j = R.lo; j <= R.o; ++j) cost += fwd[j - 4].cost;
+            o += "        cur = " + V(R.o) + ";\n        cost += " + std::to_string(cost) + "u;\n        records += " +
+                 std::to_string(R.o - R.lo + 1) + "u;\n                break; }\n";
+        }
+        o += "                default: break;\n                }\n"
+             "                np |= dp ? 0u : 1u << b;\n                tp = dw ? i : tp;\n";
+        if (rev_kernel)
+            o += "                // the reverse pass visits the segments that some cell has not decided for p\n"
+                 "                if (PUSH && __builtin_amdgcn_ballot_w64(act && !dp) != 0) {\n"
+                 "                    stk[size_t(rows) * 64u + lane] = make_float2(pin.lo, pin.hi);\n"
+                 "                    rows += 1u;\n                    lw |= 1u << b;\n                }\n";
+        o += "                if (m == 0u) break;\n                b = nb;\n                c_ = next;\n            }\n        }\n"
+             "        if (cols) cols[(" + std::to_string(2 * X) + "u + w) * 64u] = np;\n"
+             "        live = lane == w ? lw : live;\n    }\n"
+             "    if (cols) cols[" + std::to_string((2 * X + W) * 64u) + "u] = tp;\n";
+        o += "    return FwdOut{" + chain_fwd(-1, n - 1, "cur", "ZI").first + ", cost, records, live, rows};\n}\n\n";
+        if (!rev_kernel) return;
+        // ---- reverse ----
+        o += "__device__ __noinline__ RevOut tape_reverse(const float2 *stk_, uint32_t lane, uint32_t live, uint32_t rows, bool act) {\n"
+             "    const gfloat2 *stk = (const gfloat2 *)stk_;\n    const Iv ZI = I_FROM(0.0f), ONE = I_FROM(1.0f);\n"
+             "    const FixK K = fix_consts();\n    uint32_t ops = 0;\n";
+        for (uint32_t k = 0; k < n; ++k)
+            if (CH.row[k] >= 0) {
+                const std::string sv = "sv" + std::to_string(k);
+                o += "    float2 " + sv + ";\n    " + sv + " = " + row(uint32_t(CH.row[k])) + ";\n    const Iv " + V(k) + " = I(" + sv + ".x, " +
+                     sv + ".y);\n";
+            }
+        for (uint32_t k = 0; k + 1 < n; ++k) {
+            if (k >= 4 && CH.seg[k] >= 0) break;
+            o += "    Iv " + S(k) + " = ZI;\n";
+        }
+        uint64_t static_ops = 0;
+        for (uint32_t j = 4; j < n; ++j)
+            if (CH.seg[j] >= 0 && !single_use(rev[(n - 1) - j], side_of(tape[j]))) static_ops += rev[(n - 1) - j].cost;
+        o += "    Iv s = ZI;\n    {\n";
+        chain_rule(-1, n - 1, "ONE", "ZI", "ZI", false, static_ops,
+                   [&](bool, const std::string &e, const std::string &) { o += "        s = " + e + ";\n"; });
+        o += "    }\n    // segments decided for p in every cell pass the sensitivity on: their ops, where it is not zero\n"
+             "    auto through = [&](uint32_t hi, uint32_t lo) { ops += s.lo == 0.0f && s.hi == 0.0f ? 0u : kThrough[hi] - kThrough[lo]; };\n"
+             "    uint32_t above = " + std::to_string(NS) + "u;   // segments from here on are done\n"
+             "#pragma unroll 1\n    for (uint32_t w = " + std::to_string(W) + "u; w-- > 0u;) {\n"
+             "        uint32_t m = uint32_t(__builtin_amdgcn_readlane(int(live), int(w)));\n"
+             "        if (m == 0u) continue;\n        uint32_t b = 31u - uint32_t(__builtin_clz(m));\n"
+             "        SegEntry c_ = seg_entry(w * 32u + b);\n        rows -= 1u;\n        float2 pv = stk[size_t(rows) * 64u + lane];\n"
+             "#pragma unroll 1\n        for (;;) {\n            m &= ~(1u << b);\n"
+             "            const uint32_t nb = m ? 31u - uint32_t(__builtin_clz(m)) : b;\n"
+             "            uint32_t cls = c_.v[0], ni = w * 32u + nb;\n"
+             "            asm volatile(\"\" : \"+s\"(cls), \"+s\"(ni));\n"
+             "            const SegEntry next = seg_entry(ni);\n"
+             "            if (m) rows -= 1u;\n            const float2 pnext = stk[size_t(rows) * 64u + lane];\n"
+             "            through(above, w * 32u + b + 1u);\n            above = w * 32u + b;\n"
+             "            // (nothing below has a sensitivity, or an op to count)\n"
+             "            if (__builtin_amdgcn_ballot_w64(act && !(s.lo == 0.0f && s.hi == 0.0f)) == 0) break;\n"
+             "            const Iv p = I(pv.x, pv.y);\n            switch (cls) {\n";
+        for (uint32_t c = 0; c < CH.classes.size(); ++c) {
+            const JitChain::Segment &R = CH.segs[CH.classes[c].rep];
+            const bool base = CH.classes[c].rep == 0;
+            const auto nm = chain_names(c);
+            o += "            case " + std::to_string(c) + "u: {\n";
+            std::vector<char> f(R.o - R.lo + 1, 0), live(n, 0);
+            for (uint32_t j = R.lo; j <= R.o; ++j) {
+                const uint32_t side = side_of(tape[j]);
+                const std::string l = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
+                const std::string r = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
+                const auto e = chain_fwd(int(c), j, l, r);
+                f[j - R.lo] = e.second;
+                o += "        const Iv " + V(j) + " = " + e.first + ";\n";
+                if (j != R.o) o += "        Iv " + S(j) + " = ZI;\n";
+            }
+            if (!base) o += "        Iv sp = ZI;\n";
+            bool open = false, plive = false;
+            for (uint32_t j = R.o + 1; j-- > R.lo;) {
+                if (!base && j == R.w) {   // the segment's own operand: where some cell keeps it
+                    const std::string lv = "lv" + std::to_string(j);
+                    o += "        const bool " + lv + " = __builtin_amdgcn_ballot_w64(act && !(" + S(j) + ".lo == 0.0f && " + S(j) +
+                         ".hi == 0.0f)) != 0;\n        if (" + lv + ") {\n";
+                    open = true;
+                }
+                const uint32_t side = side_of(tape[j]);
+                const std::string a = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
+                const std::string b = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
+                chain_rule(int(c), j, j == R.o ? "s" : S(j), a, b, f[j - R.lo], static_ops,
+                           [&](bool first, const std::string &e, const std::string &z) {
+                               const uint32_t k = first ? larg_of(tape[j]) : rarg_of(tape[j]);
+                               const bool isp = !base && k == R.p;
+                               const std::string t = isp ? std::string("sp") : S(k);
+                               const bool global = !isp && (k < 4 || CH.seg[k] < 0);
+                               const bool has = global || (isp ? plive : bool(live[k]));
+                               std::string v = has ? "ADD_II(" + e + ", " + t + ")" : e;
+                               if (!z.empty()) v = "sel(" + z + ", " + (global ? t : std::string("ZI")) + ", " + v + ")";
+                               o += "        " + t + " = " + v + ";\n";
+                               if (isp) plive = true; else live[k] = 1;
+                           });
+            }
+            if (open) o += "        }\n";
+            o += std::string("        s = ") + (base ? "ZI" : "sp") + ";\n            break; }\n";
+        }
+        o += "            default: break;\n            }\n            if (m == 0u) break;\n            b = nb;\n            c_ = next;\n"
+             "            pv = pnext;\n        }\n"
+             "        if (__builtin_amdgcn_ballot_w64(act && !(s.lo == 0.0f && s.hi == 0.0f)) == 0) break;\n    }\n"
+             "    through(above, 0u);\n    {\n";
+        for (uint32_t j = n; j-- > 4;) {
+            if (j == n - 1 || CH.seg[j] >= 0) continue;
+            const uint32_t side = side_of(tape[j]);
+            const std::string a = (side == 0 || side == 1) ? (CH.row[larg_of(tape[j])] >= 0 ? V(larg_of(tape[j])) : "ZI") : "ZI";
+            const std::string b = (side == 0 || side == 2) ? (CH.row[rarg_of(tape[j])] >= 0 ? V(rarg_of(tape[j])) : "ZI") : "ZI";
+            chain_rule(-1, j, S(j), a, b, false, static_ops,
+                       [&](bool first, const std::string &e, const std::string &z) {
+                           const uint32_t k = first ? larg_of(tape[j]) : rarg_of(tape[j]);
+                           std::string v = "ADD_II(" + e + ", " + S(k) + ")";
+                           if (!z.empty()) v = "sel(" + z + ", ZI, " + v + ")";
+                           o += "        " + S(k) + " = " + v + ";\n";
+                       });
+        }
+        o += "    }\n    ops += " + std::to_string(static_ops) + "u;\n    return RevOut{s0, s1, s2, s3, ops};\n}\n\n";
+    };
+
     // choices: the MIN/MAX choices go to chbuf (always with pr)
     auto emit_forward = [&](const std::string &fname, bool choices) {
     o += "template <bool PUSH>\n__device__ __noinline__ FwdOut " + fname + "(Iv v0, Iv v1, Iv v2, Iv v3, float2 *" +
@@ -637,19 +1217,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         // has a finite bound (it is ordered, or a decision code), so the product with a zero
         // sensitivity is already +-0: the select would only fix the sign of a zero, and it is
         // left out (the work count stays).
-        auto zero_product = [&](uint32_t form) {
-            return is_code_form(form) || form == F_ADD_RR || form == F_ADD_RL || form == F_SUB_RR ||
-                   form == F_SUB_RL || form == F_SUB_LR || form == F_NEG || form == F_RET || form == F_MUL_RL ||
-                   form == F_DIV_RL || form == F_MUL_RR || form == F_SQR || form == F_SQRT || form == F_DIV_RR ||
-                   form == F_DIV_LR || form == F_MOD_RL;
-        };
-        auto single_use = [&](uint32_t j) {   // the rule's operands all single-use (short-circuit applies)
-            const RevIns &rv = rev[(n - 1) - j];
-            const uint32_t side = side_of(tape[j]);
-            if (side == 1) return (rv.flags & R_U1_A) != 0;
-            if (side == 2) return (rv.flags & R_U1_B) != 0;
-            return (rv.flags & R_U1_A) && (rv.flags & R_U1_B);
-        };
+        auto single_use = [&](uint32_t j) { return tsi::single_use(rev[(n - 1) - j], side_of(tape[j])); };
         // Skipped subtrees (unpruned modules).  Record g dominates record k when every path from
         // the output to k passes through g: k's sensitivity is then a sum of products along paths
         // through g's.  With g's sensitivity [0, 0] and every record that g dominates either
@@ -865,7 +1433,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                 }
                 if (lo > 4u) emit_loads(lo, region_lo(lo));   // the next region's operands go in flight
             }
-            // the open guarded block (its guard, the sensitivities first assigned in it)
+            // the open guarded block: its guard, and the sensitivities first assigned in it
             int cur = -1;
             std::vector<uint32_t> first;
             auto close_block = [&]() {
@@ -1008,8 +1576,12 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
     // pruned modules carry three forward variants: pruned (the parents' records apply and skip
     // enough regions), full with the MIN/MAX choices recorded (some cell may write a liveness
     // record its children can use) and full; and two reverse ones, pruned and full
-    emit_forward("tape_forward", prune);
-    if (rev_kernel) emit_reverse("tape_reverse");
+    if (ch) {
+        emit_chain();
+    } else {
+        emit_forward("tape_forward", prune);
+        if (rev_kernel) emit_reverse("tape_reverse");
+    }
     if (prune) {
         pr = false;
         emit_forward("tape_forward_full", false);
@@ -1079,8 +1651,65 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         o += "    }\n}\n\n";
     }
 
+    if (ch) {
+        // ---- the chain's engine: the parents' decisions in, this wavefront's out ----
+        const std::string W = std::to_string(CH.words), X2 = std::to_string(2 * CH.x_records.size());
+        const std::string CW = std::to_string(CH.col_words), RWs = std::to_string(CH.record_words);
+        uint64_t full_cost = 0;
+        for (uint32_t j = 4; j < n; ++j) full_cost += fwd[j - 4].cost;
+        o += "struct TapeEngine {\n    static constexpr bool kPrune = true, kSkip = true, kExactT = " + std::string(CH.exact_t ? "true" : "false") +
+             ";\n    static constexpr uint32_t kRecWords = " + RWs + "u;\n"
+             "    uint32_t lane;\n    const uint32_t *lrec;\n    uint32_t *colbase, *cols;\n    RegionMask mask;\n"
+             "    uint32_t live, rows, nrec;\n    bool act, ran;\n"
+             "    template <class KA>\n    TSI_DI TapeEngine(const KA &a, uint32_t wave, uint32_t l)\n"
+             "        : lane(l), lrec(nullptr), cols(nullptr), mask{0u, 0u}, live(0u), rows(0u), nrec(kTapeRecords), act(true), ran(false) {\n"
+             "        colbase = a.choice ? a.choice + size_t(wave) * " + CW + "u * 64u + l : nullptr;\n    }\n"
+             "    template <class KA>\n    TSI_DI void select(const KA &a, int, uint32_t, bool pruned_ok, const uint32_t *prec_in, uint32_t pidx,\n"
+             "                       bool need_choices, bool act_) {\n"
+             "        lrec = nullptr;\n        act = act_;\n        ran = false;\n        cols = need_choices ? colbase : nullptr;\n"
+             "        if (pruned_ok) {\n            lrec = prec_in + pidx;\n            mask.w = 0u;\n"
+             "            // 8 words at a time: each lane one word of its parent, OR over the 8 parents\n"
+             "            for (uint32_t q = 0; q * 8u < " + W + "u; ++q) {\n"
+             "                const uint32_t w = q * 8u + (lane & 7u);\n"
+             "                uint32_t v = w < " + W + "u ? lrec[size_t(2u + " + X2 + "u + w) * a.prune_cap] : 0u;\n"
+             "                v |= uint32_t(__shfl_xor(int(v), 8, 64));\n"
+             "                v |= uint32_t(__shfl_xor(int(v), 16, 64));\n"
+             "                v |= uint32_t(__shfl_xor(int(v), 32, 64));\n"
+             "                mask.w = (lane >> 3) == q ? v : mask.w;\n            }\n"
+             "            mask.top = lrec[size_t(2u + " + X2 + "u + " + W + "u) * a.prune_cap];\n        }\n    }\n"
+             "    template <bool PUSH, class KA>\n"
+             "    TSI_DI uint32_t forward(const KA &a, Iv x, Iv y, Iv z, Iv t, float2 *stk, Iv &field, Slots &, Slots &) {\n"
+             "        const FwdOut r = tape_forward<PUSH>(x, y, z, t, stk, lane, lrec, a.prune_cap, cols, mask, act);\n"
+             "        live = r.live;\n        rows = __builtin_amdgcn_readfirstlane(r.rows);\n"
+             "        ran = ran || cols != nullptr;\n        field = r.field;\n"
+             "        // what ran, or (pruning refused) the whole tape's counts\n"
+             "        const bool whole = a.prune != 1;\n"
+             "        nrec = whole ? kTapeRecords : __builtin_amdgcn_readfirstlane(r.records);\n"
+             "        return whole ? " + std::to_string(full_cost) + "u : __builtin_amdgcn_readfirstlane(r.cost);\n    }\n";
+        if (rev_kernel)
+            o += "    template <class KA>\n    TSI_DI uint32_t reverse(const KA &, const float2 *stk, Iv sens[4], Slots &, Slots &) {\n"
+                 "        const RevOut r = tape_reverse(stk, lane, live, rows, act);\n"
+                 "        sens[0] = r.s0; sens[1] = r.s1; sens[2] = r.s2; sens[3] = r.s3;\n        return r.ops;\n    }\n";
+        else
+            o += "    template <class KA>\n    TSI_DI uint32_t reverse(const KA &, const float2 *, Iv sens[4], Slots &, Slots &) {\n"
+                 "        for (int k = 0; k < 4; ++k) sens[k] = I_FROM(0.0f);\n        return 0u;\n    }\n";
+        o += "    TSI_DI uint32_t records() const { return nrec; }\n"
+             "    TSI_DI bool choices_recorded() const { return ran; }\n"
+             "    TSI_DI void hold_choices() { cols = nullptr; }\n"
+             "    // the cell's record: segments below the highest that keeps only its own operand are not needed\n"
+             "    template <class KA>\n    TSI_DI void liveness(const KA &, uint32_t *rec, uint32_t cap) {\n"
+             "        if (!rec) return;\n"
+             "        const uint32_t tp = colbase[(" + X2 + "u + " + W + "u) * 64u];\n"
+             "        for (uint32_t i = 0; i < " + X2 + "u; ++i) rec[size_t(2u + i) * cap] = colbase[i * 64u];\n"
+             "        for (uint32_t w = 0; w < " + W + "u; ++w) {\n"
+             "            const uint32_t v = colbase[(" + X2 + "u + w) * 64u];\n"
+             "            const uint32_t keep = w > (tp >> 5) ? 0xFFFFFFFFu : (w == (tp >> 5) ? 0xFFFFFFFFu << (tp & 31u) : 0u);\n"
+             "            rec[size_t(2u + " + X2 + "u + w) * cap] = v & keep;\n        }\n"
+             "        rec[size_t(2u + " + X2 + "u + " + W + "u) * cap] = tp;\n    }\n"
+             "};\n\n}  // namespace tsi\n\n";
+    } else {
     // ---- the evaluation engine of eval_level (tsi_eval.h) ----
-    o += std::string("struct TapeEngine {\n    static constexpr bool kPrune = ") + (prune ? "true" : "false") + ";\n";
+    o += std::string("struct TapeEngine {\n    static constexpr bool kPrune = ") + (prune ? "true" : "false") + ", kSkip = false, kExactT = false;\n    static constexpr uint32_t kRecWords = 0u;\n    TSI_DI void hold_choices() {}\n";
     o += "    static constexpr uint32_t kRegions = " + std::to_string(Y.regions) + "u;\n";
     o += "    uint32_t lane, recs;\n    const uint32_t *prec;\n    uint32_t *chbuf;\n    RegionMask mask;\n"
          "    uint32_t variant;   // this wavefront's: 0 full, 1 full + choices, 2 pruned\n";
@@ -1089,7 +1718,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
          "        for (uint32_t w = 0; w < kRegionWords; ++w) mask.w[w] = 0xFFFFFFFFu;\n"
          "        chbuf = a.choice ? a.choice + size_t(wave) * kModeWords * 64u + l : nullptr;\n    }\n";
     o += "    template <class KA>\n    TSI_DI void select(const KA &a, int, uint32_t, bool pruned_ok, const uint32_t *prec_in, uint32_t pidx,\n"
-         "                       bool need_choices) {\n"
+         "                       bool need_choices, bool) {\n"
          "        prec = nullptr;\n"
          "        variant = 0;\n"
          "        for (uint32_t w = 0; w < kRegionWords; ++w) mask.w[w] = 0xFFFFFFFFu;\n";
@@ -1137,10 +1766,11 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
     o += "    TSI_DI uint32_t records() const { return recs; }\n";
     o += "    TSI_DI bool choices_recorded() const { return variant != 0u; }\n";
     if (prune)
-        o += "    template <class KA>\n    TSI_DI void liveness(const KA &a, uint32_t *rec) { tape_liveness(chbuf, rec, a.prune_cap, mask); }\n";
+        o += "    template <class KA>\n    TSI_DI void liveness(const KA &a, uint32_t *rec, uint32_t) { tape_liveness(chbuf, rec, a.prune_cap, mask); }\n";
     else
-        o += "    template <class KA>\n    TSI_DI void liveness(const KA &, uint32_t *) {}\n";
+        o += "    template <class KA>\n    TSI_DI void liveness(const KA &, uint32_t *, uint32_t) {}\n";
     o += "};\n\n}  // namespace tsi\n\n";
+    }
     o += std::string("extern \"C\" __global__ void __launch_bounds__(256) ") +
          (rev_kernel ? "tsi_tape_eval_rev" : "tsi_tape_eval_fwd") +
          "(tsi::KArgs a, int level, float time) {\n    tsi::eval_level<" + (rev_kernel ? "true" : "false") +
@@ -1164,8 +1794,9 @@ std::string module_body(const std::string &src) {
 
 std::string jit_source_level(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
                              const std::vector<RevIns> &rev, const Lowered &L, bool prune, const JitDomain *domain) {
-    const std::string f = jit_source(tape, n, fwd, rev, L, false, prune, domain);
-    const std::string r = jit_source(tape, n, fwd, rev, L, true, prune, domain);
+    const JitChain chain = prune ? JitChain() : jit_chain(tape, n, fwd, rev, L);
+    const std::string f = jit_source(tape, n, fwd, rev, L, false, prune, domain, true, 0, &chain);
+    const std::string r = jit_source(tape, n, fwd, rev, L, true, prune, domain, true, 0, &chain);
     std::string o = "// generated by tsi_jit.cpp: straight-line evaluation of one tape, both lists of a level\n";
     o += "#include \"tsi_eval.h\"\n#include \"tsi_rules.h\"\n\nnamespace tsi {\nnamespace jf {   // forward-only list\n";
     o += module_body(f);
@@ -1247,7 +1878,17 @@ long long read_uint(const std::string &s, size_t i) {
 }  // namespace
 
 std::string jit_check_bounds(const std::string &src, uint32_t stack_rows, uint32_t record_words,
-                             uint32_t mode_words) {
+                             uint32_t mode_words, uint32_t chain_words, uint32_t chain_cols) {
+    // a chain's records: lrec[size_t(w u) * cap], and its columns: cols[64 w u]
+    for (size_t i = src.find("lrec[size_t("); i != std::string::npos; i = src.find("lrec[size_t(", i + 1)) {
+        const long long w = read_uint(src, i + 12);
+        if (w >= 0 && uint64_t(w) >= chain_words) return "chain record word " + std::to_string(w) + " of " + std::to_string(chain_words);
+    }
+    for (size_t i = src.find("cols["); i != std::string::npos; i = src.find("cols[", i + 1)) {
+        const long long off = read_uint(src, i + 5);
+        if (off >= 0 && (off % 64 != 0 || uint64_t(off / 64) >= chain_cols))
+            return "chain column " + std::to_string(off / 64) + " of " + std::to_string(chain_cols);
+    }
     // stack rows: (stk + 64 r u)[lane]
     for (size_t i = src.find("(stk + "); i != std::string::npos; i = src.find("(stk + ", i + 1)) {
         const long long off = read_uint(src, i + 7);
@@ -1259,6 +1900,7 @@ std::string jit_check_bounds(const std::string &src, uint32_t stack_rows, uint32
     for (const char *pat : {"prec[size_t(", "rec[size_t("}) {
         const size_t len = std::strlen(pat);
         for (size_t i = src.find(pat); i != std::string::npos; i = src.find(pat, i + 1)) {
+            if (i > 0 && src[i - 1] == 'l') continue;   // lrec: a chain's, above
             const long long w = read_uint(src, i + len);
             if (w < 0) continue;   // a word index computed at run time (bounded by its loop)
             if (uint64_t(w) >= record_words)

@@ -36,20 +36,28 @@ constexpr uint32_t kTallySlots = 64, kTallyStride = 16;
 // nchunks right-kept words, one bit per full-program record.
 constexpr uint32_t kRecHead = 2;
 
-struct Counters {
-    uint32_t list_count[kMaxLevels + 2][2];   // frontier sizes per level: [0] forward-only, [1] reverse
-    uint32_t dlist_count[kMaxLevels + 2];     // dealloc cascade list sizes
-    uint32_t alloc_tickets;                   // blocks handed out this frame
+// What the host reads back after a frame, and what a frame's kernels only read.
+struct CounterHead {
     uint32_t free_top;                        // free-stack entries at frame start
     uint32_t bump;                            // blocks ever taken from the bump region
-    uint32_t pending;                         // blocks freed this frame
     uint32_t frame_error;                     // kErr* raised this frame
     uint32_t error;                           // sticky kErr* since reset
     uint32_t root_pending;                    // buf_main has enqueued the root
     uint32_t pad;
-    uint32_t pool_used[kMaxLevels + 2];       // program-pool records taken per level
-    uint32_t pad2[2];
     uint64_t stats[kNumStats];
+};
+// Each counter that a level's wavefronts add to has a 128-byte line of its own, and none shares it
+// with what they read: an atomic takes its line for 12 ns chip-wide, and a read of a line that
+// atomics are changing waits its turn among them (a level that allocates in 20 270 groups: 1.0 ms
+// with tickets, free_top and bump in one line, two reads and an atomic per group).
+struct Counters : CounterHead {
+    alignas(128) uint32_t alloc_tickets;      // blocks handed out this frame
+    alignas(128) uint32_t pending;            // blocks freed this frame
+    struct Level {
+        alignas(128) uint32_t list[2];        // frontier sizes: [0] forward-only, [1] reverse
+        alignas(128) uint32_t dlist;          // dealloc cascade list size
+        uint32_t pool_used;                   // program-pool records taken
+    } level[kMaxLevels + 2];
 };
 
 // A speculatively evaluated cell (speculative evaluation of the shallow levels, below): the
@@ -83,7 +91,7 @@ struct KArgs {
     // normal_viz with fast_normals off (compute.wgsl:3780): every cell takes the reverse pass
     int32_t force_deriv;
     // pruned programs (per-group dense programs specialised on the parents' liveness)
-    int32_t prune;
+    int32_t prune;              // 1: on; 2: a chain's kernels with pruning refused (the counts are the whole tape's)
     uint32_t *prune_rec[2][2];  // [level parity][forward-only / reverse], see kRecHead
     uint32_t prune_cap;         // entries per list that get a record
     uint32_t nchunks;           // ceil(nfwd / 32)
@@ -104,6 +112,7 @@ struct KArgs {
     uint32_t *spec_list;        // the listed parents (breadth first from the root)
     uint32_t *spec_count;       // how many
     SpecCell *spec_res;         // 8 per listed parent
+    uint32_t *spec_rec;         // their records (kSkip engines): word w of cell c at [w * 8 spec_cap + c]
     uint64_t *tally;            // kTallySlots x kTallyStride: statistics of the frame so far
 };
 

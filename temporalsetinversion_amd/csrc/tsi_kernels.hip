@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(1024) k_spec_gather(KArgs a) { spec_gather(a, 
 // every parent decided.  Groups with an entry lacking a record run the full program.
 __global__ void __launch_bounds__(256) k_prune(KArgs a, int level, int which) {
     Counters *cnt = a.cnt;
-    const uint32_t count = min(cnt->list_count[level][which], a.list_cap);
+    const uint32_t count = min(cnt->level[level].list[which], a.list_cap);
     if (count == 0) return;
     const uint32_t lane = lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) k_prune(KArgs a, int level, int which) {
         const uint32_t off0 = s0 - n0, off1 = tot0 + s1 - n1;
         const uint32_t pad = program_stride(m);
         uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&cnt->pool_used[level], 2u * pad);
+        if (lane == 0) base = atomicAdd(&cnt->level[level].pool_used, 2u * pad);
         base = bcast(base, 0);
         if (base + 2u * pad > a.pool_cap) {
             if (lane == 0) { desc[2u * g] = 0u; desc[2u * g + 1u] = 0u; }

@@ -87,6 +87,10 @@ struct tsi_ctx {
     FwdIns *pool = nullptr;
     uint32_t prune_cap = 0, nchunks = 0, choice_len = 0, pool_cap = 0;
     bool prune = false;
+    // records of a chain's unpruned kernels (JitChain): prune_rec / choice as above, and the
+    // speculative pass's columns and records
+    bool chain = false, chain_counts = false;
+    uint32_t *spec_choice = nullptr, *spec_rec = nullptr;
     // speculative evaluation of the shallow levels (KArgs::spec_*): the listed parents, their
     // count, the records, the last frame's tag, the levels asked for
     uint32_t *spec_list = nullptr;
@@ -134,7 +138,7 @@ struct tsi_ctx {
         hipEvent_t level[2 * kMaxLevels] = {};   // around each level's evaluation launches
         hipEvent_t spec0 = nullptr, spec1 = nullptr;   // around the speculative pass
         bool spec = false;                             // the frame had one
-        Counters *h = nullptr;
+        CounterHead *h = nullptr;
     };
     // a trace runs on its slot's stream over its slot's device-side snapshot of the octree, so it
     // overlaps the next frame's set inversion on the main stream and the previous trace's last
@@ -225,7 +229,7 @@ KArgs make_args(const tsi_ctx *c) {
     a.lipschitz = c->p.lipschitz_corrected;
     a.fastenabled = c->p.fastenabled;
     a.force_deriv = (c->p.shading & (TSI_SHADE_NORMALS | TSI_SHADE_CINEMATIC)) && (c->p.shading & TSI_SHADE_GRADIENT) ? 1 : 0;
-    a.prune = c->prune ? 1 : 0;
+    a.prune = c->prune ? 1 : (c->chain ? (c->chain_counts ? 1 : 2) : 0);
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j) a.prune_rec[i][j] = c->prune_rec[i][j];
     a.prune_cap = c->prune_cap;
@@ -243,7 +247,8 @@ KArgs make_args(const tsi_ctx *c) {
 void release_prune(tsi_ctx *c) {
     for (auto &l : c->prune_rec) for (auto &x : l) dfree(x);
     dfree(c->gdesc[0]); dfree(c->gdesc[1]); dfree(c->choice); dfree(c->pool);
-    c->prune = false;
+    dfree(c->spec_choice); dfree(c->spec_rec);
+    c->prune = c->chain = false;
     c->prune_cap = c->nchunks = c->choice_len = c->pool_cap = 0;
 }
 
@@ -253,11 +258,20 @@ bool prune_wanted(uint32_t flags, const Lowered &L) {
     return !(L.prune_class == kPruneApprox && (flags & TSI_FLAG_PRUNE_EXACT_ONLY));
 }
 
+// Whether a tape's compiled kernels are its chain's (JitChain): of every chain, pruned or not, since
+// they skip what a pruned module's regions skip, give the full tape's results (a pruned module's are
+// only those where prune_class says exact), and take part in the speculative pass.  Per animated
+// frame of 64 capsules at 512^3: 350 us, pruned module 780, straight-line unpruned module 385.
+// prune_live_max asks for the pruned module and its rule.
+bool chain_wanted(uint32_t flags, uint32_t prune_live_max, const Lowered &L, const JitChain &chain) {
+    if (!chain.ok() || (flags & TSI_FLAG_INTERPRET)) return false;
+    return !prune_wanted(flags, L) || prune_live_max == 0;
+}
+
 // Buffers of pruned evaluation for a lowered tape: liveness records for prune_cap entries of
 // each frontier list (two level parities) and per-wavefront MIN/MAX choice columns; for the
 // interpreter also group descriptors and the program pool (each level reuses it from 0).
 int alloc_prune(tsi_ctx *c, const Lowered &L, const std::vector<FwdIns> &fwd) {
-    release_prune(c);
     if (!prune_wanted(c->p.flags, L)) return TSI_OK;
     const bool interp = (c->p.flags & TSI_FLAG_INTERPRET) != 0;
     uint64_t cap = c->p.prune_capacity ? c->p.prune_capacity : (uint64_t(1) << 19);
@@ -299,6 +313,31 @@ int alloc_prune(tsi_ctx *c, const Lowered &L, const std::vector<FwdIns> &fwd) {
     return TSI_OK;
 }
 
+// Buffers of the unpruned kernels of a tape that is a chain (JitChain): records for as many entries
+// of each frontier list as pruned evaluation keeps, columns per wavefront, and the speculative
+// pass's.  Without them (no memory) every cell runs the whole tape: the same results.
+void alloc_chain(tsi_ctx *c, const JitChain &chain) {
+    uint64_t cap = c->p.prune_capacity ? c->p.prune_capacity : (uint64_t(1) << 19);
+    if (cap > c->list_cap) cap = c->list_cap;
+    cap = (cap + 7) / 8 * 8;
+    const uint32_t waves = (c->grid_fwd + c->grid_rev) * 4u;
+    bool ok = true;
+    for (auto &l : c->prune_rec)
+        for (auto &x : l) ok = ok && dmalloc(&x, size_t(chain.record_words) * cap) == TSI_OK;
+    ok = ok && dmalloc(&c->choice, size_t(waves) * 64u * chain.col_words) == TSI_OK;
+    if (c->spec_max)
+        ok = ok && dmalloc(&c->spec_choice, size_t(c->num_cu) * 4u * 64u * chain.col_words) == TSI_OK &&
+             dmalloc(&c->spec_rec, size_t(chain.record_words) * c->spec_cap * 8u) == TSI_OK;
+    if (!ok) {
+        (void)hipGetLastError();
+        release_prune(c);
+        return;
+    }
+    c->prune_cap = uint32_t(cap);
+    c->choice_len = chain.col_words;
+    c->chain = true;
+}
+
 void release_jit(tsi_ctx *c) {
     for (int k = 0; k < 2; ++k) {
         if (c->mod[k]) hipModuleUnload(c->mod[k]);
@@ -315,9 +354,12 @@ const JitDomain kDefaultDomain{{-5.0f, -5.0f, -5.0f, 5.0f, 5.0f, 5.0f}, -2.0f, 6
 
 // The generated module addresses no stack row, liveness-record word or choice column beyond what
 // alloc_prune and tsi_upload_tape allocate (a module that would is refused, not run).
-int check_module(const std::string &src, const std::vector<FwdIns> &fwd, const Lowered &L, std::string &log) {
+int check_module(const std::string &src, const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
+                 const std::vector<RevIns> &rev, const Lowered &L, std::string &log) {
     const JitLayout Y = jit_layout(fwd, L, true);
-    const std::string bad = jit_check_bounds(src, L.stack + 1u, Y.record_words, Y.mode_words);
+    const JitChain chain = jit_chain(tape, n, fwd, rev, L);
+    const std::string bad =
+        jit_check_bounds(src, L.stack + 1u, Y.record_words, Y.mode_words, chain.record_words, chain.col_words);
     if (bad.empty()) return TSI_OK;
     log = "generated module out of bounds: " + bad;
     return TSI_E_JIT;
@@ -334,7 +376,7 @@ int load_jit(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n, const std:
     int rc = TSI_OK;
     try {
         src = jit_source_level(tape, n, fwd, rev, L, c->prune, domain);
-        rc = check_module(src, fwd, L, log);
+        rc = check_module(src, tape, n, fwd, rev, L, log);
         if (rc == TSI_OK) rc = jit_compile(src, c->prune, code, log, hit, ms);
     } catch (const std::runtime_error &) {   // the generator cannot lay out this tape
         return TSI_E_JIT;
@@ -403,7 +445,7 @@ namespace tsi {
 
 int read_octree(const float4 *st_dev, const float4 *grad_dev, const Counters *cnt_dev, uint64_t nodes, tsi_node *out,
                 uint64_t cap, uint64_t *count) {
-    Counters h;
+    CounterHead h;
     HIP_OK(hipMemcpy(&h, cnt_dev, sizeof h, hipMemcpyDeviceToHost));
     uint64_t used = (uint64_t(h.bump) + 1u) * 8u;
     if (used > nodes) used = nodes;
@@ -527,7 +569,7 @@ int tsi_create(const tsi_params *params, tsi_ctx **out) {
                 evok = evok && hipEventCreateWithFlags(e, hipEventDisableSystemFence) == hipSuccess;
             for (hipEvent_t &e : f.level)
                 evok = evok && hipEventCreateWithFlags(&e, hipEventDisableSystemFence) == hipSuccess;
-            evok = evok && hipHostMalloc((void **)&f.h, sizeof(Counters), hipHostMallocDefault) == hipSuccess;
+            evok = evok && hipHostMalloc((void **)&f.h, sizeof(CounterHead), hipHostMallocDefault) == hipSuccess;
         }
         for (auto &t : c->tslot) {
             for (hipEvent_t *e : {&t.begin, &t.end}) evok = evok && hipEventCreate(e) == hipSuccess;
@@ -643,20 +685,32 @@ int tsi_upload_tape(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n) {
         if ((rc = dmalloc(&c->spec_stack, spec_need / sizeof(float2)))) return rc;
         c->spec_stack_bytes = spec_need;
     }
-    if ((rc = alloc_prune(c, L, fwd))) return rc;
+    fwd.resize(L.nfwd);
+    rev.resize(L.nrev);
+    release_prune(c);
+    JitChain chain;
+    try {
+        if (!(c->p.flags & TSI_FLAG_INTERPRET)) chain = jit_chain(tape, n, fwd, rev, L);
+    } catch (...) {
+        return TSI_E_OOM;
+    }
+    const bool use_chain = chain_wanted(c->p.flags, c->p.prune_live_max, L, chain);
+    if (!use_chain && (rc = alloc_prune(c, L, fwd))) return rc;
     std::memset(&c->info, 0, sizeof c->info);
     c->info.n = n;
     c->info.stack = L.stack;
     c->info.slots = L.slots;
     c->info.prune_class = uint32_t(L.prune_class);
     if (!(c->p.flags & TSI_FLAG_INTERPRET)) {
-        fwd.resize(L.nfwd);
-        rev.resize(L.nrev);
         if ((rc = load_jit(c, tape, n, fwd, rev, L, &kDefaultDomain))) {
             c->have_tape = false;
             return rc;
         }
         c->info.engine = 1;
+        if (use_chain) {
+            alloc_chain(c, chain);
+            c->chain_counts = prune_wanted(c->p.flags, L);
+        }
     } else {
         release_jit(c);
     }
@@ -745,6 +799,7 @@ int tsi_set_inversion_async(tsi_ctx *c) {
         a.spec_list = c->spec_list;
         a.spec_count = c->spec_cnt;
         a.spec_res = c->spec_res;
+        a.spec_rec = c->spec_rec;
         // the pass reads the octree down to depth spec_levels: it starts once the previous frame
         // has run its levels 0 .. spec_max (its last levels run beside it)
         sl.stream = c->spec_stream;
@@ -754,6 +809,7 @@ int tsi_set_inversion_async(tsi_ctx *c) {
         sl.ready = c->spec_ready;
         sl.args = a;
         sl.args.stack = c->spec_stack;
+        sl.args.choice = c->spec_choice;
         sl.blocks = uint32_t(c->num_cu);
         sl.ready_level = int(c->spec_max);
         c->spec_ready_recorded = true;
@@ -762,7 +818,7 @@ int tsi_set_inversion_async(tsi_ctx *c) {
                    (void *)c->eval_fn[0], f.spec ? &sl : nullptr};
     HIP_OK(hipEventRecord(f.begin, c->stream));
     if (launch_frame(a, fl, c->stream, f.eval0, f.eval1, c->level_events ? f.level : nullptr) != 0) return TSI_E_HIP;
-    HIP_OK(hipMemcpyAsync(f.h, c->cnt, sizeof(Counters), hipMemcpyDeviceToHost, c->stream));
+    HIP_OK(hipMemcpyAsync(f.h, c->cnt, sizeof(CounterHead), hipMemcpyDeviceToHost, c->stream));
     HIP_OK(hipEventRecord(f.end, c->stream));
     c->f_issued += 1;
     return TSI_OK;
@@ -774,7 +830,7 @@ int tsi_set_inversion_result(tsi_ctx *c, double *gpu_ms, tsi_stats *stats) {
     tsi_ctx::FrameSlot &f = c->fslot[c->f_done % tsi_ctx::kFrameSlots];
     c->f_done += 1;
     HIP_OK(hipEventSynchronize(f.end));
-    const Counters &h = *f.h;
+    const CounterHead &h = *f.h;
     float ms = 0.0f, ems = 0.0f;
     hipEventElapsedTime(&ms, f.begin, f.end);
     c->last_si_ms = ms;
@@ -1064,15 +1120,21 @@ int tsi_precompile_tape(const tsi_gpu_instruction *tape, uint32_t n, uint32_t fl
             bool hit = false;
             double ms = 0.0;
             const bool prune = prune_wanted(flags, L);
-            src = jit_source_level(tape, n, fwd, rev, L, prune, &kDefaultDomain);
             info.specialized = 1;
             info.fix_kept = n - 4u;
             const std::vector<char> ff = fix_free(tape, n, fwd, kDefaultDomain);
             for (uint32_t j = 4; j < n; ++j) info.fix_kept -= ff[j] ? 1u : 0u;
-            rc = check_module(src, fwd, L, log);
-            if (rc == TSI_OK) rc = jit_compile(src, prune, code, log, hit, ms);
-            info.compile_ms = ms;
-            info.cache_hit = hit;
+            // a chain's kernels, and the pruned module that prune_live_max selects
+            const bool both = prune && chain_wanted(flags, 0, L, jit_chain(tape, n, fwd, rev, L));
+            info.cache_hit = 1;
+            for (int k = both ? 0 : 1; k < 2 && rc == TSI_OK; ++k) {
+                const bool pruned = prune && k == 1;
+                src = jit_source_level(tape, n, fwd, rev, L, pruned, &kDefaultDomain);
+                rc = check_module(src, tape, n, fwd, rev, L, log);
+                if (rc == TSI_OK) rc = jit_compile(src, pruned, code, log, hit, ms);
+                info.compile_ms += ms;
+                info.cache_hit = info.cache_hit && hit;
+            }
             if (rc != TSI_OK) std::strncpy(info.log, log.c_str(), sizeof info.log - 1);
         }
     } catch (const std::runtime_error &) {
