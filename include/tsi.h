@@ -223,6 +223,13 @@ int tsi_read_tape(tsi_ctx *ctx, tsi_gpu_instruction *out, uint32_t cap, uint32_t
 int tsi_frame_rgba8(tsi_ctx *ctx, uint8_t *rgba8_out);
 int tsi_save_frame_png(tsi_ctx *ctx, const char *path);
 
+/* No counterpart in the reference.  Pinned host memory for the pixels of tsi_trace, tsi_trace_wait,
+ * tsi_frame_rgba8 and tsi_batch_frame: copies to it run at the link's rate.  From a pool of at most
+ * 256 MiB, handed out and idle together, shared by all threads; idle buffers are given back when the
+ * last context or batch is destroyed.  NULL: the pool is exhausted, or there is no context. */
+void *tsi_host_buffer(size_t bytes);
+void tsi_host_buffer_free(void *buffer);
+
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): tsi_frame_rgba8 with
  * its RGBA8 staging buffer in the library's static device memory (TSI_STATIC_RGBA8_MAX_PIXELS

@@ -226,6 +226,7 @@ class State:
         self.uniforms = Uniforms()
         self.uniforms.resolution[0] = width
         self.uniforms.resolution[1] = height
+        self._px = 0   # pixels of a frame with the uniforms the library has
         v = diagonal_camera()
         for i in range(16):
             self.uniforms.view[i] = float(v[i])
@@ -241,6 +242,7 @@ class State:
             for i, x in enumerate(np.asarray(view, np.float32).reshape(16)):
                 u.view[i] = float(x)
         check(lib().tsi_set_uniforms(self._ctx, C.byref(u)), "tsi_set_uniforms")
+        self._px = u.resolution[0] * u.resolution[1]
 
     def reset(self):
         v = self.tape["val"]
@@ -272,11 +274,14 @@ class State:
         return FrameResult(ms.value, st.as_dict())
 
     def trace(self, pixels: bool = True):
-        rgba = np.zeros((self.height, self.width, 4), np.float32) if pixels else None
-        depth = np.zeros((self.height, self.width), np.float32) if pixels else None
+        rgba, depth = self._frame_arrays() if pixels else (None, None)
         check(lib().tsi_trace(self._ctx, rgba.ctypes.data if pixels else None,
                               depth.ctypes.data if pixels else None), "tsi_trace")
         return rgba, depth
+
+    def _frame_arrays(self):
+        return (_lib.frame_array((self.height, self.width, 4), np.float32, 4 * self._px),
+                _lib.frame_array((self.height, self.width), np.float32, self._px))
 
     def last_trace(self) -> tuple[float, int]:
         """(device ms, octree node visits) of the last trace."""
@@ -290,8 +295,7 @@ class State:
         check(lib().tsi_trace_async(self._ctx), "tsi_trace_async")
 
     def trace_wait(self, pixels: bool = True):
-        rgba = np.zeros((self.height, self.width, 4), np.float32) if pixels else None
-        depth = np.zeros((self.height, self.width), np.float32) if pixels else None
+        rgba, depth = self._frame_arrays() if pixels else (None, None)
         check(lib().tsi_trace_wait(self._ctx, rgba.ctypes.data if pixels else None,
                                    depth.ctypes.data if pixels else None), "tsi_trace_wait")
         return rgba, depth
@@ -309,7 +313,7 @@ class State:
 
     def frame_rgba8(self) -> np.ndarray:
         """The last traced frame as RGBA8 (main.rs:709-711 conversion), rows top to bottom."""
-        out = np.zeros((self.height, self.width, 4), np.uint8)
+        out = _lib.frame_array((self.height, self.width, 4), np.uint8, 4 * self._px)
         check(lib().tsi_frame_rgba8(self._ctx, out.ctypes.data), "tsi_frame_rgba8")
         return out
 

@@ -8,6 +8,9 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
+
+import numpy as np
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("TSI_LIB", os.path.join(HERE, "_build", "libtsi.so"))
@@ -126,6 +129,8 @@ SIGNATURES = {
                                    C.POINTER(C.c_uint64)]),
     "tsi_frame_rgba8": (C.c_int, [C.c_void_p, C.c_void_p]),
     "tsi_frame_rgba8_noalloc": (C.c_int, [C.c_void_p, C.c_void_p]),
+    "tsi_host_buffer": (C.c_void_p, [C.c_size_t]),
+    "tsi_host_buffer_free": (None, [C.c_void_p]),
     "tsi_save_frame_png": (C.c_int, [C.c_void_p, C.c_char_p]),
     "tsi_write_png": (C.c_int, [C.c_char_p, C.c_void_p, C.c_uint32, C.c_uint32]),
     "tsi_frame_device": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p)]),
@@ -175,6 +180,22 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+def frame_array(shape, dtype, used):
+    """An array for a frame's pixels, of which the library is about to write the first `used` elements
+    (the others are 0): in pinned memory (tsi_host_buffer) that goes back with the array's last
+    view, or pageable where there is none."""
+    n = int(np.prod(shape, dtype=np.int64))
+    nbytes = n * np.dtype(dtype).itemsize
+    p = lib().tsi_host_buffer(nbytes) if nbytes else None
+    if not p:
+        return np.zeros(shape, dtype)
+    buf = (C.c_char * nbytes).from_address(p)
+    weakref.finalize(buf, lib().tsi_host_buffer_free, p).atexit = False
+    out = np.frombuffer(buf, dtype)
+    out[used:] = 0
+    return out.reshape(shape)
 
 
 def check(rc: int, what: str):

@@ -58,6 +58,7 @@ class Batch:
         self._b = C.c_void_p()
         check(lib().tsi_batch_create(ptrs, lens, len(self._bufs), C.byref(cfg), C.byref(self._b)), "tsi_batch_create")
         self.sessions = {}   # id -> (max_width, max_height)
+        self._traced = {}    # id -> pixels of its last traced frame
         self._pending = None
 
     @staticmethod
@@ -103,6 +104,7 @@ class Batch:
     def close_session(self, sid: int):
         check(lib().tsi_batch_close(self._b, sid), "tsi_batch_close")
         self.sessions.pop(sid, None)
+        self._traced.pop(sid, None)
 
     def reset(self, sid: int):
         check(lib().tsi_batch_reset(self._b, sid), "tsi_batch_reset")
@@ -122,6 +124,9 @@ class Batch:
                 reqs[i].view[k] = float(v[k])
         check(lib().tsi_batch_submit(self._b, reqs, len(frames)), "tsi_batch_submit")
         self._pending = list(frames)
+        for f in frames:
+            if f[2] and f[3]:
+                self._traced[f[0]] = f[2] * f[3]
 
     def done(self) -> bool:
         """Whether the submitted frames have finished (does not wait)."""
@@ -160,8 +165,9 @@ class Batch:
         return out
 
     def frame(self, sid: int, width: int, height: int):
-        rgba = np.zeros((height, width, 4), np.float32)
-        depth = np.zeros((height, width), np.float32)
+        used = self._traced.get(sid, 0)
+        rgba = _lib.frame_array((height, width, 4), np.float32, 4 * used)
+        depth = _lib.frame_array((height, width), np.float32, used)
         check(lib().tsi_batch_frame(self._b, sid, rgba.ctypes.data, depth.ctypes.data), "tsi_batch_frame")
         return rgba, depth
 

@@ -16,7 +16,7 @@ OUT_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libtsi.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
-SOURCES = ["tsi_kernels.hip", "tsi_trace.hip", "tsi_runtime.hip", "tsi_batch.hip", "tsi_lower.cpp", "tsi_ir.cpp", "tsi_jit.cpp", "tsi_png.cpp"]
+SOURCES = ["tsi_kernels.hip", "tsi_trace.hip", "tsi_runtime.hip", "tsi_batch.hip", "tsi_hostmem.hip", "tsi_lower.cpp", "tsi_ir.cpp", "tsi_jit.cpp", "tsi_png.cpp"]
 # headers the per-tape kernels are compiled against at run time (embedded in the library)
 JIT_HEADERS = ["tsi_interval.h", "tsi_tape.h", "tsi_kernels.h", "tsi_wave.h", "tsi_rules.h", "tsi_eval.h",
                "tsi_batch.h"]

@@ -20,6 +20,7 @@
 #include "tsi.h"
 #include "tsi_batch.h"
 #include "tsi_jit.h"
+#include "tsi_hostmem.h"
 #include "tsi_launch.h"
 #include "tsi_tape.h"
 
@@ -110,6 +111,7 @@ bool params_ok(const tsi_params &p) {
 }  // namespace
 
 struct tsi_batch {
+    HostPoolUser pool_user;
     int device = 0, num_cu = 256;
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -127,6 +129,7 @@ struct tsi_batch {
     BatchSession *sess_d = nullptr, *sess_h = nullptr;
     BatchCtl *ctl = nullptr;
     CounterHead *out_d = nullptr, *out_h = nullptr;
+    uint32_t *error_h = nullptr;                // BatchCtl::error of the run
     TraceJob *jobs_d = nullptr, *jobs_h = nullptr;
     unsigned long long *visits_d = nullptr, *visits_h = nullptr;
     uint64_t *tally = nullptr;                  // each session's statistics (KArgs::tally)
@@ -184,7 +187,7 @@ void release(tsi_batch *b) {
     b->mod = nullptr;
     dfree(b->stack); dfree(b->sess_d); dfree(b->ctl); dfree(b->out_d); dfree(b->jobs_d);
     dfree(b->visits_d); dfree(b->tally); dfree(b->arena);
-    hfree(b->sess_h); hfree(b->out_h); hfree(b->jobs_h); hfree(b->visits_h);
+    hfree(b->sess_h); hfree(b->out_h); hfree(b->error_h); hfree(b->jobs_h); hfree(b->visits_h);
     for (auto &e : b->ev)
         if (e) { hipEventDestroy(e); e = nullptr; }
     if (b->stream) { hipStreamDestroy(b->stream); b->stream = nullptr; }
@@ -389,7 +392,7 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
             (rc = dmalloc(&b->visits_d, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)) ||
             (rc = dmalloc(&b->tally, size_t(C.max_sessions) * kTallySlots * kTallyStride)) ||
             (rc = hmalloc(&b->sess_h, C.max_sessions)) ||
-            (rc = hmalloc(&b->out_h, C.max_sessions)) || (rc = hmalloc(&b->jobs_h, C.max_sessions)) ||
+            (rc = hmalloc(&b->out_h, C.max_sessions)) || (rc = hmalloc(&b->error_h, 1)) || (rc = hmalloc(&b->jobs_h, C.max_sessions)) ||
             (rc = hmalloc(&b->visits_h, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)))
             break;
         uint64_t arena = C.arena_bytes;
@@ -629,6 +632,7 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
                               b->stream));
     }
     HIP_OK(hipMemcpyAsync(b->out_h, b->out_d, n * sizeof(CounterHead), hipMemcpyDeviceToHost, b->stream));
+    HIP_OK(hipMemcpyAsync(b->error_h, &b->ctl->error[0], sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream));
     HIP_OK(hipEventRecord(b->ev[3], b->stream));
     b->pending = true;
     return TSI_OK;
@@ -653,8 +657,7 @@ int tsi_batch_wait(tsi_batch *b, tsi_frame_result *results, double *set_ms, doub
     if (set_ms) *set_ms = sms;
     if (trace_ms) *trace_ms = tms;
     // a barrier that timed out abandons the whole run
-    BatchCtl ctl;
-    HIP_OK(hipMemcpy(&ctl, b->ctl, sizeof ctl, hipMemcpyDeviceToHost));
+    const bool barrier_error = *b->error_h != 0u;
     const uint32_t n = uint32_t(b->reqs.size());
     for (uint32_t j = 0; j < n; ++j) {
         const uint32_t i = b->order[j];
@@ -664,7 +667,7 @@ int tsi_batch_wait(tsi_batch *b, tsi_frame_result *results, double *set_ms, doub
         std::memset(&r, 0, sizeof r);
         r.status = (h.frame_error & kErrPool) ? TSI_E_POOL_EXHAUSTED
                  : (h.frame_error & kErrQueue) ? TSI_E_QUEUE_FULL : TSI_OK;
-        if (ctl.error[0]) r.status = TSI_E_HIP;
+        if (barrier_error) r.status = TSI_E_HIP;
         r.stats.gpu_ms = sms;
         r.stats.eval_ms = sms;
         r.stats.cell_evals = h.stats[kStatCells];
@@ -683,7 +686,7 @@ int tsi_batch_wait(tsi_batch *b, tsi_frame_result *results, double *set_ms, doub
             for (uint32_t k = 0; k < kBatchVisitSlots; ++k)
                 r.node_visits += b->visits_h[(size_t(b->job_of[i]) * kBatchVisitSlots + k) * kTallyStride];
     }
-    return ctl.error[0] ? TSI_E_HIP : TSI_OK;
+    return barrier_error ? TSI_E_HIP : TSI_OK;
 }
 
 int tsi_batch_read_nodes(tsi_batch *b, uint32_t session, tsi_node *out, uint64_t cap, uint64_t *count) {
@@ -701,9 +704,8 @@ int tsi_batch_frame(tsi_batch *b, uint32_t session, float *rgba_out, float *dept
     if (s.w == 0 || s.h == 0) return TSI_E_ARG;   // nothing traced yet
     HIP_OK(hipStreamSynchronize(b->stream));
     const size_t px = size_t(s.w) * s.h;
-    if (rgba_out) HIP_OK(hipMemcpy(rgba_out, s.rgba, px * sizeof(float4), hipMemcpyDeviceToHost));
-    if (depth_out) HIP_OK(hipMemcpy(depth_out, s.depth, px * sizeof(float), hipMemcpyDeviceToHost));
-    return TSI_OK;
+    const CopyOut out[2] = {{rgba_out, s.rgba, px * sizeof(float4)}, {depth_out, s.depth, px * sizeof(float)}};
+    return copy_out(out, 2, b->stream);
 }
 
 }  // extern "C"

@@ -17,6 +17,7 @@
 
 #include "tsi.h"
 #include "tsi_jit.h"
+#include "tsi_hostmem.h"
 #include "tsi_launch.h"
 #include "tsi_tape.h"
 
@@ -62,6 +63,7 @@ constexpr size_t kVisitBytes = size_t(tsi::kVisitSlots) * tsi::kTallyStride * si
 constexpr size_t kTraceCounters = size_t(tsi::kVisitSlots + tsi::kTraceQueues) * tsi::kTallyStride;
 
 struct tsi_ctx {
+    HostPoolUser pool_user;
     tsi_params p{};
     int device = 0;
     int num_cu = 256;
@@ -76,6 +78,8 @@ struct tsi_ctx {
     uint32_t *pending = nullptr, *free_stack = nullptr;
     Counters *cnt = nullptr;
     uint64_t *tally = nullptr;          // KArgs::tally
+    uchar4 *rgba8 = nullptr;            // tsi_frame_rgba8's image, grown to the largest frame asked for
+    size_t rgba8_px = 0;
     float2 *stack = nullptr;
     size_t stack_bytes = 0;
     FwdIns *fprog = nullptr;
@@ -430,7 +434,7 @@ void release(tsi_ctx *c) {
     dfree(c->st); dfree(c->blo); dfree(c->bhi); dfree(c->grad);
     for (auto &l : c->lists) for (auto &x : l) dfree(x);
     dfree(c->dlists[0]); dfree(c->dlists[1]);
-    dfree(c->pending); dfree(c->free_stack); dfree(c->cnt); dfree(c->tally); dfree(c->stack);
+    dfree(c->pending); dfree(c->free_stack); dfree(c->cnt); dfree(c->tally); dfree(c->rgba8); dfree(c->stack);
     dfree(c->spec_list); dfree(c->spec_cnt); dfree(c->spec_res); dfree(c->spec_stack);
     if (c->spec_ready) { hipEventDestroy(c->spec_ready); c->spec_ready = nullptr; }
     if (c->spec_stream) { hipStreamDestroy(c->spec_stream); c->spec_stream = nullptr; }
@@ -1013,9 +1017,9 @@ int tsi_trace_wait(tsi_ctx *c, float *rgba_out, float *depth_out) {
     const tsi_ctx::TraceSlot &ts = c->tslot[c->last_tslot];
     const size_t px = size_t(c->u.resolution[0]) * c->u.resolution[1];
     if ((rgba_out || depth_out) && (c->t_issued == 0 || px > ts.px)) return TSI_E_ARG;   // nothing traced at this size
-    if (rgba_out) HIP_OK(hipMemcpy(rgba_out, ts.rgba, px * sizeof(float4), hipMemcpyDeviceToHost));
-    if (depth_out) HIP_OK(hipMemcpy(depth_out, ts.depth, px * sizeof(float), hipMemcpyDeviceToHost));
-    return TSI_OK;
+    if (!rgba_out && !depth_out) return TSI_OK;
+    const CopyOut out[2] = {{rgba_out, ts.rgba, px * sizeof(float4)}, {depth_out, ts.depth, px * sizeof(float)}};
+    return copy_out(out, 2, ts.stream);
 }
 
 int tsi_trace(tsi_ctx *c, float *rgba_out, float *depth_out) {
@@ -1040,14 +1044,16 @@ int tsi_frame_rgba8(tsi_ctx *c, uint8_t *rgba8_out) {
     const tsi_ctx::TraceSlot &ts = c->tslot[c->last_tslot];
     const size_t px = size_t(c->u.resolution[0]) * c->u.resolution[1];
     if (px == 0 || c->t_issued == 0 || px > ts.px) return TSI_E_ARG;   // nothing traced at this size
-    uchar4 *tmp = nullptr;
-    if ((rc = dmalloc(&tmp, px))) return rc;
-    rc = launch_rgba8(ts.rgba, tmp, uint32_t(px), c->stream) == 0 ? TSI_OK : TSI_E_HIP;
-    if (rc == TSI_OK && hipMemcpyAsync(rgba8_out, tmp, px * 4u, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-        rc = TSI_E_HIP;
-    if (rc == TSI_OK && hipStreamSynchronize(c->stream) != hipSuccess) rc = TSI_E_HIP;
-    dfree(tmp);
-    return rc;
+    if (px > c->rgba8_px) {   // kept for the next frame: allocating and freeing wait for the device
+        dfree(c->rgba8);
+        c->rgba8_px = 0;
+        if ((rc = dmalloc(&c->rgba8, px))) return rc;
+        c->rgba8_px = px;
+    }
+    // (on the frame's own stream: the trace is done, set inversions in flight are not waited for)
+    if (launch_rgba8(ts.rgba, c->rgba8, uint32_t(px), ts.stream) != 0) return TSI_E_HIP;
+    const CopyOut out{rgba8_out, c->rgba8, px * 4u};
+    return copy_out(&out, 1, ts.stream);
 }
 
 int tsi_frame_rgba8_noalloc(tsi_ctx *c, uint8_t *rgba8_out) {
