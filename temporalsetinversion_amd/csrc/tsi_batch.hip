@@ -546,6 +546,7 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
     std::stable_sort(b->order.begin(), b->order.end(), [&](uint32_t x, uint32_t y) {
         return b->sessions[reqs[x].session].tape < b->sessions[reqs[y].session].tape;
     });
+    uint32_t stack = 0;   // ray-stack entries of the deepest
     uint32_t njobs = 0;
     bool any_spec = false;
     for (uint32_t j = 0; j < n; ++j) {
@@ -578,6 +579,8 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             J.t.depth = s.depth;
             J.t.visits = b->visits_d + size_t(njobs) * kBatchVisitSlots * kTallyStride;
             J.t.visit_slots = kBatchVisitSlots;
+            J.t.stack = trace_stack_entries(s.p.localsubdiv);
+            stack = std::max(stack, J.t.stack);
             J.t.shading = s.p.shading;
             J.t.grad = s.a.grad;
             J.t.mask = reinterpret_cast<const uint32_t *>(s.a.grad) + 3;
@@ -624,8 +627,8 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
         HIP_OK(hipMemcpyAsync(b->jobs_d, b->jobs_h, njobs * sizeof(TraceJob), hipMemcpyHostToDevice, b->stream));
         if (launch_fill_u32(reinterpret_cast<uint32_t *>(b->visits_d), 0u, 2u * njobs * kBatchVisitSlots * kTallyStride, b->stream)) return TSI_E_HIP;
         HIP_OK(hipEventRecord(b->ev[2], b->stream));
-        if (nplain && launch_trace_batch(b->jobs_d, nplain, bplain, false, b->stream)) return TSI_E_HIP;
-        if (nplain < njobs && launch_trace_batch(b->jobs_d + nplain, njobs - nplain, bcin, true, b->stream))
+        if (nplain && launch_trace_batch(b->jobs_d, nplain, bplain, false, stack, b->stream)) return TSI_E_HIP;
+        if (nplain < njobs && launch_trace_batch(b->jobs_d + nplain, njobs - nplain, bcin, true, stack, b->stream))
             return TSI_E_HIP;
         HIP_OK(hipMemcpyAsync(b->visits_h, b->visits_d,
                               size_t(njobs) * kBatchVisitSlots * kTallyStride * sizeof(unsigned long long), hipMemcpyDeviceToHost,

@@ -118,19 +118,4 @@ struct KArgs {
 
 constexpr uint32_t kVisitSlots = 32, kBatchVisitSlots = 8;   // node-visit counters of a trace (see kTallySlots)
 
-struct TraceArgs {
-    float view[16];
-    uint32_t width, height;
-    float time, zdist;
-    float4 *rgba;
-    float *depth;
-    unsigned long long *visits; // kVisitSlots counters, kTallyStride words apart (one line each)
-    uint32_t shading;           // TSI_SHADE_* (normal_viz, gradient normals, cinematic)
-    const float4 *grad;         // the nodes' dx, dy, dz (gradient normals)
-    const uint32_t *mask;       // the nodes' surface masks (grad[n].w), mask_stride words apart
-    uint32_t mask_stride;
-    uint32_t visit_slots;       // a power of two
-};
-
-
 }  // namespace tsi

@@ -42,7 +42,23 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
                  const hipEvent_t *e_level);
 int launch_reset(const KArgs &a, const float box[6], uint64_t nodes, hipStream_t s);
 int launch_enqueue_root(const KArgs &a, hipStream_t s);
-constexpr uint32_t kTraceTile = 16;   // a batched trace block's pixels: kTraceTile x kTraceTile
+// A trace's frame.
+struct TraceArgs {
+    float view[16];
+    uint32_t width, height;
+    float time, zdist;
+    float4 *rgba;
+    float *depth;
+    unsigned long long *visits; // kVisitSlots counters, kTallyStride words apart (one line each)
+    uint32_t shading;           // TSI_SHADE_* (normal_viz, gradient normals, cinematic)
+    const float4 *grad;         // the nodes' dx, dy, dz (gradient normals)
+    const uint32_t *mask;       // the nodes' surface masks (grad[n].w), mask_stride words apart
+    uint32_t mask_stride;
+    uint32_t visit_slots;       // a power of two
+    uint32_t stack;             // ray-stack entries: more than the octree's paths need, or the reference's 16
+};
+
+constexpr uint32_t kTraceTile = 8;   // a batched trace block's pixels: kTraceTile x kTraceTile
 // claim counters of the persistent trace, each in a line of its own (2 * kTallyStride uint32 apart)
 constexpr uint32_t kTraceQueues = 8;
 // blocks > 0 (with next_quad, kTraceQueues counters zeroed on `s` before): the persistent form on that many
@@ -60,7 +76,13 @@ struct TraceJob {
     uint32_t block0;    // the frame's first block in the launch
 };
 // (cinematic: every job's session shades with TSI_SHADE_CINEMATIC; no job mixes the two)
-int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, hipStream_t s);
+// stack: the largest of the jobs' TraceArgs::stack.
+int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, uint32_t stack,
+                       hipStream_t s);
+// Whether a frame is traced with four lanes per ray (by its size; full launches only).
+bool trace_quads(const TraceArgs &t);
+// TraceArgs::stack for an octree whose nodes lie at depths up to `depth`.
+uint32_t trace_stack_entries(int depth);
 // The canonical node records of an octree (tsi_read_nodes): every node reachable from the root
 // through nodes with children, keyed by (depth, i, j, k).  Synchronous device reads.
 int read_octree(const float4 *st_dev, const float4 *grad_dev, const Counters *cnt_dev, uint64_t nodes, tsi_node *out,

@@ -104,15 +104,12 @@ struct tsi_ctx {
     // events around each level's launch (tsi_stats.eval_kernel_ms as the levels' summed kernel
     // time); $TSI_LEVEL_EVENTS=0 leaves them out (eval_kernel_ms is then the levels' span)
     bool level_events = true;
-    // The trace's form.  A full launch of 16x16-pixel blocks fills every CU's wave slots while
-    // blocks are pending, and the next frame's level kernels, launched beside it, wait for slots;
-    // the persistent form on one block per CU leaves them free but, with fewer wavefronts, takes
-    // ~15 % longer.  It is chosen while its trace time stays under 1.6 set inversions (the two
-    // trace slots then keep up), from the last frame's measured times; $TSI_TRACE_BLOCKS fixes
-    // it (0: full launches; n: the persistent form on n blocks per CU).
+    // The form of a trace that overlaps set inversions.  A full launch fills every CU's wave slots
+    // while blocks are pending, and the next frame's level kernels, launched beside it, wait for
+    // slots; persistent wavefronts leave some free (start_trace).  $TSI_TRACE_BLOCKS fixes it for
+    // every trace (0: full launches; n: 4 n persistent wavefronts per CU).
     int trace_blocks_env = -1;
-    bool trace_persistent = false;
-    float last_si_ms = 0.0f;
+    int depth_seen = 0;                 // the deepest frame since the reset: no node lies deeper
     // the pass runs on its own stream with its own saved-operand stack (one block per CU), after
     // the previous frame's levels up to spec_max have run (spec_ready, recorded by that frame)
     hipStream_t spec_stream = nullptr;
@@ -131,7 +128,6 @@ struct tsi_ctx {
     uint32_t grid_fwd = 0, grid_rev = 0, grid_misc = 0;
     uint64_t last_visits = 0;
     double last_trace_ms = 0.0;
-    bool last_trace_persistent = false;
     uint64_t used_nodes = 8;            // nodes in use after the last collected set inversion
     double trace_ms_total = 0.0;
     uint64_t trace_visits_total = 0, trace_count = 0;
@@ -158,7 +154,6 @@ struct tsi_ctx {
         float *depth = nullptr;
         size_t px = 0;
         unsigned long long *visits = nullptr;
-        bool persistent = false;   // traced by k_trace_quads
     };
     static constexpr uint32_t kFrameSlots = 2, kTraceSlots = 2;
     FrameSlot fslot[kFrameSlots];
@@ -734,6 +729,7 @@ int tsi_reset(tsi_ctx *c, const float root_box[6]) {
     std::memcpy(c->root_box, root_box, sizeof c->root_box);
     c->t_seen_lo = 1.0f;
     c->t_seen_hi = 0.0f;
+    c->depth_seen = 0;
     return TSI_OK;
 }
 
@@ -795,6 +791,7 @@ int tsi_set_inversion_async(tsi_ctx *c) {
     KArgs a = make_args(c);
     SpecLaunch sl{};
     f.spec = spec_active(c);
+    if (c->p.localsubdiv > c->depth_seen) c->depth_seen = c->p.localsubdiv;
     if (f.spec) {
         a.spec_levels = std::min<uint32_t>(c->spec_max, uint32_t(c->p.localsubdiv - 1));
         a.spec_cap = c->spec_cap;
@@ -837,7 +834,6 @@ int tsi_set_inversion_result(tsi_ctx *c, double *gpu_ms, tsi_stats *stats) {
     const CounterHead &h = *f.h;
     float ms = 0.0f, ems = 0.0f;
     hipEventElapsedTime(&ms, f.begin, f.end);
-    c->last_si_ms = ms;
     hipEventElapsedTime(&ems, f.eval0, f.eval1);
     if (gpu_ms) *gpu_ms = ms;
     if (stats) {
@@ -900,7 +896,6 @@ int harvest_trace(tsi_ctx *c) {
     for (uint32_t k = 0; k < kVisitSlots; ++k) visits += t.visits_h[k * kTallyStride];
     c->last_visits = visits;
     c->last_trace_ms = tms;
-    c->last_trace_persistent = t.persistent;
     c->trace_ms_total += tms;
     c->trace_visits_total += visits;
     c->trace_count += 1;
@@ -979,20 +974,18 @@ int start_trace(tsi_ctx *c, bool overlap) {
     t.shading = c->p.shading;
     t.grad = grad;
     t.visit_slots = kVisitSlots;
+    t.stack = trace_stack_entries(c->depth_seen);
     HIP_OK(hipMemsetAsync(ts.visits, 0, kTraceCounters * sizeof(unsigned long long), s));
     HIP_OK(hipEventRecord(ts.begin, s));
     uint32_t blocks = 0;
     if (c->trace_blocks_env >= 0) {
-        blocks = uint32_t(c->trace_blocks_env) * uint32_t(c->num_cu);
-    } else if (overlap && c->last_si_ms > 0.0f && c->last_trace_ms > 0.0f) {
-        // the persistent form's expected time, from the last trace in either form (+/-10 %
-        // hysteresis around the switch)
-        const float tp = c->last_trace_persistent ? c->last_trace_ms : 1.15f * c->last_trace_ms;
-        const float limit = 1.6f * c->last_si_ms * (c->trace_persistent ? 1.1f : 0.9f);
-        c->trace_persistent = tp < limit;
-        blocks = c->trace_persistent ? uint32_t(c->num_cu) : 0u;
+        blocks = 4u * uint32_t(c->trace_blocks_env) * uint32_t(c->num_cu);
+    } else if (overlap && !trace_quads(t)) {
+        // beside the next frame's levels: persistent wavefronts, 3 per SIMD, leave them slots
+        // (4 frames of a mixed scene with gradients 1.91 ms; full launches 2.10, one per SIMD 2.25;
+        // elsewhere, up to 1920x1080 and 8 CSG frames at 1024^3, within 4 % of full launches)
+        blocks = 12u * uint32_t(c->num_cu);
     }
-    ts.persistent = blocks != 0;
     if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + kVisitSlots * kTallyStride)) != 0) return TSI_E_HIP;
     HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, kVisitBytes, hipMemcpyDeviceToHost, s));
     HIP_OK(hipEventRecord(ts.end, s));

@@ -27,6 +27,7 @@ namespace {
 
 constexpr float kTrEps = 0.0001f;     // compute.wgsl:4140
 constexpr float kDarken = 0.98f;      // compute.wgsl:3507
+constexpr uint32_t kTraceThreads = 64;   // a wavefront: see k_trace
 constexpr uint32_t kStackDepth = 16;  // compute.wgsl's stack: a push on a full one is dropped
 
 // ---------------------------------------------------------------- layouts of a ray's vectors
@@ -118,19 +119,19 @@ struct LaneG {
     // entries are {node, children word}.
     struct Stack {
         uint2 *base;   // entry 0 of this lane
-        TSI_DI void put(uint32_t s, uint32_t node, uint32_t meta, V, V) const { base[s * 256u] = make_uint2(node, meta); }
-        TSI_DI uint2 node(uint32_t s) const { return base[s * 256u]; }
+        TSI_DI void put(uint32_t s, uint32_t node, uint32_t meta, V, V) const { base[s * kTraceThreads] = make_uint2(node, meta); }
+        TSI_DI uint2 node(uint32_t s) const { return base[s * kTraceThreads]; }
         TSI_DI void box(const KArgs &a, uint32_t, uint32_t node, V &lo, V &hi) const {
             lo = load(a.blo, node);
             hi = load(a.bhi, node);
         }
         TSI_DI void put_box(uint32_t, V, V) const {}
         TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask, uint32_t oct) const {
-            base[s * 256u] = make_uint2(meta, mask | (oct << 8));
+            base[s * kTraceThreads] = make_uint2(meta, mask | (oct << 8));
         }
         TSI_DI void get(const KArgs &a, uint32_t s, uint32_t &meta, uint32_t &mask, V &lo, V &hi) const {
-            const uint2 e = base[s * 256u];
-            const uint32_t up = base[(s == 0u ? 0u : s - 1u) * 256u].x;
+            const uint2 e = base[s * kTraceThreads];
+            const uint32_t up = base[(s == 0u ? 0u : s - 1u) * kTraceThreads].x;
             const uint32_t node = s == 0u ? 0u : (up - 1u) * 8u + (e.y >> 8);
             meta = e.x;
             mask = e.y & 0xFFu;
@@ -221,21 +222,21 @@ struct QuadG {
         uint2 *base;   // entry 0 of this lane
         TSI_DI void put(uint32_t s, uint32_t node, uint32_t meta, V lo, V hi) const {
             const bool w = fourth();
-            base[s * 256u] = make_uint2(w ? node : __float_as_uint(lo), w ? meta : __float_as_uint(hi));
+            base[s * kTraceThreads] = make_uint2(w ? node : __float_as_uint(lo), w ? meta : __float_as_uint(hi));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        TSI_DI uint2 node(uint32_t s) const { return base[s * 256u + 3u - (threadIdx.x & 3u)]; }
+        TSI_DI uint2 node(uint32_t s) const { return base[s * kTraceThreads + 3u - (threadIdx.x & 3u)]; }
         TSI_DI void box(const KArgs &, uint32_t s, uint32_t, V &lo, V &hi) const {
-            const uint2 b = base[int32_t(s * 256u) - (fourth() ? 1 : 0)];
+            const uint2 b = base[int32_t(s * kTraceThreads) - (fourth() ? 1 : 0)];
             lo = __uint_as_float(b.x);
             hi = __uint_as_float(b.y);
         }
         TSI_DI void put_box(uint32_t s, V lo, V hi) const {
-            if (!fourth()) base[s * 256u] = make_uint2(__float_as_uint(lo), __float_as_uint(hi));
+            if (!fourth()) base[s * kTraceThreads] = make_uint2(__float_as_uint(lo), __float_as_uint(hi));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
         TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask, uint32_t) const {
-            if (fourth()) base[s * 256u] = make_uint2(meta, mask);
+            if (fourth()) base[s * kTraceThreads] = make_uint2(meta, mask);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
         TSI_DI void get(const KArgs &a, uint32_t s, uint32_t &meta, uint32_t &mask, V &lo, V &hi) const {
@@ -323,7 +324,7 @@ TSI_DI float clamp01(float x) { return wmax(wmin(x, 1.0f), 0.0f); }
 template <class G, bool CIN>
 TSI_DI void walk_exact(const KArgs &a, typename G::Stack stk, typename G::V ro, typename G::V rd,
                                         float time, typename G::V &col, float &dist, uint32_t &visits,
-                                        uint32_t shading, const float4 *grad, typename G::V &nrm) {
+                                        uint32_t shading, const float4 *grad, uint32_t stack, typename G::V &nrm) {
     typedef typename G::V V;
     const bool normal_viz = (shading & TSI_SHADE_NORMALS) != 0;
     nrm = G::pick(0.0f, 0.0f, 0.0f);
@@ -404,7 +405,7 @@ TSI_DI void walk_exact(const KArgs &a, typename G::Stack stk, typename G::V ro, 
                         if (cmeta != 0u) {
                             // the walked node goes back on the stack (its entry is still there), then the child
                             ++sp;
-                            if (sp != kStackDepth) {
+                            if (sp < stack) {   // (TraceArgs::stack: full only where the reference's is)
                                 stk.put(sp, child, cmeta, lo, hi);
                                 ++sp;
                             }
@@ -559,7 +560,7 @@ TSI_DI bool walk_fast(const KArgs &a, const TraceArgs &ta, typename G::Stack stk
                 own = true;
                 entered = true;
                 ++d;
-                if (d == kStackDepth - 1u) {   // (walk_exact knows what a full stack does)
+                if (d == ta.stack - 1u) {   // (walk_exact knows what a full stack does)
                     ok = false;
                     break;
                 }
@@ -603,7 +604,7 @@ TSI_DI void trace_ray(const KArgs &a, const TraceArgs &ta, typename G::Stack stk
     uint32_t n = 0;
     if (!walk_fast<G, CIN>(a, ta, stk, ro, rd, col, dist, n, nrm)) {
         n = 0;
-        walk_exact<G, CIN>(a, stk, ro, rd, ta.time, col, dist, n, ta.shading, ta.grad, nrm);
+        walk_exact<G, CIN>(a, stk, ro, rd, ta.time, col, dist, n, ta.shading, ta.grad, ta.stack, nrm);
     }
     visits += n;
 }
@@ -848,27 +849,27 @@ TSI_DI void add_visits(const TraceArgs &t, uint32_t visits) {
 
 }  // namespace
 
-// One block per square of 2x2 wavefronts' tiles.
+// One wavefront per block: a block of four keeps its LDS (the ray stacks: 8 KB a wavefront) until its
+// slowest wavefront is done, and with times of 40 to 110 us a SIMD held 1.9 wavefronts on average
+// where 5 fit.
 template <class G, bool CIN>
-__global__ void __launch_bounds__(256) k_trace(KArgs a, TraceArgs t) {
-    __shared__ uint2 stack_lds[kStackDepth * 256u];
+__global__ void __launch_bounds__(kTraceThreads) k_trace(KArgs a, TraceArgs t) {
+    extern __shared__ uint2 stack_lds[];
     constexpr uint32_t side = G::kLanes == 1u ? 8u : 4u;
-    const uint32_t w = threadIdx.x >> 6;
     uint32_t visits = 0;
-    shade_tile<G, CIN>(a, t, (blockIdx.x * 2u + (w & 1u)) * side, (blockIdx.y * 2u + (w >> 1)) * side,
-                       typename G::Stack{stack_lds + threadIdx.x}, visits);
+    shade_tile<G, CIN>(a, t, blockIdx.x * side, blockIdx.y * side, typename G::Stack{stack_lds + threadIdx.x}, visits);
     add_visits<G>(t, visits);
 }
 
-// The same pixels on a grid of a few blocks per CU: each wavefront claims 8x8-pixel quadrants
+// The same pixels on a grid of a few wavefronts per CU: each claims 8x8-pixel quadrants
 // (row-major over the frame, dealt to kTraceQueues counters) until none is left.  A full launch keeps every CU's
 // wave slots filled with trace wavefronts while any block is pending, so the next frame's level
 // kernels, launched beside it, wait for slots; this leaves the CUs most of their slots.  Each pixel
 // is shaded by the same code as in k_trace: the frame is the same.
 template <bool CIN>
-__global__ void __launch_bounds__(256) k_trace_quads(KArgs a, TraceArgs t, uint32_t *next_quad, uint32_t quads_x,
+__global__ void __launch_bounds__(kTraceThreads) k_trace_quads(KArgs a, TraceArgs t, uint32_t *next_quad, uint32_t quads_x,
                                                      uint32_t nquads) {
-    __shared__ uint2 stack_lds[kStackDepth * 256u];
+    extern __shared__ uint2 stack_lds[];
     const uint32_t queue = blockIdx.x % kTraceQueues;
     uint32_t visits = 0;
     for (;;) {
@@ -881,14 +882,14 @@ __global__ void __launch_bounds__(256) k_trace_quads(KArgs a, TraceArgs t, uint3
     add_visits<LaneG>(t, visits);
 }
 
-// The frames of a batch in one launch: block i is a 16x16-pixel block of the frame whose blocks
-// [jobs[j].block0, jobs[j + 1].block0) hold it, row-major over ceil(width / 16) blocks per row,
-// and its wavefronts take the 8x8 quadrants, as k_trace's do (a persistent grid taking tiles
+// The frames of a batch in one launch: block i is an 8x8-pixel tile of the frame whose blocks
+// [jobs[j].block0, jobs[j + 1].block0) hold it, row-major over ceil(width / 8) blocks per row
+// (a persistent grid taking tiles
 // from a counter measured slower: a frame's slowest tiles then ran one after another in a few
 // wavefronts, where the hardware dispatcher starts each block on the first free slot).
 template <bool CIN>
-__global__ void __launch_bounds__(256) k_trace_batch(const TraceJob *jobs, uint32_t njobs) {
-    __shared__ uint2 stack_lds[kStackDepth * 256u];
+__global__ void __launch_bounds__(kTraceThreads) k_trace_batch(const TraceJob *jobs, uint32_t njobs) {
+    extern __shared__ uint2 stack_lds[];
     const uint32_t blk = blockIdx.x;
     uint32_t lo = 0, hi = njobs;   // last job with block0 <= blk
     while (hi - lo > 1u) {
@@ -915,10 +916,10 @@ __global__ void __launch_bounds__(256) k_trace_batch(const TraceJob *jobs, uint3
     t.mask = J.t.mask;
     t.mask_stride = J.t.mask_stride;
     t.visit_slots = J.t.visit_slots;
+    t.stack = J.t.stack;
     const uint32_t local = blk - J.block0;
-    const uint32_t w = threadIdx.x >> 6;
     uint32_t visits = 0;
-    shade_tile<LaneG, CIN>(a, t, (local % J.blocks_x) * 16u + (w & 1u) * 8u, (local / J.blocks_x) * 16u + (w >> 1) * 8u,
+    shade_tile<LaneG, CIN>(a, t, (local % J.blocks_x) * kTraceTile, (local / J.blocks_x) * kTraceTile,
                            LaneG::Stack{stack_lds + threadIdx.x}, visits);
     add_visits<LaneG>(t, visits);
 }
@@ -926,34 +927,47 @@ __global__ void __launch_bounds__(256) k_trace_batch(const TraceJob *jobs, uint3
 // ---------------------------------------------------------------- launchers
 
 // Frames of at most this many pixels are traced with four lanes per ray: their wavefronts then
-// still have a SIMD each, and the frame takes the latency of its longest chains (64x48: 36 against
-// 43 us).  Larger frames are bound by instructions (256x256: 100 against 90 us).
-constexpr uint64_t kQuadPixels = 32768;
+// still find free SIMDs, and the frame takes the latency of its longest chains, which are shorter so
+// (64x48: 36 against 43 us; spheres at 256x256: 113 against 137).  Larger frames are bound by
+// instructions (capsules at 300x300: 366 against 364 us, at 448x448 573 against 389).  A path-traced
+// pixel is 8 samples of up to 4 rays, chains so long that the line lies higher (csg at 320x200: 6.4
+// against 8.0 ms, at 641x361 8.5 against 8.2, spheres 2.5 against 2.8; at 960x540 12.6 against 9.3).
+constexpr uint64_t kQuadPixels = 98304, kQuadPixelsCinematic = 262144;
 
-int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, hipStream_t s) {
-    if (cinematic) hipLaunchKernelGGL(k_trace_batch<true>, dim3(total_blocks), dim3(256), 0, s, jobs, njobs);
-    else hipLaunchKernelGGL(k_trace_batch<false>, dim3(total_blocks), dim3(256), 0, s, jobs, njobs);
+// LDS of a wavefront's ray stacks: entries x 64 lanes x 8 B.
+static uint32_t stack_bytes(uint32_t entries) { return entries * kTraceThreads * uint32_t(sizeof(uint2)); }
+
+uint32_t trace_stack_entries(int depth) { return std::min(kStackDepth, uint32_t(depth) + 3u); }
+
+int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, uint32_t stack,
+                       hipStream_t s) {
+    if (cinematic) hipLaunchKernelGGL(k_trace_batch<true>, dim3(total_blocks), dim3(kTraceThreads), stack_bytes(stack), s, jobs, njobs);
+    else hipLaunchKernelGGL(k_trace_batch<false>, dim3(total_blocks), dim3(kTraceThreads), stack_bytes(stack), s, jobs, njobs);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+bool trace_quads(const TraceArgs &t) {
+    return uint64_t(t.width) * t.height <= (t.shading & TSI_SHADE_CINEMATIC ? kQuadPixelsCinematic : kQuadPixels);
 }
 
 int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blocks, uint32_t *next_quad) {
     const bool cin = (t.shading & TSI_SHADE_CINEMATIC) != 0;
     if (blocks && next_quad) {   // persistent: `blocks` blocks, *next_quad zeroed on the stream before
         const uint32_t qx = (t.width + 7u) / 8u, nq = qx * ((t.height + 7u) / 8u);
-        const uint32_t nb = std::min(blocks, std::max(kTraceQueues, (nq + 3u) / 4u));   // (a block for every queue)
-        if (cin) hipLaunchKernelGGL(k_trace_quads<true>, dim3(nb), dim3(256), 0, s, a, t, next_quad, qx, nq);
-        else hipLaunchKernelGGL(k_trace_quads<false>, dim3(nb), dim3(256), 0, s, a, t, next_quad, qx, nq);
+        const uint32_t nb = std::min(blocks, std::max(kTraceQueues, nq));   // (a block for every queue)
+        if (cin) hipLaunchKernelGGL(k_trace_quads<true>, dim3(nb), dim3(kTraceThreads), stack_bytes(t.stack), s, a, t, next_quad, qx, nq);
+        else hipLaunchKernelGGL(k_trace_quads<false>, dim3(nb), dim3(kTraceThreads), stack_bytes(t.stack), s, a, t, next_quad, qx, nq);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
-    const bool quad = uint64_t(t.width) * t.height <= kQuadPixels;
-    const uint32_t tile = quad ? 8u : 16u;
+    const bool quad = trace_quads(t);
+    const uint32_t tile = quad ? 4u : 8u;
     const dim3 grid((t.width + tile - 1u) / tile, (t.height + tile - 1u) / tile);
     if (quad) {
-        if (cin) hipLaunchKernelGGL((k_trace<QuadG, true>), grid, dim3(256), 0, s, a, t);
-        else hipLaunchKernelGGL((k_trace<QuadG, false>), grid, dim3(256), 0, s, a, t);
+        if (cin) hipLaunchKernelGGL((k_trace<QuadG, true>), grid, dim3(kTraceThreads), stack_bytes(t.stack), s, a, t);
+        else hipLaunchKernelGGL((k_trace<QuadG, false>), grid, dim3(kTraceThreads), stack_bytes(t.stack), s, a, t);
     } else {
-        if (cin) hipLaunchKernelGGL((k_trace<LaneG, true>), grid, dim3(256), 0, s, a, t);
-        else hipLaunchKernelGGL((k_trace<LaneG, false>), grid, dim3(256), 0, s, a, t);
+        if (cin) hipLaunchKernelGGL((k_trace<LaneG, true>), grid, dim3(kTraceThreads), stack_bytes(t.stack), s, a, t);
+        else hipLaunchKernelGGL((k_trace<LaneG, false>), grid, dim3(kTraceThreads), stack_bytes(t.stack), s, a, t);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
