@@ -18,6 +18,7 @@
 //   reverse(a, stk, sens[4], Rlo, Rhi) -> algorithmic f32 ops; sensitivities of x, y, z, t
 //   (Rlo/Rhi: a register file the engine may use between the two calls)
 //   records()                      records run per forward pass
+//   kTimed                         its level kernels keep the time (level_clock)
 //   choices_recorded()             the forward pass recorded the MIN/MAX choices
 //   hold_choices()                 keeps them: the next forward pass records none (kSkip)
 //   liveness(a, rec, cap)          the cell's liveness record (kPrune engines), word w at
@@ -62,6 +63,27 @@ TSI_DI uint32_t dealloc_step(const KArgs &a, int step, uint32_t wave, uint32_t n
 
 // Levels from which a launch claims its blocks ahead: above, a level has at most 8^4 / 8 groups.
 static constexpr int kClaimLevel = 5;
+
+// The cascade's last two steps in one (after the frame's last level, which drops the last blocks):
+// the blocks of list `step` and the child blocks of their nodes are freed.
+TSI_DI uint32_t dealloc_tail(const KArgs &a, int step, uint32_t wave, uint32_t nwaves) {
+    Counters *cnt = a.cnt;
+    const uint32_t count = min(cnt->level[step].dlist, a.dlist_cap);
+    const uint32_t *in = a.dlists[step & 1];
+    const uint32_t lane = lane_id();
+    const uint32_t o = lane & 7u;
+    uint32_t freed = 0;
+    for (uint32_t g = wave; g * 8u < count; g += nwaves) {
+        const uint32_t idx = g * 8u + (lane >> 3);
+        const bool active = idx < count;
+        const uint32_t b = active ? in[idx] : 0u;
+        const uint32_t m = active ? meta_of(a.st[b * 8u + o]) & kChildMask : 0u;
+        wave_append(m != 0, m - 1u, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
+        wave_append(active && o == 0, b, a.pending_free, &cnt->pending, a.nblocks, &cnt->frame_error, kErrQueue);
+        freed += popc64(ballot(active && o == 0)) + popc64(ballot(m != 0));
+    }
+    return freed;
+}
 
 // A wavefront's tallies of the cells it processed: counts of its lanes (uniform, from ballots) and
 // per-lane sums of work; added to the frame's statistics once (flush_tally).
@@ -417,7 +439,8 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
 
 // Adds a wavefront's tallies to the block's slot of the frame's statistics: one atomic instruction,
 // lane k adding statistic k.
-TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t) {
+// level >= 0: of a timed level kernel: also the time, the latest of the wavefronts' (level_clock).
+TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t, int level = -1) {
     const uint64_t rev_ops = wave_sum64(t.rev_ops), fwd_ops = wave_sum64(t.fwd_ops), pruned = wave_sum64(t.pruned);
     const uint32_t k = lane_id();
     uint64_t v = 0;
@@ -430,9 +453,35 @@ TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t) {
     v = k == kStatFwdOps ? fwd_ops : v;
     v = k == kStatPruned ? pruned : v;
     v = k == kStatSpec ? t.spec : v;
-    if (v)
-        atomicAdd(reinterpret_cast<unsigned long long *>(tally + (blockIdx.x % kTallySlots) * kTallyStride + k),
-                  (unsigned long long)v);
+    uint64_t *slot = tally + (blockIdx.x % kTallySlots) * kTallyStride;
+    if (v) atomicAdd(reinterpret_cast<unsigned long long *>(slot + k), (unsigned long long)v);
+    if (level >= 0 && k == 0)
+        atomicMax(reinterpret_cast<unsigned long long *>(slot + kNumStats + (level & 1)),
+                  (unsigned long long)__builtin_amdgcn_s_memrealtime());
+}
+
+// The level kernels' time without events between them (3.2 us each, two a level: an eighth of a
+// 256 x 256 preview).  One wavefront of a level's launch notes when it began and, from the latest end
+// of the level before (two words per slot in turn: nothing of this level writes that one), adds
+// that level's time.  The last level's is added by the commit.
+TSI_DI uint64_t latest_end(const KArgs &a, int level) {
+    static_assert(kTallySlots == 64 && kNumStats + 2 <= kTallyStride, "a slot per lane, two words after the statistics");
+    uint64_t v = a.tally[lane_id() * kTallyStride + kNumStats + (level & 1)];
+    for (int d = 32; d; d >>= 1) {
+        const uint64_t o = uint64_t(__shfl_xor((unsigned long long)v, d, 64));
+        v = v > o ? v : o;
+    }
+    return v;
+}
+
+TSI_DI void level_clock(const KArgs &a, int level) {
+    const uint64_t now = __builtin_amdgcn_s_memrealtime();
+    const uint64_t end = level > 0 ? latest_end(a, level - 1) : 0u;
+    if (lane_id() != 0) return;
+    Counters *c = a.cnt;
+    if (level > 0 && end > c->clk_start) c->level_ticks += end - c->clk_start;
+    c->clk_start = now;
+    c->clk_level = level;
 }
 
 // Tickets for the new parents (entries without children) of this wavefront's groups: a look ahead
@@ -487,7 +536,7 @@ TSI_DI void eval_level(const KArgs &a, int level, float time, uint32_t wave_, ui
     //      descendants (forward-only kernel; the reverse kernel of the level does not touch the
     //      list, which the previous level's kernels finished) ----
     if (!REV && level > 0) tl.freed = dealloc_step(a, level, wave, nwaves);
-    flush_tally(a.tally, tl);
+    flush_tally(a.tally, tl, Engine::kTimed ? level : -1);
 }
 
 // The speculative pass's parents (KArgs::spec_*): every node at depth < spec_levels as the frame
@@ -548,6 +597,8 @@ TSI_DI void frame_begin(const KArgs &a, uint32_t t, uint32_t nt) {
         c->alloc_tickets = 0;
         c->pending = 0;
         c->frame_error = 0;
+        c->level_ticks = 0;
+        c->clk_level = -1;
         if (c->root_pending) {
             c->root_pending = 0;
             const float4 s = a.st[0];
@@ -583,7 +634,9 @@ TSI_DI void frame_commit(const KArgs &a) {
         for (uint32_t i = 0; i < kTallySlots; ++i) v += a.tally[i * kTallyStride + k];
         cnt->stats[k] = v;
     }
+    const uint64_t end = cnt->clk_level >= 0 ? latest_end(a, cnt->clk_level) : 0u;
     if (k != 0) return;
+    if (end > cnt->clk_start) cnt->level_ticks += end - cnt->clk_start;
     const uint32_t T = cnt->alloc_tickets, F = cnt->free_top, P = min(cnt->pending, a.nblocks);
     const uint32_t used = T < F ? T : F;
     uint32_t bump = cnt->bump + (T > F ? T - F : 0u);

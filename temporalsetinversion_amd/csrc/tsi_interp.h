@@ -344,7 +344,7 @@ TSI_DI void live_walk(const FwdIns *prog, uint32_t n, uint32_t out_slot, const C
 
 // ---- the interpreter as an evaluation engine of eval_level --------------------------------
 struct InterpEngine {
-    static constexpr bool kPrune = true, kSkip = false, kExactT = false;
+    static constexpr bool kPrune = true, kSkip = false, kExactT = false, kTimed = false;
     static constexpr uint32_t kRecWords = 0;
     TSI_DI void hold_choices() {}
     const FwdIns *fprog;

@@ -1658,7 +1658,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         uint64_t full_cost = 0;
         for (uint32_t j = 4; j < n; ++j) full_cost += fwd[j - 4].cost;
         o += "struct TapeEngine {\n    static constexpr bool kPrune = true, kSkip = true, kExactT = " + std::string(CH.exact_t ? "true" : "false") +
-             ";\n    static constexpr uint32_t kRecWords = " + RWs + "u;\n"
+             ", kTimed = true;\n    static constexpr uint32_t kRecWords = " + RWs + "u;\n"
              "    uint32_t lane;\n    const uint32_t *lrec;\n    uint32_t *colbase, *cols;\n    RegionMask mask;\n"
              "    uint32_t live, rows, nrec;\n    bool act, ran;\n"
              "    template <class KA>\n    TSI_DI TapeEngine(const KA &a, uint32_t wave, uint32_t l)\n"
@@ -1709,7 +1709,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
              "};\n\n}  // namespace tsi\n\n";
     } else {
     // ---- the evaluation engine of eval_level (tsi_eval.h) ----
-    o += std::string("struct TapeEngine {\n    static constexpr bool kPrune = ") + (prune ? "true" : "false") + ", kSkip = false, kExactT = false;\n    static constexpr uint32_t kRecWords = 0u;\n    TSI_DI void hold_choices() {}\n";
+    o += std::string("struct TapeEngine {\n    static constexpr bool kPrune = ") + (prune ? "true" : "false") + ", kSkip = false, kExactT = false, kTimed = true;\n    static constexpr uint32_t kRecWords = 0u;\n    TSI_DI void hold_choices() {}\n";
     o += "    static constexpr uint32_t kRegions = " + std::to_string(Y.regions) + "u;\n";
     o += "    uint32_t lane, recs;\n    const uint32_t *prec;\n    uint32_t *chbuf;\n    RegionMask mask;\n"
          "    uint32_t variant;   // this wavefront's: 0 full, 1 full + choices, 2 pruned\n";
@@ -1813,6 +1813,7 @@ std::string jit_source_level(const tsi_gpu_instruction *tape, uint32_t n, const 
     o += "    const uint32_t nb = gridDim.x, b = blockIdx.x, w = threadIdx.x >> 6;\n"
          "    // level -1: the frame's speculative pass, on the whole grid (reverse list code)\n"
          "    const uint32_t nf = level < 0 ? 0u : __builtin_amdgcn_readfirstlane(tsi::level_split(a, level, nb));\n"
+         "    if (level >= 0 && b == nb - 1u && w == 3u) tsi::level_clock(a, level);\n"
          "    const uint32_t bwave = b * 4u + w;\n"
          "    if (b < nf)\n"
          "        tsi::eval_level<false, tsi::jf::TapeEngine>(a, level, time, bwave, nf * 4u, bwave);\n"

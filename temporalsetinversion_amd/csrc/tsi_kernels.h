@@ -44,6 +44,7 @@ struct CounterHead {
     uint32_t error;                           // sticky kErr* since reset
     uint32_t root_pending;                    // buf_main has enqueued the root
     uint32_t pad;
+    uint64_t level_ticks;                     // the compiled level kernels' time, 10 ns (level_clock)
     uint64_t stats[kNumStats];
 };
 // Each counter that a level's wavefronts add to has a 128-byte line of its own, and none shares it
@@ -53,6 +54,9 @@ struct CounterHead {
 struct Counters : CounterHead {
     alignas(128) uint32_t alloc_tickets;      // blocks handed out this frame
     alignas(128) uint32_t pending;            // blocks freed this frame
+    alignas(128) uint32_t finished;           // blocks of k_frame_end that are done
+    alignas(128) uint64_t clk_start;          // when the level kernel running now began (level_clock)
+    int32_t clk_level;
     struct Level {
         alignas(128) uint32_t list[2];        // frontier sizes: [0] forward-only, [1] reverse
         alignas(128) uint32_t dlist;          // dealloc cascade list size

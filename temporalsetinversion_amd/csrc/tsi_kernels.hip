@@ -10,8 +10,8 @@
 //                            live values in a uniformly indexed VGPR file), then the cell is
 //                            classified; subdivision / dealloc outputs are compacted with
 //                            wavefront ballots + one atomic per wave and list
-//   k_dealloc x levels       the dealloc cascade of compute.wgsl:3533-3543 / 4036-4044
-//   k_frame_end/commit       free-list merge
+//   k_dealloc                the end of the dealloc cascade of compute.wgsl:3533-3543 / 4036-4044
+//   k_frame_end              free-list merge, commit
 // Frontier lists are split by whether the children will need the reverse pass, so the
 // forward-only kernel carries no reverse-mode code or stack traffic.
 #include <hip/hip_runtime.h>
@@ -134,22 +134,35 @@ __global__ void __launch_bounds__(256) k_prune(KArgs a, int level, int which) {
     }
 }
 
-// The dealloc cascade's steps after the last level (dealloc_step, tsi_eval.h).
+// The dealloc cascade's steps after the last level (dealloc_tail, tsi_eval.h).
 __global__ void __launch_bounds__(256) k_dealloc(KArgs a, int step) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     LevelTally tl;
-    tl.freed = dealloc_step(a, step, wave, nwaves);
+    tl.freed = dealloc_tail(a, step, wave, nwaves);
     if (tl.freed) flush_tally(a.tally, tl);
 }
 
-// Free-list merge and counter commit at the end of a frame (frame_end / frame_commit, tsi_eval.h).
-__global__ void __launch_bounds__(256) k_frame_end(KArgs a) {
+// The end of a frame: free-list merge (frame_end, tsi_eval.h) and, by the block that finishes last,
+// the commit of the counters and the copy of what the host reads, into its memory (out).
+// A launch and a copy kernel less than apart: 10 us of a frame's 300 at 256 x 256.
+__global__ void __launch_bounds__(256) k_frame_end(KArgs a, CounterHead *out) {
+    __shared__ uint32_t last;
     frame_end(a, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(&a.cnt->finished, 1u) == gridDim.x - 1u;
+    }
+    __syncthreads();
+    if (!last || threadIdx.x >= 64u) return;
+    __threadfence();
+    frame_commit(a);
+    if (threadIdx.x == 0) a.cnt->finished = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the lanes' writes, for the copy
+    const uint32_t *from = reinterpret_cast<const uint32_t *>(a.cnt);
+    for (uint32_t i = threadIdx.x; i < uint32_t(sizeof(CounterHead) / 4u); i += 64u) reinterpret_cast<uint32_t *>(out)[i] = from[i];
 }
-
-__global__ void k_frame_commit(KArgs a) { frame_commit(a); }
-
 __global__ void k_clear_nodes(KArgs a, uint64_t n) {
     for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x) {
         a.st[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -253,10 +266,8 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
     if (e_eval1) hipEventRecord(e_eval1, s);
     // levels 1..L-1 ran the cascade's steps 1..L-1 (eval_level); blocks dropped by the last
     // level and the descendants of earlier drops need at most two more
-    for (int c = fl.levels; c <= fl.levels + 1; ++c)
-        hipLaunchKernelGGL(k_dealloc, dim3(fl.grid_misc), dim3(256), 0, s, a, c);
-    hipLaunchKernelGGL(k_frame_end, dim3(fl.grid_misc), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_frame_commit, dim3(1), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(k_dealloc, dim3(fl.grid_misc), dim3(256), 0, s, a, fl.levels);
+    hipLaunchKernelGGL(k_frame_end, dim3(64), dim3(256), 0, s, a, fl.out);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -34,6 +34,7 @@ struct FrameLaunch {
     uint32_t grid_fwd, grid_rev, grid_misc;
     void *tape_eval;   // the tape's compiled level kernel (hipFunction_t), or null: k_eval
     const SpecLaunch *spec;   // or null
+    CounterHead *out;         // host memory (pinned): the counters after the frame
 };
 
 // e_eval0 / e_eval1 (may be null) bracket the level loop; e_level (may be null) holds an event
@@ -83,6 +84,9 @@ int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_bloc
 bool trace_quads(const TraceArgs &t);
 // TraceArgs::stack for an octree whose nodes lie at depths up to `depth`.
 uint32_t trace_stack_entries(int depth);
+// After a trace (visits as in TraceArgs): the visits' sum to *out (pinned host memory), and the counters
+// (n_clear words from visits on) cleared for the slot's next trace.
+int launch_trace_end(unsigned long long *visits, uint32_t n_clear, unsigned long long *out, hipStream_t s);
 // The canonical node records of an octree (tsi_read_nodes): every node reachable from the root
 // through nodes with children, keyed by (depth, i, j, k).  Synchronous device reads.
 int read_octree(const float4 *st_dev, const float4 *grad_dev, const Counters *cnt_dev, uint64_t nodes, tsi_node *out,

@@ -59,8 +59,10 @@ int scratch_setup(int device, uchar4 **out) {
 }  // namespace
 
 // A trace slot's counters: the node visits (TraceArgs::visits), then the persistent trace's claims.
-constexpr size_t kVisitBytes = size_t(tsi::kVisitSlots) * tsi::kTallyStride * sizeof(unsigned long long);
 constexpr size_t kTraceCounters = size_t(tsi::kVisitSlots + tsi::kTraceQueues) * tsi::kTallyStride;
+constexpr size_t kTallyBytes = size_t(tsi::kTallySlots) * tsi::kTallyStride * sizeof(uint64_t);
+constexpr uint32_t kTraceSlotCount = 2;
+constexpr size_t kCounterBytes = sizeof(tsi::Counters) + kTallyBytes + kTraceSlotCount * kTraceCounters * sizeof(unsigned long long);
 
 struct tsi_ctx {
     HostPoolUser pool_user;
@@ -76,6 +78,7 @@ struct tsi_ctx {
     uint32_t *lists[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     uint32_t *dlists[2] = {nullptr, nullptr};
     uint32_t *pending = nullptr, *free_stack = nullptr;
+    char *counters = nullptr;           // one allocation: Counters, tally, the trace slots' visits
     Counters *cnt = nullptr;
     uint64_t *tally = nullptr;          // KArgs::tally
     uchar4 *rgba8 = nullptr;            // tsi_frame_rgba8's image, grown to the largest frame asked for
@@ -101,8 +104,9 @@ struct tsi_ctx {
     uint32_t *spec_cnt = nullptr;
     SpecCell *spec_res = nullptr;
     uint32_t spec_cap = 0, spec_tag = 0, spec_max = 0;
-    // events around each level's launch (tsi_stats.eval_kernel_ms as the levels' summed kernel
-    // time); $TSI_LEVEL_EVENTS=0 leaves them out (eval_kernel_ms is then the levels' span)
+    // tsi_stats.eval_kernel_ms: the levels' summed kernel time, from events around each level's
+    // launches (interpreter) or the device's clock (compiled kernels, level_clock);
+    // $TSI_LEVEL_EVENTS=0: the levels' span, no events
     bool level_events = true;
     // The form of a trace that overlaps set inversions.  A full launch fills every CU's wave slots
     // while blocks are pending, and the next frame's level kernels, launched beside it, wait for
@@ -135,7 +139,8 @@ struct tsi_ctx {
     // and pinned host copies of what the host reads back
     struct FrameSlot {
         hipEvent_t begin = nullptr, end = nullptr, eval0 = nullptr, eval1 = nullptr;
-        hipEvent_t level[2 * kMaxLevels] = {};   // around each level's evaluation launches
+        hipEvent_t level[2 * kMaxLevels] = {};   // around each level's evaluation launches (interpreter)
+        bool timed = false, events = false;      // the levels' times from the device's clock / these events
         hipEvent_t spec0 = nullptr, spec1 = nullptr;   // around the speculative pass
         bool spec = false;                             // the frame had one
         CounterHead *h = nullptr;
@@ -155,7 +160,7 @@ struct tsi_ctx {
         size_t px = 0;
         unsigned long long *visits = nullptr;
     };
-    static constexpr uint32_t kFrameSlots = 2, kTraceSlots = 2;
+    static constexpr uint32_t kFrameSlots = 2, kTraceSlots = kTraceSlotCount;
     FrameSlot fslot[kFrameSlots];
     TraceSlot tslot[kTraceSlots];
     uint64_t f_issued = 0, f_done = 0, t_issued = 0, t_done = 0;
@@ -423,13 +428,13 @@ void release(tsi_ctx *c) {
         for (hipEvent_t *e : {&t.begin, &t.end, &t.snap})
             if (*e) { hipEventDestroy(*e); *e = nullptr; }
         if (t.visits_h) { hipHostFree(t.visits_h); t.visits_h = nullptr; }
-        dfree(t.st); dfree(t.blo); dfree(t.bhi); dfree(t.mask); dfree(t.grad); dfree(t.rgba); dfree(t.depth); dfree(t.visits);
+        dfree(t.st); dfree(t.blo); dfree(t.bhi); dfree(t.mask); dfree(t.grad); dfree(t.rgba); dfree(t.depth);
         if (t.stream) { hipStreamDestroy(t.stream); t.stream = nullptr; }
     }
     dfree(c->st); dfree(c->blo); dfree(c->bhi); dfree(c->grad);
     for (auto &l : c->lists) for (auto &x : l) dfree(x);
     dfree(c->dlists[0]); dfree(c->dlists[1]);
-    dfree(c->pending); dfree(c->free_stack); dfree(c->cnt); dfree(c->tally); dfree(c->rgba8); dfree(c->stack);
+    dfree(c->pending); dfree(c->free_stack); dfree(c->counters); dfree(c->rgba8); dfree(c->stack);
     dfree(c->spec_list); dfree(c->spec_cnt); dfree(c->spec_res); dfree(c->spec_stack);
     if (c->spec_ready) { hipEventDestroy(c->spec_ready); c->spec_ready = nullptr; }
     if (c->spec_stream) { hipStreamDestroy(c->spec_stream); c->spec_stream = nullptr; }
@@ -567,12 +572,13 @@ int tsi_create(const tsi_params *params, tsi_ctx **out) {
             for (hipEvent_t *e : {&f.eval0, &f.eval1, &f.spec0})
                 evok = evok && hipEventCreateWithFlags(e, hipEventDisableSystemFence) == hipSuccess;
             for (hipEvent_t &e : f.level)
-                evok = evok && hipEventCreateWithFlags(&e, hipEventDisableSystemFence) == hipSuccess;
+                if (params->flags & TSI_FLAG_INTERPRET)
+                    evok = evok && hipEventCreateWithFlags(&e, hipEventDisableSystemFence) == hipSuccess;
             evok = evok && hipHostMalloc((void **)&f.h, sizeof(CounterHead), hipHostMallocDefault) == hipSuccess;
         }
         for (auto &t : c->tslot) {
             for (hipEvent_t *e : {&t.begin, &t.end}) evok = evok && hipEventCreate(e) == hipSuccess;
-            evok = evok && hipHostMalloc((void **)&t.visits_h, kVisitBytes, hipHostMallocDefault) == hipSuccess;
+            evok = evok && hipHostMalloc((void **)&t.visits_h, sizeof *t.visits_h, hipHostMallocDefault) == hipSuccess;
         }
         if (!evok) { rc = TSI_E_HIP; break; }
         uint64_t nodes = params->voxel_capacity ? params->voxel_capacity : (uint64_t(1) << 24);
@@ -610,12 +616,20 @@ int tsi_create(const tsi_params *params, tsi_ctx **out) {
             break;
         if ((rc = dmalloc(&c->dlists[0], c->dlist_cap)) || (rc = dmalloc(&c->dlists[1], c->dlist_cap)) ||
             (rc = dmalloc(&c->pending, c->nblocks)) || (rc = dmalloc(&c->free_stack, c->nblocks)) ||
-            (rc = dmalloc(&c->cnt, 1)) || (rc = dmalloc(&c->tally, size_t(kTallySlots) * kTallyStride)))
+            (rc = dmalloc(&c->counters, kCounterBytes)))
             break;
-        for (auto &t : c->tslot)
-            if (!rc) rc = dmalloc(&t.visits, kTraceCounters);
-        if (rc) break;
-        if (hipMemsetAsync(c->cnt, 0, sizeof(Counters), c->stream) != hipSuccess) { rc = TSI_E_HIP; break; }
+        if (hipMemsetAsync(c->counters, 0, kCounterBytes, c->stream) != hipSuccess) { rc = TSI_E_HIP; break; }
+        {
+            char *at = c->counters;
+            c->cnt = reinterpret_cast<Counters *>(at);
+            at += sizeof(Counters);
+            c->tally = reinterpret_cast<uint64_t *>(at);
+            at += kTallyBytes;
+            for (auto &t : c->tslot) {
+                t.visits = reinterpret_cast<unsigned long long *>(at);
+                at += kTraceCounters * sizeof(unsigned long long);
+            }
+        }
         // level kernels stride over their frontier; 4 blocks (16 wavefronts) per CU for both lists
         // (measured: the reverse list of a large frontier needs 4 wavefronts per SIMD to hide its
         // latency, more only grows the saved-operand stack; the forward-only list is insensitive)
@@ -791,6 +805,8 @@ int tsi_set_inversion_async(tsi_ctx *c) {
     KArgs a = make_args(c);
     SpecLaunch sl{};
     f.spec = spec_active(c);
+    f.timed = c->eval_fn[0] != nullptr;
+    f.events = c->level_events && !f.timed;
     if (c->p.localsubdiv > c->depth_seen) c->depth_seen = c->p.localsubdiv;
     if (f.spec) {
         a.spec_levels = std::min<uint32_t>(c->spec_max, uint32_t(c->p.localsubdiv - 1));
@@ -816,10 +832,9 @@ int tsi_set_inversion_async(tsi_ctx *c) {
         c->spec_ready_recorded = true;
     }
     FrameLaunch fl{c->p.localsubdiv, c->u.time, c->grid_fwd, c->grid_rev, c->grid_misc,
-                   (void *)c->eval_fn[0], f.spec ? &sl : nullptr};
+                   (void *)c->eval_fn[0], f.spec ? &sl : nullptr, f.h};
     HIP_OK(hipEventRecord(f.begin, c->stream));
-    if (launch_frame(a, fl, c->stream, f.eval0, f.eval1, c->level_events ? f.level : nullptr) != 0) return TSI_E_HIP;
-    HIP_OK(hipMemcpyAsync(f.h, c->cnt, sizeof(CounterHead), hipMemcpyDeviceToHost, c->stream));
+    if (launch_frame(a, fl, c->stream, f.eval0, f.eval1, f.events ? f.level : nullptr) != 0) return TSI_E_HIP;
     HIP_OK(hipEventRecord(f.end, c->stream));
     c->f_issued += 1;
     return TSI_OK;
@@ -840,8 +855,8 @@ int tsi_set_inversion_result(tsi_ctx *c, double *gpu_ms, tsi_stats *stats) {
         std::memset(stats, 0, sizeof *stats);
         stats->gpu_ms = ms;
         stats->eval_ms = ems;
-        double kms = c->level_events ? 0.0 : double(ems);
-        for (int d = 0; c->level_events && d < c->p.localsubdiv; ++d) {
+        double kms = !c->level_events ? double(ems) : (f.timed ? 1e-5 * double(h.level_ticks) : 0.0);
+        for (int d = 0; f.events && d < c->p.localsubdiv; ++d) {
             float x = 0.0f;
             hipEventElapsedTime(&x, f.level[2 * d], f.level[2 * d + 1]);
             kms += x;
@@ -892,8 +907,7 @@ int harvest_trace(tsi_ctx *c) {
     HIP_OK(hipEventSynchronize(t.end));
     float tms = 0.0f;
     hipEventElapsedTime(&tms, t.begin, t.end);
-    uint64_t visits = 0;
-    for (uint32_t k = 0; k < kVisitSlots; ++k) visits += t.visits_h[k * kTallyStride];
+    const uint64_t visits = *t.visits_h;
     c->last_visits = visits;
     c->last_trace_ms = tms;
     c->trace_ms_total += tms;
@@ -975,7 +989,6 @@ int start_trace(tsi_ctx *c, bool overlap) {
     t.grad = grad;
     t.visit_slots = kVisitSlots;
     t.stack = trace_stack_entries(c->depth_seen);
-    HIP_OK(hipMemsetAsync(ts.visits, 0, kTraceCounters * sizeof(unsigned long long), s));
     HIP_OK(hipEventRecord(ts.begin, s));
     uint32_t blocks = 0;
     if (c->trace_blocks_env >= 0) {
@@ -987,7 +1000,7 @@ int start_trace(tsi_ctx *c, bool overlap) {
         blocks = 12u * uint32_t(c->num_cu);
     }
     if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + kVisitSlots * kTallyStride)) != 0) return TSI_E_HIP;
-    HIP_OK(hipMemcpyAsync(ts.visits_h, ts.visits, kVisitBytes, hipMemcpyDeviceToHost, s));
+    if (launch_trace_end(ts.visits, uint32_t(kTraceCounters), ts.visits_h, s) != 0) return TSI_E_HIP;
     HIP_OK(hipEventRecord(ts.end, s));
     c->last_tslot = k;
     c->t_issued += 1;
