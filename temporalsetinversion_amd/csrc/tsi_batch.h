@@ -138,7 +138,7 @@ TSI_DI uint32_t dealloc_group(const KA &a, int step, uint32_t g) {
     return popc64(ballot(active && o == 0));
 }
 
-// The persistent kernel's body.  Tapes::group<REV>(tape, a, level, time, g, count, stk, tally)
+// The persistent kernel's body.  Tapes::group<REV>(tape, a, level, time, g, count, stk, wave, tally)
 // runs eval_group with the tape's engine.  One block per CU, of 4, 8, 12 or 16 wavefronts (one
 // to four per SIMD).
 template <class Tapes>
@@ -238,9 +238,9 @@ TSI_DI void batch_run(const BatchArgs &b) {
                 LevelTally tl;
                 if (kind == 0u)
                     Tapes::template group<true>(tape, a, d, time, g,
-                                                d < 0 ? min(*a.spec_count, a.spec_cap) : list_entries(a, d, 1), stk, tl);
+                                                d < 0 ? min(*a.spec_count, a.spec_cap) : list_entries(a, d, 1), stk, bwave, tl);
                 else if (kind == 1u)
-                    Tapes::template group<false>(tape, a, d, time, g, list_entries(a, d, 0), stk, tl);
+                    Tapes::template group<false>(tape, a, d, time, g, list_entries(a, d, 0), stk, bwave, tl);
                 else
                     tl.freed = dealloc_group(a, d, g);
                 flush_tally(a.tally, tl);

@@ -132,6 +132,14 @@ struct tsi_batch {
     uint32_t *error_h = nullptr;                // BatchCtl::error of the run
     TraceJob *jobs_d = nullptr, *jobs_h = nullptr;
     unsigned long long *visits_d = nullptr, *visits_h = nullptr;
+    // records of chain tapes (JitChain), outside the arena: per session rec_stride words, four lists of
+    // rec_cap entries and the speculative pass's cells; a tape's words per entry (0: no chain), and
+    // the wavefronts' columns
+    uint32_t *rec = nullptr, *choice = nullptr;
+    size_t rec_stride = 0;
+    uint32_t rec_cap = 0, choice_len = 0;
+    bool rec_spec = false;
+    std::vector<uint32_t> rec_words, col_words;
     uint64_t *tally = nullptr;                  // each session's statistics (KArgs::tally)
     char *arena = nullptr;
     uint64_t arena_bytes = 0, arena_used = 0;
@@ -186,7 +194,7 @@ void release(tsi_batch *b) {
     if (b->mod) hipModuleUnload(b->mod);
     b->mod = nullptr;
     dfree(b->stack); dfree(b->sess_d); dfree(b->ctl); dfree(b->out_d); dfree(b->jobs_d);
-    dfree(b->visits_d); dfree(b->tally); dfree(b->arena);
+    dfree(b->visits_d); dfree(b->tally); dfree(b->rec); dfree(b->choice); dfree(b->arena);
     hfree(b->sess_h); hfree(b->out_h); hfree(b->error_h); hfree(b->jobs_h); hfree(b->visits_h);
     for (auto &e : b->ev)
         if (e) { hipEventDestroy(e); e = nullptr; }
@@ -221,6 +229,31 @@ void arena_give(tsi_batch *b, uint64_t off, uint64_t bytes) {
             prev->second += it->second;
             b->free_ranges.erase(it);
         }
+    }
+}
+
+// Records for up to 32 768 entries of each of a session's lists, fewer where many sessions share
+// 4 GiB (the speculative pass's cells first, if they take less than half).  Cells beyond them, or all (no memory), run the whole tape: the same results.
+void alloc_records(tsi_batch *b) {
+    uint32_t words = 0, cols = 0;
+    for (uint32_t w : b->rec_words) words = std::max(words, w);
+    for (uint32_t w : b->col_words) cols = std::max(cols, w);
+    if (!words) return;
+    const uint64_t budget = (uint64_t(4) << 30) / 4u / b->cfg.max_sessions;   // words per session
+    uint64_t spec = uint64_t(b->spec_cap) * 8u * words;
+    if (budget < 2u * spec) spec = 0;
+    b->rec_spec = spec != 0;
+    uint64_t cap = std::min<uint64_t>(32768u, (budget - spec) / (4u * words));
+    cap = cap / 8u * 8u;
+    if (cap < 64) return;
+    b->rec_cap = uint32_t(cap);
+    b->choice_len = cols;
+    b->rec_stride = size_t(4u * words * cap + spec);
+    if (dmalloc(&b->rec, b->rec_stride * b->cfg.max_sessions) != TSI_OK ||
+        dmalloc(&b->choice, size_t(b->num_cu) * b->max_bpc * 4u * 64u * cols) != TSI_OK) {
+        (void)hipGetLastError();
+        dfree(b->rec);
+        dfree(b->choice);
     }
 }
 
@@ -259,7 +292,20 @@ void session_args(const tsi_batch *b, Session &s, const Layout &L) {
     a.lipschitz = s.p.lipschitz_corrected;
     a.fastenabled = s.p.fastenabled;
     a.force_deriv = (s.p.shading & (TSI_SHADE_NORMALS | TSI_SHADE_CINEMATIC)) && (s.p.shading & TSI_SHADE_GRADIENT) ? 1 : 0;
-    a.prune = 0;
+    const uint32_t words = b->rec_words[s.tape];
+    if (b->rec && words) {   // a chain's records (JitChain): counts stay the whole tape's
+        a.prune = 2;
+        uint32_t *at = b->rec + size_t(&s - b->sessions.data()) * b->rec_stride;
+        for (auto &l : a.prune_rec)
+            for (auto &x : l) {
+                x = at;
+                at += size_t(words) * b->rec_cap;
+            }
+        a.prune_cap = std::min(b->rec_cap, s.list_cap / 8u * 8u);
+        a.choice = b->choice;
+        a.choice_len = b->choice_len;
+        if (b->rec_spec) a.spec_rec = at;
+    }
     if (b->spec_max && s.p.localsubdiv >= 2) {
         a.spec_levels = std::min<uint32_t>(b->spec_max, uint32_t(s.p.localsubdiv - 1));
         a.spec_cap = b->spec_cap;
@@ -281,7 +327,8 @@ int reset_session(tsi_batch *b, Session &s) {
 // Lowers the tapes and compiles (or finds in the code-object cache) the batch module.
 int compile_batch(const tsi_gpu_instruction *const *tapes, const uint32_t *lens, uint32_t ntapes,
                   std::vector<std::vector<tsi_gpu_instruction>> &copies, std::vector<Lowered> &low,
-                  uint32_t &stack_rows, std::vector<char> &code, tsi_batch_info &info) {
+                  uint32_t &stack_rows, std::vector<uint32_t> &rec_words, std::vector<uint32_t> &col_words,
+                  std::vector<char> &code, tsi_batch_info &info) {
     std::vector<std::vector<FwdIns>> fwd(ntapes);
     std::vector<std::vector<RevIns>> rev(ntapes);
     low.assign(ntapes, Lowered{});
@@ -297,6 +344,9 @@ int compile_batch(const tsi_gpu_instruction *const *tapes, const uint32_t *lens,
             fwd[i].resize(low[i].nfwd);
             rev[i].resize(low[i].nrev);
             stack_rows = std::max(stack_rows, low[i].stack + 1u);
+            const JitChain chain = jit_chain(copies[i].data(), lens[i], fwd[i], rev[i], low[i]);
+            rec_words.push_back(chain.ok() ? chain.record_words : 0u);
+            col_words.push_back(chain.ok() ? chain.col_words : 0u);
         }
         std::vector<BatchTape> bt;
         for (uint32_t i = 0; i < ntapes; ++i)
@@ -331,7 +381,8 @@ int tsi_batch_precompile(const tsi_gpu_instruction *const *tapes, const uint32_t
     uint32_t rows = 0;
     std::vector<char> code;
     tsi_batch_info info{};
-    const int rc = compile_batch(tapes, lens, ntapes, copies, low, rows, code, info);
+    std::vector<uint32_t> rec_words, col_words;
+    const int rc = compile_batch(tapes, lens, ntapes, copies, low, rows, rec_words, col_words, code, info);
     if (out) *out = info;
     return rc;
 }
@@ -358,7 +409,8 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
     do {
         // ---- tapes: lowering, then the module of all of them ----
         std::vector<char> code;
-        if ((rc = compile_batch(tapes, lens, ntapes, b->tapes, b->low, b->stack_rows, code, b->info))) break;
+        if ((rc = compile_batch(tapes, lens, ntapes, b->tapes, b->low, b->stack_rows, b->rec_words, b->col_words, code,
+                                b->info))) break;
         if (hipModuleLoadData(&b->mod, code.data()) != hipSuccess ||
             hipModuleGetFunction(&b->fn, b->mod, "tsi_batch_run") != hipSuccess) {
             rc = TSI_E_HIP;
@@ -395,6 +447,7 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
             (rc = hmalloc(&b->out_h, C.max_sessions)) || (rc = hmalloc(&b->error_h, 1)) || (rc = hmalloc(&b->jobs_h, C.max_sessions)) ||
             (rc = hmalloc(&b->visits_h, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)))
             break;
+        alloc_records(b);
         uint64_t arena = C.arena_bytes;
         if (arena == 0) {
             size_t fr = 0, tot = 0;

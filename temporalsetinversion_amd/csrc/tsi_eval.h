@@ -301,7 +301,7 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             }
             if (sp) {
                 // the record of the speculative pass, and the parent's tag for this frame
-                if (Engine::kSkip && E.choices_recorded()) {
+                if (Engine::kSkip && E.choices_recorded() && a.spec_rec) {
                     const uint32_t cell = (g * 8u + ps) * 8u + o;
                     E.liveness(a, ok ? a.spec_rec + cell : nullptr, a.spec_cap * 8u);
                 }
@@ -416,7 +416,7 @@ TSI_DI void eval_group(const KA &a, int level, float time, uint32_t g, uint32_t 
             if (at_r < a.prune_cap) rec = prec_r + at_r;
             // (a group the speculative pass evaluated as a whole ran no forward pass: its records)
             const bool ran = E.choices_recorded();
-            const bool valid = kids_ok && (ran || (Engine::kSkip && have));
+            const bool valid = kids_ok && (ran || (Engine::kSkip && have && a.spec_rec));
             if (rec) {
                 const Iv win = ran ? rwin : targ;
                 rec[0] = valid ? __float_as_uint(win.lo) : 0x7f800000u;

@@ -573,6 +573,34 @@ JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vecto
         return C;
     }
     C.seg = seg;
+    // ---- bounds of the sensitivities: fixed derivatives are at most 1e6, a smooth minimum's own
+    //      growth was bounded above.  All finite, an interval times [1, 1] is itself, times [-1, -1]
+    //      its negation, and the products are left out ----
+    {
+        std::vector<double> B(n, 0.0);
+        B[n - 1] = 1.0;
+        double most = 0.0;
+        for (uint32_t j = n; j-- > 4;) {
+            if (j != n - 1 && seg[j] < 0) break;   // (the globals: their rules take any product)
+            const uint32_t f = form(j);
+            double d = 1e6;
+            if (f == F_ADD_RR || f == F_SUB_RR || f == F_ADD_RL || f == F_SUB_RL || f == F_SUB_LR || f == F_NEG || f == F_RET ||
+                is_code_form(f))
+                d = 1.0;
+            else if (f == F_MUL_RL)
+                d = std::min(1e6, double(std::fabs(tape[j].literal)));
+            if (side(j) == 0 || side(j) == 1) B[left(j)] += B[j] * d;
+            if (side(j) == 0 || side(j) == 2) B[right(j)] += B[j] * d;
+            // (a smooth minimum's square has a derivative of 2 h <= 2 k, not 1e6)
+            const int sg = seg[j];
+            if (f == F_SQR && sg > 0 && C.segs[size_t(sg)].lit >= 0 && left(j) == uint32_t(C.segs[size_t(sg)].lit))
+                B[left(j)] = B[j] * 2.0 * std::fabs(double(tape[left(uint32_t(C.segs[size_t(sg)].lit))].literal));
+            most = std::max(most, B[j]);
+        }
+        for (uint32_t k = 0; k < n; ++k)
+            if (k < 4 || seg[k] < 0) most = std::max(most, B[k]);
+        C.finite = most < 0x1p126;   // (not for a NaN)
+    }
     C.words = uint32_t(C.segs.size() + 31) / 32;
     C.col_words = 2u * uint32_t(C.x_records.size()) + C.words + 1u;
     C.record_words = 2u + C.col_words;
@@ -835,6 +863,14 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                                 : "fwd_form_t<true>(" + std::to_string(form) + "u, " + l + ", " + r + ", " + lt + ")";
         return std::make_pair(f ? e : "fixk(" + e + ", K)", f);
     };
+    // The zero tests of a body's sensitivities and the ops counted with each: a sensitivity passed on
+    // as it is (or negated) is zero where its source is, and the counts of such records add up.
+    std::map<uint32_t, std::string> zof;        // record -> its sensitivity's zero test
+    std::map<std::string, uint64_t> zcost;
+    auto flush_zcost = [&]() {
+        for (const auto &x : zcost) o += "        ops += " + x.first + " ? 0u : " + std::to_string(x.second) + "u;\n";
+        zcost.clear();
+    };
     // one reverse rule: record j, sensitivity s (name), operand names a / b, the derivatives from the
     // operands' values; add(k, product, zero test or empty) receives the contributions
     auto chain_rule = [&](int c, uint32_t j, const std::string &s, const std::string &a, const std::string &b, bool f_,
@@ -844,46 +880,74 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         const RevIns &rv = rev[(n - 1) - j];
         const std::string J = "_" + std::to_string(j);
         const std::string lt = c >= 0 ? chain_lit(uint32_t(c), j) : lit(g.literal);
-        std::string rule = "rev_form_t<true>(" + std::to_string(form) + "u, " + (side == 0 || side == 1 ? a : b) + ", " +
-                           (side == 0 ? b : "ZI") + ", " + lt + ")";
-        if (form == F_SQRT && side == 1 && f_) rule = "Iv2{sqrt_rr_of_value(v" + std::to_string(j) + "), ZI}";
-        const bool code = is_code_form(form);
-        if (code) {
-            const std::string kc = "kc" + J;
-            const bool rl = form == F_MIN_RL || form == F_MAX_RL;
-            o += "        const uint32_t " + kc + " = " + code_expr(j, a, rl ? "I_FROM(" + lt + ")" : b) + ";\n";
+        const bool code = is_code_form(form), rl = form == F_MIN_RL || form == F_MAX_RL;
+        const bool fin = CH.finite && (c >= 0 || j == n - 1);
+        const std::string kc = "kc" + J;
+        if (code) o += "        const uint32_t " + kc + " = " + code_expr(j, a, rl ? "I_FROM(" + lt + ")" : b) + ";\n";
+        // the contributions: finite sensitivities are passed on by the forms of derivative 1, -1 or 0
+        std::string ca, cb;
+        bool same = false;   // the first operand's is zero exactly where s is
+        if (fin && (form == F_ADD_RR || form == F_SUB_RR || form == F_ADD_RL || form == F_SUB_RL || form == F_RET)) {
+            ca = s;
+            cb = form == F_SUB_RR ? "NEG_I(" + s + ")" : s;
+            same = true;
+        } else if (fin && (form == F_SUB_LR || form == F_NEG)) {
+            ca = "NEG_I(" + s + ")";
+            same = true;
+        } else if (fin && form == F_ABS) {
+            o += "        const Iv w" + J + " = I(wmin(" + s + ".lo, -" + s + ".hi), wmax(-" + s + ".lo, " + s + ".hi));\n";
+            ca = "sel(" + kc + " == 3u, w" + J + ", sel(" + kc + " == 2u, NEG_I(" + s + "), " + s + "))";
+            same = true;
+        } else if (fin && code) {
+            ca = "sel((" + kc + " & 1u) != 0u, " + s + ", ZI)";
+            cb = "sel((" + kc + " & 2u) != 0u, " + s + ", ZI)";
+        } else {
+            std::string rule = "rev_form_t<true>(" + std::to_string(form) + "u, " + (side == 0 || side == 1 ? a : b) + ", " +
+                               (side == 0 ? b : "ZI") + ", " + lt + ")";
+            if (form == F_SQRT && side == 1 && f_) rule = "Iv2{sqrt_rr_of_value(v" + std::to_string(j) + "), ZI}";
             if (form == F_ABS)
                 rule = "Iv2{sel(" + kc + " == 3u, I(-1.0f, 1.0f), sel(" + kc + " == 2u, I_FROM(-1.0f), ONE)), ZI}";
             else if (rl)
                 rule = "Iv2{sel((" + kc + " & 1u) != 0u, ONE, ZI), ZI}";
-            else
+            else if (code)
                 rule = "Iv2{sel((" + kc + " & 1u) != 0u, ONE, ZI), sel((" + kc + " & 2u) != 0u, ONE, ZI)}";
+            o += "        const Iv2 d" + J + " = " + rule + ";\n";
+            // fix of the derivative: as in the straight-line pass (emit_reverse)
+            auto d = [&](const char *x) {
+                const std::string e = "d" + J + "." + x;
+                const uint32_t other = x[0] == 'a' ? rarg_of(g) : larg_of(g);
+                if (code || (form == F_MUL_RR && other >= 4u)) return e;
+                if (domain && (form == F_MUL_RR || (form == F_SQR && f_))) return e;
+                return "fixk(" + e + ", K)";
+            };
+            ca = "MUL_II(" + d("a") + ", " + s + ")";
+            cb = "MUL_II(" + d("b") + ", " + s + ")";
         }
-        o += "        const Iv2 d" + J + " = " + rule + ";\n";
-        // fix of the derivative: as in the straight-line pass (emit_reverse)
-        auto d = [&](const char *x) {
-            const std::string e = "d" + J + "." + x;
-            const uint32_t other = x[0] == 'a' ? rarg_of(g) : larg_of(g);
-            if (code || (form == F_MUL_RR && other >= 4u)) return e;
-            if (domain && (form == F_MUL_RR || (form == F_SQR && f_))) return e;
-            return "fixk(" + e + ", K)";
-        };
         const bool u1 = single_use(rv, side);
-        const std::string z = "z" + J;
+        std::string z = "false";
+        if (j != n - 1) {
+            const auto known = zof.find(j);
+            z = known != zof.end() && zero_product(form) ? known->second : "z" + J;
+            if (z == "z" + J) o += "        const bool " + z + " = (" + s + ".lo == 0.0f && " + s + ".hi == 0.0f);\n";
+        }
         if (u1) {
-            o += "        const bool " + z + " = " + (j == n - 1 ? std::string("false") : "(" + s + ".lo == 0.0f && " + s + ".hi == 0.0f)") +
-                 ";\n        ops += " + z + " ? 0u : " + std::to_string(unsigned(rv.cost)) + "u;\n";
+            if (j == n - 1) o += "        ops += " + std::to_string(unsigned(rv.cost)) + "u;\n";
+            else zcost[z] += rv.cost;
+            if (same && j != n - 1) {
+                if (side == 0 || side == 1) zof[larg_of(g)] = z;
+                if ((side == 0 && form != F_ABS) || side == 2) zof[rarg_of(g)] = z;
+            }
         } else if (c < 0) {   // (a segment's: counted for all segments at once)
             static_ops += rv.cost;
         }
         const std::string zt = u1 && !zero_product(form) ? z : std::string();
         // both products before either is added (an operand may be both)
         if (side == 0) {
-            o += "        const Iv na" + J + " = MUL_II(" + d("a") + ", " + s + "), nb" + J + " = MUL_II(" + d("b") + ", " + s + ");\n";
+            o += "        const Iv na" + J + " = " + ca + ", nb" + J + " = " + cb + ";\n";
             add(true, "na" + J, zt);
             add(false, "nb" + J, zt);
         } else {
-            add(side == 1, "MUL_II(" + d("a") + ", " + s + ")", zt);
+            add(side == 1, ca, zt);
         }
     };
     auto emit_chain = [&]() {
@@ -1063,6 +1127,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
             for (uint32_t j = R.o + 1; j-- > R.lo;) {
                 if (!base && j == R.w) {   // the segment's own operand: where some cell keeps it
                     const std::string lv = "lv" + std::to_string(j);
+                    flush_zcost();
+                    zof.clear();
                     o += "        const bool " + lv + " = __builtin_amdgcn_ballot_w64(act && !(" + S(j) + ".lo == 0.0f && " + S(j) +
                          ".hi == 0.0f)) != 0;\n        if (" + lv + ") {\n";
                     open = true;
@@ -1083,6 +1149,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                                if (isp) plive = true; else live[k] = 1;
                            });
             }
+            flush_zcost();
+            zof.clear();
             if (open) o += "        }\n";
             o += std::string("        s = ") + (base ? "ZI" : "sp") + ";\n            break; }\n";
         }
@@ -1103,6 +1171,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                            o += "        " + S(k) + " = " + v + ";\n";
                        });
         }
+        flush_zcost();
+        zof.clear();
         o += "    }\n    ops += " + std::to_string(static_ops) + "u;\n    return RevOut{s0, s1, s2, s3, ops};\n}\n\n";
     };
 
@@ -1654,7 +1724,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
     if (ch) {
         // ---- the chain's engine: the parents' decisions in, this wavefront's out ----
         const std::string W = std::to_string(CH.words), X2 = std::to_string(2 * CH.x_records.size());
-        const std::string CW = std::to_string(CH.col_words), RWs = std::to_string(CH.record_words);
+        const std::string RWs = std::to_string(CH.record_words);
         uint64_t full_cost = 0;
         for (uint32_t j = 4; j < n; ++j) full_cost += fwd[j - 4].cost;
         o += "struct TapeEngine {\n    static constexpr bool kPrune = true, kSkip = true, kExactT = " + std::string(CH.exact_t ? "true" : "false") +
@@ -1663,7 +1733,8 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
              "    uint32_t live, rows, nrec;\n    bool act, ran;\n"
              "    template <class KA>\n    TSI_DI TapeEngine(const KA &a, uint32_t wave, uint32_t l)\n"
              "        : lane(l), lrec(nullptr), cols(nullptr), mask{0u, 0u}, live(0u), rows(0u), nrec(kTapeRecords), act(true), ran(false) {\n"
-             "        colbase = a.choice ? a.choice + size_t(wave) * " + CW + "u * 64u + l : nullptr;\n    }\n"
+             "        // (choice_len: of the tapes of a batch, the most)\n"
+             "        colbase = a.choice ? a.choice + size_t(wave) * a.choice_len * 64u + l : nullptr;\n    }\n"
              "    template <class KA>\n    TSI_DI void select(const KA &a, int, uint32_t, bool pruned_ok, const uint32_t *prec_in, uint32_t pidx,\n"
              "                       bool need_choices, bool act_) {\n"
              "        lrec = nullptr;\n        act = act_;\n        ran = false;\n        cols = need_choices ? colbase : nullptr;\n"
@@ -1834,8 +1905,9 @@ std::string jit_source_batch(const std::vector<BatchTape> &tapes, const JitDomai
         // (with 64: 611 against 643 frames/s batched, served p50 2.01 against 1.80 ms)
         const bool skip = batch_skip();
         const uint32_t group = batch_region_records();
-        const std::string f = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, false, false, domain, skip, group);
-        const std::string r = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, true, false, domain, skip, group);
+        const JitChain chain = jit_chain(t.tape, t.n, *t.fwd, *t.rev, *t.low);
+        const std::string f = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, false, false, domain, skip, group, &chain);
+        const std::string r = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, true, false, domain, skip, group, &chain);
         o += "namespace tb" + std::to_string(i) + " {\nnamespace jf {   // forward-only list\n" + module_body(f);
         o += "}  // namespace jf\nnamespace jr {   // reverse list\n" + module_body(r);
         o += "}  // namespace jr\n}  // namespace tb" + std::to_string(i) + "\n";
@@ -1844,20 +1916,20 @@ std::string jit_source_batch(const std::vector<BatchTape> &tapes, const JitDomai
     o += "struct BatchTapes {\n"
          "    template <bool REV, class E, class KA>\n"
          "    static TSI_DI void run(const KA &a, int level, float time, uint32_t g, uint32_t count, float2 *stk,\n"
-         "                           LevelTally &tl) {\n"
-         "        E eng(a, 0u, lane_id());\n"
+         "                           uint32_t wave, LevelTally &tl) {\n"
+         "        E eng(a, wave, lane_id());\n"
          "        Slots Rlo, Rhi;\n"
          "        eval_group<REV, E>(a, level, time, g, count, stk, eng, Rlo, Rhi, tl, REV && level < 0);\n"
          "    }\n"
          "    template <bool REV, class KA>\n"
          "    static TSI_DI void group(uint32_t tape, const KA &a, int level, float time, uint32_t g, uint32_t count,\n"
-         "                             float2 *stk, LevelTally &tl) {\n"
+         "                             float2 *stk, uint32_t wave, LevelTally &tl) {\n"
          "        switch (tape) {\n";
     for (size_t i = 0; i < tapes.size(); ++i) {
         const std::string ns = "tb" + std::to_string(i);
         o += "        case " + std::to_string(i) + "u:\n"
-             "            if constexpr (REV) run<true, " + ns + "::jr::TapeEngine>(a, level, time, g, count, stk, tl);\n"
-             "            else run<false, " + ns + "::jf::TapeEngine>(a, level, time, g, count, stk, tl);\n"
+             "            if constexpr (REV) run<true, " + ns + "::jr::TapeEngine>(a, level, time, g, count, stk, wave, tl);\n"
+             "            else run<false, " + ns + "::jf::TapeEngine>(a, level, time, g, count, stk, wave, tl);\n"
              "            break;\n";
     }
     o += "        default: break;\n        }\n    }\n};\n}  // namespace tsi\n\n";

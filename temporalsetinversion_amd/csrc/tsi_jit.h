@@ -53,6 +53,7 @@ struct JitChain {
     std::vector<uint32_t> x_records;  // sin / cos / exp / log of the cell's position: not monotone to the ulp,
                                       // so a cell checks that its values lie inside its parent's
     bool exact_t = false;             // some depend on t alone: the t-windows must be equal
+    bool finite = false;              // no sensitivity can overflow (see jit_chain)
     uint32_t rows = 0;                // saved-operand rows of globals; a visited segment takes one more
     uint32_t lit_words = 0;           // words of a segment's table entry
     uint32_t words = 0, record_words = 0, col_words = 0;

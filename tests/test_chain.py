@@ -148,3 +148,31 @@ def test_chains_match_the_full_tape(case):
                 assert gs["fwd_ops"] == rs["fwd_ops"] and gs["pruned_instr"] == 0
             elif k == 0:    # new cells' parents have decided most segments
                 assert gs["fwd_ops"] < rs["fwd_ops"] and gs["pruned_instr"] > 0
+
+
+@pytest.mark.gpu
+def test_batched_chains_match_the_plain_path():
+    """Chains of several record lengths, and tapes that are none, in one batch: sessions of different
+    tapes run side by side (each wavefront's columns have the room of the longest record)."""
+    from temporalsetinversion_amd.batch import Batch
+    tapes = [union(20, ["min"]), union(120, ["smin", "min"], "linear", 3), union(65, ["smin", "rmin"], "sine", 4),
+             union(40, ["min", "max"], "warp", 6), union(6, ["min"], "static", 9)]
+    sessions = [(0, 6, {}), (1, 6, dict(lipschitz_corrected=True)), (2, 6, {}), (3, 6, {}), (4, 5, {}),
+                (1, 5, dict(swept_volume=True, swept_window=0.2)), (2, 6, dict(swept_volume=True, swept_window=0.1)),
+                (3, 5, dict(point_sample=False)), (1, 7, {})]
+    times = [0.0, 1 / 60, 2 / 60, 0.2, 0.15]
+    with Batch(tapes, arena_bytes=sum(100 << 18 for _ in sessions) + (256 << 20), max_sessions=len(sessions)) as b:
+        sids = [b.open(tape=t, localsubdiv=L, voxel_capacity=1 << 18, max_width=16, max_height=16, **kw)
+                for t, L, kw in sessions]
+        got = []
+        for k, t in enumerate(times):
+            res, _, _ = b.run([(sid, float(np.float32(t + 0.01 * i)), 0, 0, None) for i, sid in enumerate(sids)])
+            got.append([(r, b.read_nodes(sid)) for r, sid in zip(res, sids)])
+    for i, (t, L, kw) in enumerate(sessions):
+        want = frames(tapes[t], [x + 0.01 * i for x in times], localsubdiv=L, engine="interpreter", prune=False, **kw)
+        for k, (rs, r) in enumerate(want):
+            gs, g = got[k][i]
+            assert gs["status"] == 0
+            assert_same_nodes(g, r, f"session {i} frame {k}")
+            for key in ("cell_evals", "rev_evals", "fwd_ops", "rev_ops", "parents", "enqueued", "deallocs", "allocated_nodes"):
+                assert gs[key] == rs[key], f"session {i} frame {k}: {key}"
