@@ -126,15 +126,13 @@ struct LaneG {
             hi = load(a.bhi, node);
         }
         TSI_DI void put_box(uint32_t, V, V) const {}
-        TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask, uint32_t oct) const {
-            base[s * kTraceThreads] = make_uint2(meta, mask | (oct << 8));
-        }
+        TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask) const { base[s * kTraceThreads] = make_uint2(meta, mask); }
         TSI_DI void get(const KArgs &a, uint32_t s, uint32_t &meta, uint32_t &mask, V &lo, V &hi) const {
             const uint2 e = base[s * kTraceThreads];
             const uint32_t up = base[(s == 0u ? 0u : s - 1u) * kTraceThreads].x;
             const uint32_t node = s == 0u ? 0u : (up - 1u) * 8u + (e.y >> 8);
             meta = e.x;
-            mask = e.y & 0xFFu;
+            mask = e.y;
             lo = load(a.blo, node);
             hi = load(a.bhi, node);
         }
@@ -235,7 +233,7 @@ struct QuadG {
             if (!fourth()) base[s * kTraceThreads] = make_uint2(__float_as_uint(lo), __float_as_uint(hi));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask, uint32_t) const {
+        TSI_DI void put_node(uint32_t s, uint32_t meta, uint32_t mask) const {
             if (fourth()) base[s * kTraceThreads] = make_uint2(meta, mask);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
@@ -435,6 +433,9 @@ TSI_DI void walk_exact(const KArgs &a, typename G::Stack stk, typename G::V ro, 
     dist = intersected ? fabsf(glength<G>(o2 - ro)) : -1.0f;
 }
 
+// Keeps a number a number, in a vector register (no instruction).
+TSI_DI void in_vgpr(uint32_t &x) { asm volatile("" : "+v"(x)); }
+
 // The same traversal, the same values bit for bit, for rays of moderate numbers; returns false where
 // it cannot tell (walk_exact then takes the ray from its start).  What differs:
 //   * divisions without their scaling steps (recip_mid, div_mid) while a node's box, the ray's
@@ -466,19 +467,24 @@ TSI_DI bool walk_fast(const KArgs &a, const TraceArgs &ta, typename G::Stack stk
     V q0 = p0, q1 = p1;                                 // the node's stored box
     uint32_t d = 0u;                                    // the node's depth: its entry on the stack
     uint32_t node = 0u;                                 // (of a node just entered)
+    // (the stack's mask word: the surface mask, and above it the node's octant in its parent)
     uint32_t meta = meta_of(a.st[0]) & kChildMask, mask = ta.mask[0];
-    bool entered = false;        // the node was entered by the last iteration: it may be a leaf
-    bool own = true;             // p0/p1 are the node's (else the box of a node below, see walk_exact)
+    // The walk's conditions are numbers in vector registers (in_vgpr): as conditions, each kept over
+    // the divergent branches below takes three scalar instructions per change to merge, and a
+    // wavefront issued nearly as many scalar instructions as vector ones (capsules at 512x512: 434
+    // -> 348 us, at 1280x720 609 -> 465; path-traced csg at 960x540 9.7 -> 8.2 ms).
+    uint32_t entered = 0u;       // the node was entered by the last iteration: it may be a leaf
+    uint32_t own = 1u;           // p0/p1 are the node's (else the box of a node below, see walk_exact)
+    uint32_t end = 0u;           // why the walk ended: it left (0), at a leaf (1), it cannot tell (2)
     float t_node = 0.0f;
     stk.put_box(0u, q0, q1);
-    stk.put_node(0u, meta, mask, 0u);
+    stk.put_node(0u, meta, mask);
     Slab hit = slabs<G>(p0, p1, o2, inv);
-    bool on = hit.hit, ok = true;
-    bool intersected = false;
-    for (uint32_t iter = 0; on && iter < 5000u; ++iter) {
-        bool up = true;          // back to the parent
-        bool box_up = true;      // ... and to its box
-        if (hit.hit) {
+    uint32_t inside = hit.hit ? 1u : 0u;   // the walked box is hit
+    if (inside != 0u) {
+    for (uint32_t iter = 0; iter < 5000u; ++iter) {
+        uint32_t way = 2u;       // 0: into a child, 1: back to the parent, 2: ... and to its box
+        if (inside != 0u) {
             const V e = p1 - p0;
             const V eh = e * 0.5f;
             const V e2 = G::map(eh, recip_mid);       // 2 / e
@@ -491,50 +497,42 @@ TSI_DI bool walk_fast(const KArgs &a, const TraceArgs &ta, typename G::Stack stk
             const float dark = !CIN && !normal_viz && G::maxc(e) < 1.0f ? kDarken : 1.0f;   // 4265
             const float leave = hit.far_ - kTrEps;
             const V h = (q1 - q0) * 0.5f;
-            ok = G::mid(eh, r, rdl) && G::minc(eh) > 0.0f;
-            if (entered) {
-                if (meta == 0u) {   // a leaf: the hit
-                    intersected = true;
-                    ok = true;
-                } else {
-                    stk.put_node(d, meta, mask, node & 7u);
-                }
-                entered = false;
-            }
-            if (intersected || !ok) break;
+            const bool ok = G::mid(eh, r, rdl) && G::minc(eh) > 0.0f;
+            end = (entered != 0u && meta == 0u) ? 1u : (ok ? 0u : 2u);   // a leaf: the hit
+            if (end != 0u) break;
+            stk.put_node(d, meta, mask);
+            entered = 0u;
             const V old = o2;
             // children that stop the march: those with a surface, and any number outside the grid
             const uint32_t stop = mask | 0xFFFFFF00u;
             float len = 0.0f, t;
-            uint32_t k = 0, steps = 0;
-            bool out, enter = false, tie = false;
+            uint32_t steps = 0, tie = 0;
+            way = 1u;
             for (;;) {
                 for (;;) {
                     c = c * dark;
                     t = (len + hit.near_) + kTrEps;
-                    out = t >= leave;
-                    if (out || ((stop >> min(ci, 31u)) & 1u) || steps == 32u) break;
-                    ++k;
+                    const bool halt = t >= leave || ((stop >> min(ci, 31u)) & 1u) != 0u || steps == 32u;
+                    if (halt) break;
                     ++steps;
                     int32_t inc;
-                    tie = tie || G::advance(sd, dd, st, len, inc);
+                    tie = G::advance(sd, dd, st, len, inc) ? 1u : tie;
                     ci = ci + uint32_t(inc);
                 }
                 o2 = old + t * rd;
-                if (out || ci >= 8u || tie || steps == 32u) break;
-                ++k;
+                if (t >= leave || ci >= 8u || (tie | (steps >> 5)) != 0u) break;
                 ++steps;
                 // the child's box as eval_level stored it (tsi_eval.h), from its parent's
                 const V oc = G::octant(ci);
                 V lo = G::fma(h, oc, q0), hi = G::fma(h, 1.0f + oc, q0);
-                if (!own) {
+                if (own == 0u) {
                     lo = G::load(a.blo, (meta - 1u) * 8u + ci);
                     hi = G::load(a.bhi, (meta - 1u) * 8u + ci);
                 }
                 const V w0 = lo - kTrEps, w1 = hi + kTrEps;
                 const Slab th = slabs<G>(w0, w1, o2, inv);
                 if (th.hit) {
-                    enter = true;
+                    way = 0u;
                     hit = th;
                     p0 = w0;
                     p1 = w1;
@@ -543,53 +541,53 @@ TSI_DI bool walk_fast(const KArgs &a, const TraceArgs &ta, typename G::Stack stk
                     break;
                 }
                 int32_t inc;
-                tie = tie || G::advance(sd, dd, st, len, inc);
+                tie = G::advance(sd, dd, st, len, inc) ? 1u : tie;
                 ci = ci + uint32_t(inc);
             }
-            visits += meta != 0u ? k : 0u;
-            if (tie || steps == 32u) {
-                ok = false;
-                break;
-            }
-            if (enter) {
-                up = false;
+            in_vgpr(way);
+            in_vgpr(tie);
+            visits += meta != 0u ? steps : 0u;
+            end = (tie | (steps >> 5)) != 0u ? 2u : 0u;
+            if (way == 0u) {
                 node = (meta - 1u) * 8u + ci;
                 meta = meta_of(a.st[node]) & kChildMask;
                 t_node = a.st[node].y;
-                mask = ta.mask[size_t(node) * ta.mask_stride];
-                own = true;
-                entered = true;
+                mask = ta.mask[size_t(node) * ta.mask_stride] | (ci << 8);
+                own = 1u;
+                entered = 1u;
                 ++d;
-                if (d == ta.stack - 1u) {   // (walk_exact knows what a full stack does)
-                    ok = false;
-                    break;
-                }
+                if (d == ta.stack - 1u) end = 2u;   // (walk_exact knows what a full stack does)
                 stk.put_box(d, q0, q1);
+            } else if (t >= leave) {
+                way = 2u;
+                o2 = old + hit.far_ * rd;
+            }
+            if (end != 0u) break;
+        }
+        in_vgpr(way);
+        if (way != 0u) {         // back to the parent
+            if (d == 0u) break;
+            --d;
+            if (way == 2u) {
+                stk.get(a, d, meta, mask, q0, q1);
+                p0 = q0;
+                p1 = q1;
+                own = 1u;
+                hit = slabs<G>(p0, p1, o2, inv);
+                inside = hit.hit ? 1u : 0u;
             } else {
-                box_up = out;
-                if (out) o2 = old + hit.far_ * rd;
+                V u, v;
+                stk.get(a, d, meta, mask, u, v);
+                own = 0u;
             }
         }
-        if (up) {
-            if (d == 0u) {
-                on = false;
-            } else {
-                --d;
-                if (box_up) {
-                    stk.get(a, d, meta, mask, q0, q1);
-                    p0 = q0;
-                    p1 = q1;
-                    own = true;
-                    hit = slabs<G>(p0, p1, o2, inv);
-                } else {
-                    V u, v;
-                    stk.get(a, d, meta, mask, u, v);
-                    own = false;
-                }
-            }
-        }
+        in_vgpr(own);
+        in_vgpr(inside);
+        in_vgpr(entered);
     }
-    if (entered && meta == 0u) intersected = true;   // (the iterations ended on a leaf)
+    }
+    const bool ok = end != 2u;
+    const bool intersected = end == 1u || (end == 0u && entered != 0u && meta == 0u);   // (or the iterations ended on a leaf)
     if (!ok) return false;
     col = G::pick(c, c, c);
     if (intersected) col = hit_colour<G, CIN>(c, ta.time, t_node, node, ta.shading, ta.grad, nrm);
@@ -940,11 +938,11 @@ int launch_trace_end(unsigned long long *visits, uint32_t n_clear, unsigned long
 
 // Frames of at most this many pixels are traced with four lanes per ray: their wavefronts then
 // still find free SIMDs, and the frame takes the latency of its longest chains, which are shorter so
-// (64x48: 36 against 43 us; spheres at 256x256: 113 against 137).  Larger frames are bound by
-// instructions (capsules at 300x300: 366 against 364 us, at 448x448 573 against 389).  A path-traced
-// pixel is 8 samples of up to 4 rays, chains so long that the line lies higher (csg at 320x200: 6.4
-// against 8.0 ms, at 641x361 8.5 against 8.2, spheres 2.5 against 2.8; at 960x540 12.6 against 9.3).
-constexpr uint64_t kQuadPixels = 98304, kQuadPixelsCinematic = 262144;
+// (64x48 spheres: 88 against 108 us; csg at 362x362: 296 against 307).  Larger frames are bound by
+// instructions (448x448: capsules 382 against 327 us, csg 332 against 290, spheres 116 against 122).
+// A path-traced pixel is 8 samples of up to 4 rays, chains so long that the line lies higher (csg at
+// 641x361: 6.7 against 7.2 ms, capsules 7.1 against 8.2; at 960x540 9.2 against 8.0 and 9.1 against 8.8).
+constexpr uint64_t kQuadPixels = 147456, kQuadPixelsCinematic = 393216;
 
 // LDS of a wavefront's ray stacks: entries x 64 lanes x 8 B.
 static uint32_t stack_bytes(uint32_t entries) { return entries * kTraceThreads * uint32_t(sizeof(uint2)); }
