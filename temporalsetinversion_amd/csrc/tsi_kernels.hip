@@ -5,7 +5,7 @@
 // global memory (compute.wgsl:3513-4056).  Here one frame is a fixed sequence of launches
 // over a level-synchronous frontier:
 //   k_frame_begin            seed the root (buf_main / first-frame seeding)
-//   k_eval<REV> x levels     one 64-lane wavefront = 8 parents x 8 child octants; the tape
+//   k_eval x levels          one 64-lane wavefront = 8 parents x 8 child octants; the tape
 //                            is interpreted wave-uniformly (instructions via scalar loads,
 //                            live values in a uniformly indexed VGPR file), then the cell is
 //                            classified; subdivision / dealloc outputs are compacted with
@@ -28,10 +28,13 @@ namespace tsi {
 
 // ---------------------------------------------------------------- frame kernels
 
-// One level of one frontier list with the interpreter (eval_level, tsi_eval.h).
-template <bool REV>
+// One level with the interpreter (eval_level, tsi_eval.h), both lists side by side as in the compiled
+// level kernel (a launch per list: 10 us more a level, of 110).
 __global__ void __launch_bounds__(256) k_eval(KArgs a, int level, float time) {
-    eval_level<REV, InterpEngine>(a, level, time);
+    const uint32_t nb = gridDim.x, b = blockIdx.x, w = threadIdx.x >> 6, bwave = b * 4u + w;
+    const uint32_t nf = __builtin_amdgcn_readfirstlane(level_split(a, level, nb));
+    if (b < nf) eval_level<false, InterpEngine>(a, level, time, bwave, nf * 4u, bwave);
+    else eval_level<true, InterpEngine>(a, level, time, (b - nf) * 4u + w, (nb - nf) * 4u, bwave);
 }
 
 __global__ void k_frame_begin(KArgs a) { frame_begin(a, threadIdx.x, blockDim.x); }
@@ -39,7 +42,8 @@ __global__ void k_frame_begin(KArgs a) { frame_begin(a, threadIdx.x, blockDim.x)
 // The speculative pass's node list (spec_gather, tsi_eval.h): one block.
 __global__ void __launch_bounds__(1024) k_spec_gather(KArgs a) { spec_gather(a, threadIdx.x, blockDim.x); }
 // every parent decided.  Groups with an entry lacking a record run the full program.
-__global__ void __launch_bounds__(256) k_prune(KArgs a, int level, int which) {
+__global__ void __launch_bounds__(256) k_prune(KArgs a, int level) {
+    const int which = int(blockIdx.y);
     Counters *cnt = a.cnt;
     const uint32_t count = min(cnt->level[level].list[which], a.list_cap);
     if (count == 0) return;
@@ -241,23 +245,20 @@ int launch_frame(const KArgs &a, const FrameLaunch &fl, hipStream_t s, hipEvent_
         const bool compiled = fl.tape_eval != nullptr;
         if (e_level) hipEventRecord(e_level[2 * d], s);
         if (a.prune && d > 0 && !compiled) {   // the interpreter's group programs
-            hipLaunchKernelGGL(k_prune, dim3(fl.grid_misc), dim3(256), 0, s, a, d, 0);
-            hipLaunchKernelGGL(k_prune, dim3(fl.grid_misc), dim3(256), 0, s, a, d, 1);
+            hipLaunchKernelGGL(k_prune, dim3(fl.grid_misc, 2), dim3(256), 0, s, a, d);
         }
+        // both lists of the level in one launch, which splits the grid: each list gets at least one block
+        const uint32_t nb = std::min(fl.grid_fwd + fl.grid_rev, 2u * level_blocks(d, fl.grid_rev));
         if (compiled) {
             KArgs ka = a;
             int level = d;
             float t = fl.time;
             void *args[] = {&ka, &level, &t};
-            // both lists of the level in one launch (tsi_tape_eval_level splits the grid: each
-            // list gets at least one block)
-            const uint32_t nb = std::min(fl.grid_fwd + fl.grid_rev, 2u * level_blocks(d, fl.grid_rev));
             if (hipModuleLaunchKernel((hipFunction_t)fl.tape_eval, nb, 1, 1, 256, 1, 1, 0, s, args, nullptr) !=
                 hipSuccess)
                 return -1;
         } else {
-            hipLaunchKernelGGL(k_eval<false>, dim3(level_blocks(d, fl.grid_fwd)), dim3(256), 0, s, a, d, fl.time);
-            hipLaunchKernelGGL(k_eval<true>, dim3(level_blocks(d, fl.grid_rev)), dim3(256), 0, s, a, d, fl.time);
+            hipLaunchKernelGGL(k_eval, dim3(nb), dim3(256), 0, s, a, d, fl.time);
         }
         if (e_level) hipEventRecord(e_level[2 * d + 1], s);
         if (sp && d == (sp->ready_level < fl.levels - 1 ? sp->ready_level : fl.levels - 1))

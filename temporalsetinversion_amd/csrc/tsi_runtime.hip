@@ -877,10 +877,9 @@ int tsi_set_inversion_result(tsi_ctx *c, double *gpu_ms, tsi_stats *stats) {
         stats->deallocs = h.stats[kStatDeallocs];
         stats->enqueued = h.stats[kStatEnqueued];
         stats->allocated_nodes = h.stats[kStatLive] * 8u;
-        // the compiled engine runs both lists of a level in one launch (and the speculative pass
-        // in one more), the interpreter in two
-        stats->eval_launches = uint64_t((c->eval_fn[0] ? 1 : 2) * c->p.localsubdiv) + (spec_active(c) ? 1u : 0u);
-        stats->prune_launches = c->prune && !c->eval_fn[0] ? uint64_t(2 * (c->p.localsubdiv - 1)) : 0u;
+        // both lists of a level in one launch, the speculative pass in one more
+        stats->eval_launches = uint64_t(c->p.localsubdiv) + (spec_active(c) ? 1u : 0u);
+        stats->prune_launches = c->prune && !c->eval_fn[0] ? uint64_t(c->p.localsubdiv - 1) : 0u;
     }
     c->used_nodes = (uint64_t(h.bump) + 1u) * 8u;
     if (c->used_nodes > c->nodes) c->used_nodes = c->nodes;
