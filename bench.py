@@ -173,7 +173,7 @@ def summarize_profile(args) -> None:
             lines.append(f"  level {d:>4} {sum(v) / len(v):>9.1f} {min(v):>9.1f} {max(v):>9.1f}")
     lines.append("")
     lines.append("timed frames only (the figures bench.py reads):")
-    for name in ("tsi_tape_eval_level", "void tsi::k_trace<false>", "void tsi::k_trace_quads<false>"):
+    for name in ["tsi_tape_eval_level"] + sorted(k for k in timed if k.startswith("void tsi::k_trace")):
         if name in timed:
             n, t = timed[name]
             lines.append(f"{name} timed {n} dispatches avg_us {t / n:.2f}")
@@ -204,7 +204,7 @@ def summarize_profile(args) -> None:
         lines += ["", f"copy calibration ({args.copy_mib} MiB device-to-device): FETCH_SIZE scale {sf:.3f}, "
                       f"WRITE_SIZE scale {sw:.3f} (bytes = KiB x scale x 1024); level launches of the timed frames",
                   f"{'kernel':<24} {'':>4} {'dispatches':>10} {'fetch_KiB/disp':>15} {'write_KiB/disp':>15} {'bytes/disp':>15}"]
-        for k in ("tsi_tape_eval_level", "void tsi::k_trace<false>", "void tsi::k_trace_quads<false>", "tsi::k_snapshot"):
+        for k in ["tsi_tape_eval_level"] + sorted(k for k in f if k.startswith("void tsi::k_trace")) + ["tsi::k_snapshot"]:
             if k in f and k in w:
                 vf, vw = f[k], w[k]
                 if not vf or not vw:
@@ -952,15 +952,17 @@ def main():
         "roofline": {"bound": "valu",
                      "kernel": ("tsi_tape_eval_level (one launch per octree level: forward-only and reverse lists)"
                                 if info["engine"] == "compiled" else
-                                "k_eval<false>/<true> (one forward-only and one reverse launch per octree level)"),
+                                "k_eval (one launch per octree level: forward-only and reverse lists)"),
                      "achieved": achieved, "peak": PEAK_VALU_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_VALU_TFLOPS,
                      "frac_vs_unpacked_issue": achieved / PEAK_VALU_UNPACKED_TOPS,
                      "peak_unpacked_issue": PEAK_VALU_UNPACKED_TOPS,
                      "traffic": traffic, "traffic_unit": "HBM bytes per launch", "traffic_source": traffic_src,
+                     # (of the full tape in every cell: records whose outcome a cell's parents decided are
+                     # counted, not run)
                      "algorithmic_ops_per_launch": ops / launches,
                      "ops_per_cell_eval": ops / max(tot["cells"], 1),
-                     # HIP events right before and after each level launch, over the timed frames
+                     # the levels' time by the device's clock (tsi_stats.eval_kernel_ms), over the timed frames
                      "avg_launch_us": tot["kernel_ms"] * 1e3 / launches,
                      # the same kernel's average over the timed frames of the committed rocprofv3 summary
                      "profile_avg_kernel_us": prof_avg_us,

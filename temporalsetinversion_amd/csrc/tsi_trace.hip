@@ -23,7 +23,7 @@
 
 namespace tsi {
 
-namespace {
+namespace rays {
 
 constexpr float kTrEps = 0.0001f;     // compute.wgsl:4140
 constexpr float kDarken = 0.98f;      // compute.wgsl:3507
@@ -845,7 +845,8 @@ TSI_DI void add_visits(const TraceArgs &t, uint32_t visits) {
     if (lane_id() == 0 && v) atomicAdd((unsigned long long *)t.visits + slot * kTallyStride, (unsigned long long)v);
 }
 
-}  // namespace
+}  // namespace rays
+using namespace rays;
 
 // One wavefront per block: a block of four keeps its LDS (the ray stacks: 8 KB a wavefront) until its
 // slowest wavefront is done, and with times of 40 to 110 us a SIMD held 1.9 wavefronts on average
