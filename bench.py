@@ -8,8 +8,8 @@ re-enqueue, at t_k = k/60.  The first W frames are untimed warm-up (frame 0 eval
 cell); the next K frames are timed with the device synchronised on both sides.
 
 Prints one JSON line.  `value` = interval cell-evals per second over the timed frames;
-`roofline` reports the tape-evaluation kernel against the FP32 VALU peak (its device time from
-HIP events right around each level launch); `temporal_vs_full` compares the set inversion of
+`roofline` reports the tape-evaluation kernel against the FP32 VALU peak (its device time by the
+device's clock, from a level's first block to its last); `temporal_vs_full` compares the set inversion of
 the temporal frames with full re-evaluation (every frame from an empty octree), the quantity
 the reference publishes (~3x at 1024^3, delta 0.01); `cpu_baseline` times the oracle (the C
 restatement of the reference) on a bounded sample of the same workload.
@@ -502,7 +502,7 @@ def cinematic_form(T, args) -> dict:
         gbs = (visits * 40 + px * 20) / (ms * 1e-3) / 1e9
         out[name] = {"trace_ms_per_frame": ms, "pixels_per_s": px / (ms * 1e-3), "node_visits_per_frame": visits,
                      "node_visits_per_pixel": visits / px, "frame": f"{w['width']}x{w['height']}",
-                     "roofline": {"bound": "hbm", "kernel": "k_trace<true>", "achieved": gbs, "peak": PEAK_HBM_GBS,
+                     "roofline": {"bound": "hbm", "kernel": "k_trace<G, true>", "achieved": gbs, "peak": PEAK_HBM_GBS,
                                   "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS}, "frames": frames}
     return out
 

@@ -71,9 +71,11 @@ typedef struct {
     uint32_t flags;               /* TSI_FLAG_* */
     uint32_t prune_capacity;      /* frontier entries per list and level that get a pruned
                                      program (0 = min(queue_capacity, 2^19)) */
-    uint32_t prune_live_max;      /* compiled engine: a wavefront runs its pruned code when at
-                                     most this percentage of the tape's regions is live for it
-                                     (0 = 75; 100 = whenever its parents' records apply) */
+    uint32_t prune_live_max;      /* compiled engine, pruned by regions: a wavefront runs its
+                                     pruned code when at most this percentage of the tape's
+                                     regions is live for it (0 = 75; 100 = whenever its parents'
+                                     records apply).  Not 0: prune by regions also where the
+                                     tape is a chain (TSI_FLAG_INTERPRET below) */
     uint32_t shading;             /* TSI_SHADE_* (0: the reference's default colouring; other
                                      bits than TSI_SHADE_* give TSI_E_ARG) */
 } tsi_params;
@@ -102,11 +104,13 @@ enum {
     TSI_FLAG_NO_PRUNE = 1u,
     TSI_FLAG_PRUNE_EXACT_ONLY = 2u, /* prune only tapes of the first (exact) kind */
     /* Evaluate tapes with the interpreter (programs in constant memory) instead of compiling
-     * each uploaded tape into straight-line evaluation kernels (which prune by regions of
-     * 16 records, see prune_live_max). */
+     * each uploaded tape into evaluation kernels.  A tape that is a chain (a union of at least
+     * 16 segments under min / max / smooth-min) compiles to loops over the segments that a
+     * cell's ancestors left undecided, whatever the pruning flags say where that is exact; any
+     * other tape to straight-line code, which prunes by regions of 16 records (prune_live_max). */
     TSI_FLAG_INTERPRET = 4u,
     /* Do not evaluate the shallow levels speculatively.  By default the compiled engine, when
-     * the tape is not pruned, evaluates at each frame's start, in one launch, the children of
+     * the tape is not pruned by regions, evaluates at each frame's start, in one launch, the children of
      * every node of the first levels (depth < 7, $TSI_SPEC_LEVELS sets another count, 0 none)
      * as the octree stands (a leaf's children as new cells), where each of those levels
      * otherwise runs one wavefront's dependent chain through the tape on an idle device; a
@@ -123,7 +127,8 @@ typedef struct {
     double eval_ms;               /* of which: tape-evaluation kernels */
     uint64_t cell_evals;          /* child cells that passed the evaluation guard (compute.wgsl:3629) */
     uint64_t rev_evals;           /* of those, cells that ran the reverse pass (compute.wgsl:3780) */
-    uint64_t fwd_ops;             /* of the records actually run (pruned programs run fewer) */
+    uint64_t fwd_ops;             /* of the records run (pruned programs run fewer; with
+                                     TSI_FLAG_NO_PRUNE always the whole tape's) */
     uint64_t rev_ops;
     uint64_t parents;             /* non-dealloc work items (parents subdivided) */
     uint64_t deallocs;            /* node blocks freed by the dealloc cascade */
@@ -132,9 +137,10 @@ typedef struct {
     uint64_t eval_launches;       /* tape-evaluation kernel launches */
     uint64_t pruned_instr;        /* sum over evaluated cells of instructions skipped by pruning */
     uint64_t prune_launches;      /* group-program generator launches */
-    double eval_kernel_ms;        /* the evaluation launches alone: device time between events
-                                     recorded right before and after each level's launches
-                                     (eval_ms also holds the gaps between levels) */
+    double eval_kernel_ms;        /* the evaluation launches alone (eval_ms also holds the gaps
+                                     between levels): compiled kernels by the device's clock,
+                                     from a level's first block to its last; the interpreter's
+                                     by events around each level's launches */
     uint64_t spec_cells;          /* of cell_evals, cells whose results came from the frame's
                                      speculative pass (TSI_FLAG_NO_SPECULATE) */
 } tsi_stats;
@@ -313,7 +319,8 @@ typedef struct {
     tsi_params params;            /* localsubdiv, delta, point_sample, swept_volume, swept_window,
                                      lipschitz_corrected, fastenabled, fast_multiplier, shading,
                                      voxel_capacity (0 = 2^22 nodes), queue_capacity; flags,
-                                     prune_* are ignored: batches evaluate the full tape */
+                                     prune_* are ignored: counts and results are
+                                     those of the full tape in every cell */
     float root_box[6];            /* x.lo, y.lo, z.lo, x.hi, y.hi, z.hi (inside [-5,5]^3) */
     uint32_t max_width, max_height;   /* largest frame it traces (0, 0: 1920 x 1080) */
 } tsi_session_desc;

@@ -194,15 +194,16 @@ class State:
             p.flags = _lib.TSI_FLAG_PRUNE_EXACT_ONLY
         else:
             p.flags = 0 if prune else _lib.TSI_FLAG_NO_PRUNE
-        # engine: "compiled" = the tape compiled into straight-line kernels at upload (pruned by
-        # regions of 16 records; unpruned modules use 64-record regions), "interpreter" =
-        # programs in constant memory, pruned per frontier group and record
+        # engine: "compiled" = the tape compiled at upload: a union of at least 16 segments into
+        # loops over the segments a cell's ancestors left undecided, any other tape into
+        # straight-line kernels (pruned by regions of 16 records; unpruned modules use 64-record
+        # regions), "interpreter" = programs in constant memory, pruned per frontier group and record
         if engine not in ("compiled", "interpreter"):
             raise ValueError(f"engine must be 'compiled' or 'interpreter', not {engine!r}")
         if engine == "interpreter":
             p.flags |= _lib.TSI_FLAG_INTERPRET
-        # speculate: the compiled, unpruned engine evaluates the shallow levels of each frame in
-        # one launch at its start from the previous frame's frontier (TSI_FLAG_NO_SPECULATE)
+        # speculate: unless the tape is pruned by regions, the compiled engine evaluates the shallow
+        # levels of each frame in one launch at its start (TSI_FLAG_NO_SPECULATE)
         if not speculate:
             p.flags |= _lib.TSI_FLAG_NO_SPECULATE
         p.prune_capacity = prune_capacity
