@@ -15,9 +15,9 @@
 //                      is left: for each session, groups of 8 entries of its reverse list, of its
 //                      forward-only list (levels below its depth), and of its dealloc list
 //                      (step d of the cascade, d >= 1; steps D and D+1 are the cascade's tail)
-//   phase "end"        every session's frame_end, then frame_commit
+//   phase "end"        every session's frame_end and frame_commit
 //
-// with a grid barrier between phases.  A unit is exactly what the per-level kernels do with one
+// with a grid barrier after each phase that has units.  A unit is exactly what the per-level kernels do with one
 // group (eval_group / dealloc_step, tsi_eval.h), on the session's own pool and lists, so a
 // session's frame is the same whether it runs alone or in a batch.  Within a phase, units of
 // every session are in one queue ordered reverse units first (the costly ones), then
@@ -25,7 +25,7 @@
 // session, so a level's work fills the machine as long as the batch has any.
 //
 // Tape: each session names a tape of the module (Tapes::group<REV> switches on it); the tape
-// code is the per-tape straight-line code of tsi_jit.cpp, one namespace per tape.
+// code is the per-tape code of tsi_jit.cpp (a chain's loops or a straight line), one namespace per tape.
 #pragma once
 #include "tsi_eval.h"
 
@@ -210,6 +210,12 @@ TSI_DI void batch_run(const BatchArgs &b) {
             __syncthreads();
         }
         const uint32_t total = pre[m];
+        // a phase of no units (every block sees the same counts, which no later phase and no frame end
+        // writes) changes nothing: no barrier.  The dealloc cascade's tail is that in most frames.
+        if (total == 0u) {
+            __syncthreads();   // pre is read above and built again
+            continue;
+        }
 
         // ---- the queue's units (q, q + nq, q + 2 nq, ..): in the first round wavefront slot i takes
         //      unit i of the queue; then wavefronts claim cu units at a time from the queue's counter,
@@ -253,20 +259,22 @@ TSI_DI void batch_run(const BatchArgs &b) {
         if (!grid_sync(b, gen)) return;
     }
 
-    // ---- frame end: free-list merge (all threads of a block per session), then commit ----
-    for (uint32_t s = blockIdx.x; s < ns; s += nb) frame_end(b.sess[s].a, tid, blockDim.x);
-    if (!grid_sync(b, gen)) return;
-    // commit, the frame's counters for the host, and buf_main: the root re-enqueued for the
-    // session's next frame (compute.wgsl:4690-4707)
-    // (a wavefront per session)
-    for (uint32_t s = blockIdx.x * wpb + (tid >> 6); s < ns; s += nb * wpb) {
+    // ---- frame end, a block per session: free-list merge by all its threads, then by one wavefront the
+    //      commit, the frame's counters for the host, and buf_main: the root re-enqueued for the
+    //      session's next frame (compute.wgsl:4690-4707).  (With a session's end in one block
+    //      and the empty phases left out, a submit passes three grid barriers fewer.) ----
+    for (uint32_t s = blockIdx.x; s < ns; s += nb) {
         const KArgs &a = b.sess[s].a;
-        frame_commit(a);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the lanes' writes, for the copy below
-        const uint32_t *from = reinterpret_cast<const uint32_t *>(a.cnt);
-        uint32_t *to = reinterpret_cast<uint32_t *>(b.out + s);
-        for (uint32_t i = lane; i < uint32_t(sizeof(CounterHead) / 4); i += 64u) to[i] = from[i];
-        if (lane == 0) a.cnt->root_pending = 1u;
+        frame_end(a, tid, blockDim.x);
+        __syncthreads();   // every thread has read the counters that the commit changes
+        if (tid < 64u) {
+            frame_commit(a);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");   // the lanes' writes, for the copy below
+            const uint32_t *from = reinterpret_cast<const uint32_t *>(a.cnt);
+            uint32_t *to = reinterpret_cast<uint32_t *>(b.out + s);
+            for (uint32_t i = lane; i < uint32_t(sizeof(CounterHead) / 4); i += 64u) to[i] = from[i];
+            if (lane == 0) a.cnt->root_pending = 1u;
+        }
     }
 }
 
