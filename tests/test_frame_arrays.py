@@ -63,14 +63,14 @@ def test_buffers_are_bounded_and_outlive_their_context():
         st.set_inversion()
         kept = [st.trace()[0] for _ in range(4)]
         assert len({x.ctypes.data for x in kept}) == 4            # all in use
-        sizes, held = [96 << 20, 96 << 20, 96 << 20], []
-        for s in sizes:                                           # 256 MiB in all, kept's included
+        sizes, held = [384 << 20, 384 << 20, 384 << 20], []
+        for s in sizes:                                           # 1 GiB in all, kept's included
             p = lib.tsi_host_buffer(s)
             held.append(p)
         assert held[0] and held[1] and not held[2]
-        assert lib.tsi_host_buffer((256 << 20) + 1) is None
+        assert lib.tsi_host_buffer((1 << 30) + 1) is None
         for p in held[:2]:
-            C.memset(p, 1, 96 << 20)
+            C.memset(p, 1, 384 << 20)
             lib.tsi_host_buffer_free(p)
         # several threads
         seen, lock = [], threading.Lock()
