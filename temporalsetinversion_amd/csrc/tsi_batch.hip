@@ -638,7 +638,6 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
             J.t.grad = s.a.grad;
             J.t.mask = reinterpret_cast<const uint32_t *>(s.a.grad) + 3;
             J.t.mask_stride = 4u;
-            J.blocks_x = (r.width + kTraceTile - 1u) / kTraceTile;
             b->job_of[i] = int32_t(njobs);
             s.w = r.width;
             s.h = r.height;
@@ -668,20 +667,32 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
         // cinematic frames after the others, each group with its own launch (the path tracer's
         // kernel holds more registers; the plain trace keeps its own)
         TraceJob *jb = b->jobs_h;
-        std::stable_partition(jb, jb + njobs, [](const TraceJob &J) { return !(J.t.shading & TSI_SHADE_CINEMATIC); });
-        uint32_t nplain = 0, bplain = 0, bcin = 0;
+        // and in each the deepest octrees first: their rays are the longest chains, and a launch ends
+        // with the wavefronts that started last (28 frames up to 512x512 of depths 7-9 1.17 -> 0.95 ms, 24
+        // up to 640x480 of depths 6-9 0.88 -> 0.75)
+        auto cinematic = [](const TraceJob &J) { return (J.t.shading & TSI_SHADE_CINEMATIC) != 0; };
+        std::stable_sort(jb, jb + njobs, [&](const TraceJob &x, const TraceJob &y) {
+            return cinematic(x) != cinematic(y) ? cinematic(y) : x.t.stack > y.t.stack;
+        });
+        uint32_t nplain = 0, blocks[2] = {0, 0};
+        uint64_t pixels[2] = {0, 0};
         for (uint32_t j = 0; j < njobs; ++j) {
-            const bool cin = (jb[j].t.shading & TSI_SHADE_CINEMATIC) != 0;
-            uint32_t &acc = cin ? bcin : bplain;
-            jb[j].block0 = acc;
-            acc += jb[j].blocks_x * ((jb[j].t.height + kTraceTile - 1u) / kTraceTile);
-            nplain += cin ? 0u : 1u;
+            pixels[cinematic(jb[j])] += uint64_t(jb[j].t.width) * jb[j].t.height;
+            nplain += cinematic(jb[j]) ? 0u : 1u;
+        }
+        const bool quads[2] = {trace_quads(pixels[0], false), trace_quads(pixels[1], true)};
+        for (uint32_t j = 0; j < njobs; ++j) {
+            const bool cin = cinematic(jb[j]);
+            const uint32_t tile = quads[cin] ? 4u : 8u;   // a block's pixels: tile x tile
+            jb[j].block0 = blocks[cin];
+            jb[j].blocks_x = (jb[j].t.width + tile - 1u) / tile;
+            blocks[cin] += jb[j].blocks_x * ((jb[j].t.height + tile - 1u) / tile);
         }
         HIP_OK(hipMemcpyAsync(b->jobs_d, b->jobs_h, njobs * sizeof(TraceJob), hipMemcpyHostToDevice, b->stream));
         if (launch_fill_u32(reinterpret_cast<uint32_t *>(b->visits_d), 0u, 2u * njobs * kBatchVisitSlots * kTallyStride, b->stream)) return TSI_E_HIP;
         HIP_OK(hipEventRecord(b->ev[2], b->stream));
-        if (nplain && launch_trace_batch(b->jobs_d, nplain, bplain, false, stack, b->stream)) return TSI_E_HIP;
-        if (nplain < njobs && launch_trace_batch(b->jobs_d + nplain, njobs - nplain, bcin, true, stack, b->stream))
+        if (nplain && launch_trace_batch(b->jobs_d, nplain, blocks[0], false, quads[0], stack, b->stream)) return TSI_E_HIP;
+        if (nplain < njobs && launch_trace_batch(b->jobs_d + nplain, njobs - nplain, blocks[1], true, quads[1], stack, b->stream))
             return TSI_E_HIP;
         HIP_OK(hipMemcpyAsync(b->visits_h, b->visits_d,
                               size_t(njobs) * kBatchVisitSlots * kTallyStride * sizeof(unsigned long long), hipMemcpyDeviceToHost,

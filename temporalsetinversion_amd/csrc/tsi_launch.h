@@ -59,7 +59,6 @@ struct TraceArgs {
     uint32_t stack;             // ray-stack entries: more than the octree's paths need, or the reference's 16
 };
 
-constexpr uint32_t kTraceTile = 8;   // a batched trace block's pixels: kTraceTile x kTraceTile
 // claim counters of the persistent trace, each in a line of its own (2 * kTallyStride uint32 apart)
 constexpr uint32_t kTraceQueues = 8;
 // blocks > 0 (with next_quad, kTraceQueues counters zeroed on `s` before): the persistent form on that many
@@ -73,15 +72,16 @@ int launch_rgba8(const float4 *in, uchar4 *out, uint32_t n, hipStream_t s);
 struct TraceJob {
     const float4 *st, *blo, *bhi, *grad;
     TraceArgs t;
-    uint32_t blocks_x;  // ceil(width / kTraceTile): blocks per row
+    uint32_t blocks_x;  // blocks per row: ceil(width / side of a block's tile)
     uint32_t block0;    // the frame's first block in the launch
 };
 // (cinematic: every job's session shades with TSI_SHADE_CINEMATIC; no job mixes the two)
 // stack: the largest of the jobs' TraceArgs::stack.
-int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, uint32_t stack,
+int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, bool quads, uint32_t stack,
                        hipStream_t s);
 // Whether a frame is traced with four lanes per ray (by its size; full launches only).
 bool trace_quads(const TraceArgs &t);
+bool trace_quads(uint64_t pixels, bool cinematic);
 // TraceArgs::stack for an octree whose nodes lie at depths up to `depth`.
 uint32_t trace_stack_entries(int depth);
 // After a trace (visits as in TraceArgs): the visits' sum to *out (pinned host memory), and the counters

@@ -881,12 +881,12 @@ __global__ void __launch_bounds__(kTraceThreads) k_trace_quads(KArgs a, TraceArg
     add_visits<LaneG>(t, visits);
 }
 
-// The frames of a batch in one launch: block i is an 8x8-pixel tile of the frame whose blocks
-// [jobs[j].block0, jobs[j + 1].block0) hold it, row-major over ceil(width / 8) blocks per row
+// The frames of a batch in one launch: block i is a tile (shade_tile) of the frame whose blocks
+// [jobs[j].block0, jobs[j + 1].block0) hold it, row-major over blocks_x blocks per row
 // (a persistent grid taking tiles
 // from a counter measured slower: a frame's slowest tiles then ran one after another in a few
 // wavefronts, where the hardware dispatcher starts each block on the first free slot).
-template <bool CIN>
+template <class G, bool CIN>
 __global__ void __launch_bounds__(kTraceThreads) k_trace_batch(const TraceJob *jobs, uint32_t njobs) {
     extern __shared__ uint2 stack_lds[];
     const uint32_t blk = blockIdx.x;
@@ -917,10 +917,11 @@ __global__ void __launch_bounds__(kTraceThreads) k_trace_batch(const TraceJob *j
     t.visit_slots = J.t.visit_slots;
     t.stack = J.t.stack;
     const uint32_t local = blk - J.block0;
+    constexpr uint32_t side = G::kLanes == 1u ? 8u : 4u;
     uint32_t visits = 0;
-    shade_tile<LaneG, CIN>(a, t, (local % J.blocks_x) * kTraceTile, (local / J.blocks_x) * kTraceTile,
-                           LaneG::Stack{stack_lds + threadIdx.x}, visits);
-    add_visits<LaneG>(t, visits);
+    shade_tile<G, CIN>(a, t, (local % J.blocks_x) * side, (local / J.blocks_x) * side,
+                       typename G::Stack{stack_lds + threadIdx.x}, visits);
+    add_visits<G>(t, visits);
 }
 
 // See launch_trace_end: one wavefront.  (A memset before the trace and a copy after it: 7 us more.)
@@ -937,10 +938,11 @@ int launch_trace_end(unsigned long long *visits, uint32_t n_clear, unsigned long
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Frames of at most this many pixels are traced with four lanes per ray: their wavefronts then
+// Frames (a batch's together) of at most this many pixels are traced with four lanes per ray: their wavefronts then
 // still find free SIMDs, and the frame takes the latency of its longest chains, which are shorter so
 // (64x48 spheres: 88 against 108 us; csg at 362x362: 296 against 307).  Larger frames are bound by
 // instructions (448x448: capsules 382 against 327 us, csg 332 against 290, spheres 116 against 122).
+// A batch of one frame of 320x240: 90 against 118 us.
 // A path-traced pixel is 8 samples of up to 4 rays, chains so long that the line lies higher (csg at
 // 641x361: 6.7 against 7.2 ms, capsules 7.1 against 8.2; at 960x540 9.2 against 8.0 and 9.1 against 8.8).
 constexpr uint64_t kQuadPixels = 147456, kQuadPixelsCinematic = 393216;
@@ -950,15 +952,18 @@ static uint32_t stack_bytes(uint32_t entries) { return entries * kTraceThreads *
 
 uint32_t trace_stack_entries(int depth) { return std::min(kStackDepth, uint32_t(depth) + 3u); }
 
-int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, uint32_t stack,
+int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_blocks, bool cinematic, bool quads, uint32_t stack,
                        hipStream_t s) {
-    if (cinematic) hipLaunchKernelGGL(k_trace_batch<true>, dim3(total_blocks), dim3(kTraceThreads), stack_bytes(stack), s, jobs, njobs);
-    else hipLaunchKernelGGL(k_trace_batch<false>, dim3(total_blocks), dim3(kTraceThreads), stack_bytes(stack), s, jobs, njobs);
+    auto *k = quads ? (cinematic ? k_trace_batch<QuadG, true> : k_trace_batch<QuadG, false>)
+                    : (cinematic ? k_trace_batch<LaneG, true> : k_trace_batch<LaneG, false>);
+    hipLaunchKernelGGL(k, dim3(total_blocks), dim3(kTraceThreads), stack_bytes(stack), s, jobs, njobs);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+bool trace_quads(uint64_t pixels, bool cinematic) { return pixels <= (cinematic ? kQuadPixelsCinematic : kQuadPixels); }
+
 bool trace_quads(const TraceArgs &t) {
-    return uint64_t(t.width) * t.height <= (t.shading & TSI_SHADE_CINEMATIC ? kQuadPixelsCinematic : kQuadPixels);
+    return trace_quads(uint64_t(t.width) * t.height, (t.shading & TSI_SHADE_CINEMATIC) != 0);
 }
 
 int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blocks, uint32_t *next_quad) {
