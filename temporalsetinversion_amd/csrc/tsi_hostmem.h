@@ -21,7 +21,7 @@ struct CopyOut {
     const void *src;   // device
     size_t bytes;
 };
-// Device to host on an idle stream, complete on return.
+// Device to host, after the work queued on s; complete on return.
 int copy_out(const CopyOut *copies, int n, hipStream_t s);
 
 }  // namespace tsi

@@ -155,6 +155,8 @@ int copy_out(const CopyOut *copies, int n, hipStream_t s) {
     if (total == 0) return TSI_OK;
     char *stage = !pinned && total <= kStageBytes ? static_cast<char *>(acquire(total)) : nullptr;
     if (!pinned && !stage) {
+        // (these copies run on the null stream, which does not wait for the library's own streams)
+        if (hipStreamSynchronize(s) != hipSuccess) return TSI_E_HIP;
         for (int i = 0; i < n; ++i)
             if (copies[i].dst &&
                 hipMemcpy(copies[i].dst, copies[i].src, copies[i].bytes, hipMemcpyDeviceToHost) != hipSuccess)
