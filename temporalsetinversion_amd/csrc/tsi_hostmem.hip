@@ -40,8 +40,9 @@ Pool &pool() {
     return *p;
 }
 
-// idle buffers, the largest first, until `bytes` more fit (m held)
+// idle buffers, the largest first, until `bytes` more fit (m held; throws before it takes any)
 void trim(Pool &P, size_t bytes, std::vector<void *> &gone) {
+    if (P.bytes + bytes > kPoolBytes) gone.reserve(P.idle.size());
     while (!P.idle.empty() && P.bytes + bytes > kPoolBytes) {
         const auto it = std::prev(P.idle.end());
         gone.push_back(it->second);
@@ -65,7 +66,7 @@ bool pooled(const void *p, size_t bytes) {
     return b + bytes <= a + it->second;
 }
 
-void *acquire(size_t bytes) {
+void *acquire_or_throw(size_t bytes) {
     Pool &P = pool();
     bytes = (bytes + kGrain - 1) / kGrain * kGrain;
     if (bytes == 0 || bytes > kPoolBytes) return nullptr;
@@ -102,6 +103,15 @@ void *acquire(size_t bytes) {
         return nullptr;
     }
     return p;
+}
+
+// (null as well where the host has no memory for the pool's own records)
+void *acquire(size_t bytes) noexcept {
+    try {
+        return acquire_or_throw(bytes);
+    } catch (...) {
+        return nullptr;
+    }
 }
 
 void release_buffer(void *p) {
@@ -189,11 +199,7 @@ using namespace tsi;
 extern "C" {
 
 void *tsi_host_buffer(size_t bytes) {
-    try {
-        return acquire(bytes);
-    } catch (...) {
-        return nullptr;
-    }
+    return acquire(bytes);
 }
 
 void tsi_host_buffer_free(void *p) {
