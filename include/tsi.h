@@ -232,7 +232,8 @@ int tsi_save_frame_png(tsi_ctx *ctx, const char *path);
 /* No counterpart in the reference.  Pinned host memory for the pixels of tsi_trace, tsi_trace_wait,
  * tsi_frame_rgba8 and tsi_batch_frame: copies to it run at the link's rate.  From a pool of at most
  * 1 GiB, handed out and idle together, shared by all threads; idle buffers are given back when the
- * last context or batch is destroyed.  NULL: the pool is exhausted, or there is no context. */
+ * last context or batch is destroyed.  NULL: the pool is exhausted, or there is no context.  A
+ * forked process has copies of the buffers handed out, in ordinary memory, and gets no new ones. */
 void *tsi_host_buffer(size_t bytes);
 void tsi_host_buffer_free(void *buffer);
 

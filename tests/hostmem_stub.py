@@ -15,6 +15,7 @@ RUNTIME = r"""
 #include <cstring>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <new>
 #include <cstdlib>
 #include <vector>
@@ -31,6 +32,7 @@ constexpr unsigned hipHostMallocPortable = 1u;
 struct Stream { std::vector<std::function<void()>> queue; };
 typedef Stream *hipStream_t;
 inline size_t &pinned_bytes() { static size_t n = 0; return n; }
+inline std::mutex &pinned_mutex() { static std::mutex m; return m; }
 inline std::map<void *, size_t> &pinned() { static std::map<void *, size_t> m; return m; }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
@@ -50,12 +52,14 @@ inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     *p = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
     if (*p == MAP_FAILED) return hipErrorOutOfMemory;
     madvise(*p, n, MADV_DONTFORK);
+    std::lock_guard<std::mutex> g(pinned_mutex());
     pinned()[*p] = n;
     pinned_bytes() += n;
     return hipSuccess;
 }
 inline hipError_t hipHostFree(void *p) {
     Allocating allocating;
+    std::lock_guard<std::mutex> g(pinned_mutex());
     pinned_bytes() -= pinned()[p];
     munmap(p, pinned()[p]);
     pinned().erase(p);
