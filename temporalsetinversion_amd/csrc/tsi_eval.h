@@ -461,9 +461,10 @@ TSI_DI void flush_tally(uint64_t *tally, const LevelTally &t, int level = -1) {
 }
 
 // The level kernels' time without events between them (3.2 us each, two a level: an eighth of a
-// 256 x 256 preview).  One wavefront of a level's launch notes when it began and, from the latest end
-// of the level before (two words per slot in turn: nothing of this level writes that one), adds
-// that level's time.  The last level's is added by the commit.
+// 256 x 256 preview).  The first block of a level's launch notes when it began, every wavefront when it
+// ended (flush_tally), and a wavefront of the last block, which has the least to do, adds the time of the
+// level before; the last level's is added by the commit.  Starts and ends of two levels in turn: nothing
+// of this level writes those of the one before.
 TSI_DI uint64_t latest_end(const KArgs &a, int level) {
     static_assert(kTallySlots == 64 && kNumStats + 2 <= kTallyStride, "a slot per lane, two words after the statistics");
     uint64_t v = a.tally[lane_id() * kTallyStride + kNumStats + (level & 1)];
@@ -474,13 +475,22 @@ TSI_DI uint64_t latest_end(const KArgs &a, int level) {
     return v;
 }
 
-TSI_DI void level_clock(const KArgs &a, int level) {
-    const uint64_t now = __builtin_amdgcn_s_memrealtime();
-    const uint64_t end = level > 0 ? latest_end(a, level - 1) : 0u;
-    if (lane_id() != 0) return;
+// of the level that began last in this slot of clk_start
+TSI_DI uint64_t level_time(const KArgs &a, int level) {
+    const uint64_t begin = a.cnt->clk_start[level & 1], end = latest_end(a, level);
+    return end > begin ? end - begin : 0u;
+}
+
+// Block b of a level's nb blocks, by one of its wavefronts.  (With the start taken by the last block, which
+// on a frontier of more blocks than the chip holds begins when others are done, the levels of 6.5
+// million cells counted as 0.43 ms of their 0.95.)
+TSI_DI void level_clock(const KArgs &a, int level, uint32_t b, uint32_t nb) {
     Counters *c = a.cnt;
-    if (level > 0 && end > c->clk_start) c->level_ticks += end - c->clk_start;
-    c->clk_start = now;
+    if (b == 0u && lane_id() == 0) c->clk_start[level & 1] = __builtin_amdgcn_s_memrealtime();
+    if (b != nb - 1u) return;
+    const uint64_t before = level > 0 ? level_time(a, level - 1) : 0u;
+    if (lane_id() != 0) return;
+    c->level_ticks += before;
     c->clk_level = level;
 }
 
@@ -634,9 +644,9 @@ TSI_DI void frame_commit(const KArgs &a) {
         for (uint32_t i = 0; i < kTallySlots; ++i) v += a.tally[i * kTallyStride + k];
         cnt->stats[k] = v;
     }
-    const uint64_t end = cnt->clk_level >= 0 ? latest_end(a, cnt->clk_level) : 0u;
+    const uint64_t last = cnt->clk_level >= 0 ? level_time(a, cnt->clk_level) : 0u;
     if (k != 0) return;
-    if (end > cnt->clk_start) cnt->level_ticks += end - cnt->clk_start;
+    cnt->level_ticks += last;
     const uint32_t T = cnt->alloc_tickets, F = cnt->free_top, P = min(cnt->pending, a.nblocks);
     const uint32_t used = T < F ? T : F;
     uint32_t bump = cnt->bump + (T > F ? T - F : 0u);

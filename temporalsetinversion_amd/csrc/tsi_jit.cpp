@@ -1884,7 +1884,7 @@ std::string jit_source_level(const tsi_gpu_instruction *tape, uint32_t n, const 
     o += "    const uint32_t nb = gridDim.x, b = blockIdx.x, w = threadIdx.x >> 6;\n"
          "    // level -1: the frame's speculative pass, on the whole grid (reverse list code)\n"
          "    const uint32_t nf = level < 0 ? 0u : __builtin_amdgcn_readfirstlane(tsi::level_split(a, level, nb));\n"
-         "    if (level >= 0 && b == nb - 1u && w == 3u) tsi::level_clock(a, level);\n"
+         "    if (level >= 0 && w == 3u && (b == 0u || b == nb - 1u)) tsi::level_clock(a, level, b, nb);\n"
          "    const uint32_t bwave = b * 4u + w;\n"
          "    if (b < nf)\n"
          "        tsi::eval_level<false, tsi::jf::TapeEngine>(a, level, time, bwave, nf * 4u, bwave);\n"

@@ -55,8 +55,8 @@ struct Counters : CounterHead {
     alignas(128) uint32_t alloc_tickets;      // blocks handed out this frame
     alignas(128) uint32_t pending;            // blocks freed this frame
     alignas(128) uint32_t finished;           // blocks of k_frame_end that are done
-    alignas(128) uint64_t clk_start;          // when the level kernel running now began (level_clock)
-    int32_t clk_level;
+    alignas(128) uint64_t clk_start[2];       // when a level kernel began, by the level's parity (level_clock)
+    int32_t clk_level;                        // the level running now
     struct Level {
         alignas(128) uint32_t list[2];        // frontier sizes: [0] forward-only, [1] reverse
         alignas(128) uint32_t dlist;          // dealloc cascade list size
