@@ -233,13 +233,16 @@ void arena_give(tsi_batch *b, uint64_t off, uint64_t bytes) {
 }
 
 // Records for up to 32 768 entries of each of a session's lists, fewer where many sessions share
-// 4 GiB (the speculative pass's cells first, if they take less than half).  Cells beyond them, or all (no memory), run the whole tape: the same results.
+// 4 GiB or the share of the memory left beside the arena (chain_memory); the speculative pass's cells first, if
+// they take less than half.  Cells beyond them, or all (no memory), run the whole tape: the same results.
+// (Where that matters: csg's first frame at 1024^3 from an empty octree, 1.8 million cells, takes 2.5 ms with
+// 32 768 entries and 1.7 with all; its animated frames, 0.3-0.7 million, the same 0.56 and 1.06.)
 void alloc_records(tsi_batch *b) {
     uint32_t words = 0, cols = 0;
     for (uint32_t w : b->rec_words) words = std::max(words, w);
     for (uint32_t w : b->col_words) cols = std::max(cols, w);
     if (!words) return;
-    const uint64_t budget = (uint64_t(4) << 30) / 4u / b->cfg.max_sessions;   // words per session
+    const uint64_t budget = std::min(uint64_t(4) << 30, chain_memory()) / 4u / b->cfg.max_sessions;   // words per session
     uint64_t spec = uint64_t(b->spec_cap) * 8u * words;
     if (budget < 2u * spec) spec = 0;
     b->rec_spec = spec != 0;
@@ -447,7 +450,6 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
             (rc = hmalloc(&b->out_h, C.max_sessions)) || (rc = hmalloc(&b->error_h, 1)) || (rc = hmalloc(&b->jobs_h, C.max_sessions)) ||
             (rc = hmalloc(&b->visits_h, size_t(C.max_sessions) * kBatchVisitSlots * kTallyStride)))
             break;
-        alloc_records(b);
         uint64_t arena = C.arena_bytes;
         if (arena == 0) {
             size_t fr = 0, tot = 0;
@@ -456,6 +458,7 @@ int tsi_batch_create(const tsi_gpu_instruction *const *tapes, const uint32_t *le
         }
         arena = arena / kAlign * kAlign;
         if ((rc = dmalloc(&b->arena, arena))) break;
+        alloc_records(b);
         b->arena_bytes = arena;
         b->free_ranges[0] = arena;
         b->sessions.resize(C.max_sessions);

@@ -91,6 +91,9 @@ int launch_trace_end(unsigned long long *visits, uint32_t n_clear, unsigned long
 // through nodes with children, keyed by (depth, i, j, k).  Synchronous device reads.
 int read_octree(const float4 *st_dev, const float4 *grad_dev, const Counters *cnt_dev, uint64_t nodes, tsi_node *out,
                 uint64_t cap, uint64_t *count);
+// Bytes that a chain's records (JitChain) may take on the current device: an eighth of what is free.  They
+// only save work, and a program's own allocations after them would miss them.
+uint64_t chain_memory();
 // p[0 .. n) = v (a kernel, not a memset node, so that it also replays correctly in a captured graph)
 int launch_fill_u32(uint32_t *p, uint32_t v, uint32_t n, hipStream_t s);
 

@@ -318,20 +318,24 @@ int alloc_prune(tsi_ctx *c, const Lowered &L, const std::vector<FwdIns> &fwd) {
 }
 
 // Buffers of the unpruned kernels of a tape that is a chain (JitChain): records for as many entries
-// of each frontier list as pruned evaluation keeps, columns per wavefront, and the speculative
-// pass's.  Without them (no memory) every cell runs the whole tape: the same results.
+// of each frontier list as pruned evaluation keeps, or as its share of the memory holds
+// (chain_memory), columns per wavefront, and the speculative pass's.  Without them (no memory) every cell
+// runs the whole tape: the same results.
 void alloc_chain(tsi_ctx *c, const JitChain &chain) {
     uint64_t cap = c->p.prune_capacity ? c->p.prune_capacity : (uint64_t(1) << 19);
     if (cap > c->list_cap) cap = c->list_cap;
     cap = (cap + 7) / 8 * 8;
-    const uint32_t waves = (c->grid_fwd + c->grid_rev) * 4u;
+    const size_t choice = size_t(c->grid_fwd + c->grid_rev) * 4u * 64u * chain.col_words;
+    const size_t spec_choice = c->spec_max ? size_t(c->num_cu) * 4u * 64u * chain.col_words : 0;
+    const size_t spec_rec = c->spec_max ? size_t(chain.record_words) * c->spec_cap * 8u : 0;
+    const uint64_t words = chain_memory() / sizeof(uint32_t), fixed = choice + spec_choice + spec_rec;
+    cap = std::min(cap, words > fixed ? (words - fixed) / (4u * chain.record_words) / 8u * 8u : 0u);
+    if (cap == 0) return;
     bool ok = true;
     for (auto &l : c->prune_rec)
         for (auto &x : l) ok = ok && dmalloc(&x, size_t(chain.record_words) * cap) == TSI_OK;
-    ok = ok && dmalloc(&c->choice, size_t(waves) * 64u * chain.col_words) == TSI_OK;
-    if (c->spec_max)
-        ok = ok && dmalloc(&c->spec_choice, size_t(c->num_cu) * 4u * 64u * chain.col_words) == TSI_OK &&
-             dmalloc(&c->spec_rec, size_t(chain.record_words) * c->spec_cap * 8u) == TSI_OK;
+    ok = ok && dmalloc(&c->choice, choice) == TSI_OK;
+    if (c->spec_max) ok = ok && dmalloc(&c->spec_choice, spec_choice) == TSI_OK && dmalloc(&c->spec_rec, spec_rec) == TSI_OK;
     if (!ok) {
         (void)hipGetLastError();
         release_prune(c);
@@ -340,6 +344,19 @@ void alloc_chain(tsi_ctx *c, const JitChain &chain) {
     c->prune_cap = uint32_t(cap);
     c->choice_len = chain.col_words;
     c->chain = true;
+}
+
+// Memory that a context turns out to need after its tape: a chain's records, which only save work, go
+// first.
+template <class T>
+int late_dmalloc(tsi_ctx *c, T **p, size_t count) {
+    const int rc = dmalloc(p, count);
+    if (rc == TSI_OK || !c->chain) return rc;
+    (void)hipGetLastError();
+    HIP_OK(hipStreamSynchronize(c->stream));
+    HIP_OK(hipStreamSynchronize(c->spec_stream));
+    release_prune(c);
+    return dmalloc(p, count);
 }
 
 void release_jit(tsi_ctx *c) {
@@ -446,6 +463,15 @@ void release(tsi_ctx *c) {
 }  // namespace
 
 namespace tsi {
+
+uint64_t chain_memory() {
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return free_bytes / 8u;
+}
 
 int read_octree(const float4 *st_dev, const float4 *grad_dev, const Counters *cnt_dev, uint64_t nodes, tsi_node *out,
                 uint64_t cap, uint64_t *count) {
@@ -945,7 +971,7 @@ int start_trace(tsi_ctx *c, bool overlap) {
         dfree(ts.rgba);
         dfree(ts.depth);
         ts.px = 0;
-        if ((rc = dmalloc(&ts.rgba, px)) || (rc = dmalloc(&ts.depth, px))) return rc;
+        if ((rc = late_dmalloc(c, &ts.rgba, px)) || (rc = late_dmalloc(c, &ts.depth, px))) return rc;
         ts.px = px;
     }
     KArgs a = make_args(c);
@@ -954,14 +980,14 @@ int start_trace(tsi_ctx *c, bool overlap) {
     hipStream_t s = c->stream;
     if (overlap) {
         if (!ts.st) {
-            if ((rc = dmalloc(&ts.st, c->nodes)) || (rc = dmalloc(&ts.blo, c->nodes)) || (rc = dmalloc(&ts.bhi, c->nodes)) ||
-                (rc = dmalloc(&ts.mask, c->nodes))) {
+            if ((rc = late_dmalloc(c, &ts.st, c->nodes)) || (rc = late_dmalloc(c, &ts.blo, c->nodes)) || (rc = late_dmalloc(c, &ts.bhi, c->nodes)) ||
+                (rc = late_dmalloc(c, &ts.mask, c->nodes))) {
                 dfree(ts.st); dfree(ts.blo); dfree(ts.bhi); dfree(ts.mask);
                 return rc;
             }
         }
         // snapshot of the nodes in use, in stream order after the last set inversion
-        if (gradient_normals && !ts.grad && (rc = dmalloc(&ts.grad, c->nodes))) return rc;
+        if (gradient_normals && !ts.grad && (rc = late_dmalloc(c, &ts.grad, c->nodes))) return rc;
         if (launch_snapshot(a, ts.st, ts.blo, ts.bhi, gradient_normals ? ts.grad : nullptr, ts.mask, c->nodes,
                             c->grid_misc, c->stream) != 0)
             return TSI_E_HIP;
@@ -1052,7 +1078,7 @@ int tsi_frame_rgba8(tsi_ctx *c, uint8_t *rgba8_out) {
     if (px > c->rgba8_px) {   // kept for the next frame: allocating and freeing wait for the device
         dfree(c->rgba8);
         c->rgba8_px = 0;
-        if ((rc = dmalloc(&c->rgba8, px))) return rc;
+        if ((rc = late_dmalloc(c, &c->rgba8, px))) return rc;
         c->rgba8_px = px;
     }
     // (on the frame's own stream: the trace is done, set inversions in flight are not waited for)
