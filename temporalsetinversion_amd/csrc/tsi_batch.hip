@@ -160,6 +160,7 @@ int dmalloc(T **p, size_t count) {
     *p = nullptr;
     if (count == 0) count = 1;
     if (hipMalloc(reinterpret_cast<void **>(p), count * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();   // (else the next launch reports it)
         *p = nullptr;
         return TSI_E_OOM;
     }
@@ -177,6 +178,7 @@ int hmalloc(T **p, size_t count) {
     *p = nullptr;
     if (hipHostMalloc(reinterpret_cast<void **>(p), (count ? count : 1) * sizeof(T), hipHostMallocDefault) !=
         hipSuccess) {
+        (void)hipGetLastError();   // (else the next launch reports it)
         *p = nullptr;
         return TSI_E_OOM;
     }
@@ -254,7 +256,6 @@ void alloc_records(tsi_batch *b) {
     b->rec_stride = size_t(4u * words * cap + spec);
     if (dmalloc(&b->rec, b->rec_stride * b->cfg.max_sessions) != TSI_OK ||
         dmalloc(&b->choice, size_t(b->num_cu) * b->max_bpc * 4u * 64u * cols) != TSI_OK) {
-        (void)hipGetLastError();
         dfree(b->rec);
         dfree(b->choice);
     }

@@ -184,6 +184,7 @@ int dmalloc(T **p, size_t count) {
     *p = nullptr;
     if (count == 0) count = 1;
     if (hipMalloc(reinterpret_cast<void **>(p), count * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();   // (else the next launch reports it)
         *p = nullptr;
         return TSI_E_OOM;
     }
@@ -337,7 +338,6 @@ void alloc_chain(tsi_ctx *c, const JitChain &chain) {
     ok = ok && dmalloc(&c->choice, choice) == TSI_OK;
     if (c->spec_max) ok = ok && dmalloc(&c->spec_choice, spec_choice) == TSI_OK && dmalloc(&c->spec_rec, spec_rec) == TSI_OK;
     if (!ok) {
-        (void)hipGetLastError();
         release_prune(c);
         return;
     }
@@ -352,7 +352,6 @@ template <class T>
 int late_dmalloc(tsi_ctx *c, T **p, size_t count) {
     const int rc = dmalloc(p, count);
     if (rc == TSI_OK || !c->chain) return rc;
-    (void)hipGetLastError();
     HIP_OK(hipStreamSynchronize(c->stream));
     HIP_OK(hipStreamSynchronize(c->spec_stream));
     release_prune(c);
