@@ -82,6 +82,9 @@ int launch_trace_batch(const TraceJob *jobs, uint32_t njobs, uint32_t total_bloc
 // Whether a frame is traced with four lanes per ray (by its size; full launches only).
 bool trace_quads(const TraceArgs &t);
 bool trace_quads(uint64_t pixels, bool cinematic);
+// Whether a full launch's grid holds the frame (else only the persistent form can trace it): its tiles are 4
+// or 8 pixels high and the grid at most 65 535 of them, 262 140 or 524 280 rows of pixels.
+bool trace_grid_fits(const TraceArgs &t);
 // TraceArgs::stack for an octree whose nodes lie at depths up to `depth`.
 uint32_t trace_stack_entries(int depth);
 // After a trace (visits as in TraceArgs): the visits' sum to *out (pinned host memory), and the counters

@@ -1023,6 +1023,7 @@ int start_trace(tsi_ctx *c, bool overlap) {
         // elsewhere, up to 1920x1080 and 8 CSG frames at 1024^3, within 4 % of full launches)
         blocks = 12u * uint32_t(c->num_cu);
     }
+    if (blocks == 0 && !trace_grid_fits(t)) blocks = 12u * uint32_t(c->num_cu);
     if (launch_trace(a, t, s, blocks, reinterpret_cast<uint32_t *>(ts.visits + kVisitSlots * kTallyStride)) != 0) return TSI_E_HIP;
     if (launch_trace_end(ts.visits, uint32_t(kTraceCounters), ts.visits_h, s) != 0) return TSI_E_HIP;
     HIP_OK(hipEventRecord(ts.end, s));

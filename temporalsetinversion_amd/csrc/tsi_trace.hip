@@ -966,6 +966,16 @@ bool trace_quads(const TraceArgs &t) {
     return trace_quads(uint64_t(t.width) * t.height, (t.shading & TSI_SHADE_CINEMATIC) != 0);
 }
 
+constexpr uint32_t kMaxGridRows = 65535;   // what a grid's second dimension may hold
+
+// pixels of a side of a full launch's tile (shade_tile)
+static uint32_t tile_of(bool quads) { return quads ? 4u : 8u; }
+
+bool trace_grid_fits(const TraceArgs &t) {
+    const uint32_t tile = tile_of(trace_quads(t));
+    return t.height <= kMaxGridRows * tile;
+}
+
 int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blocks, uint32_t *next_quad) {
     const bool cin = (t.shading & TSI_SHADE_CINEMATIC) != 0;
     if (blocks && next_quad) {   // persistent: `blocks` blocks, *next_quad zeroed on the stream before
@@ -976,7 +986,7 @@ int launch_trace(const KArgs &a, const TraceArgs &t, hipStream_t s, uint32_t blo
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const bool quad = trace_quads(t);
-    const uint32_t tile = quad ? 4u : 8u;
+    const uint32_t tile = tile_of(quad);
     const dim3 grid((t.width + tile - 1u) / tile, (t.height + tile - 1u) / tile);
     if (quad) {
         if (cin) hipLaunchKernelGGL((k_trace<QuadG, true>), grid, dim3(kTraceThreads), stack_bytes(t.stack), s, a, t);
