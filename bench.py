@@ -8,8 +8,10 @@ re-enqueue, at t_k = k/60.  The first W frames are untimed warm-up (frame 0 eval
 cell); the next K frames are timed with the device synchronised on both sides.
 
 Prints one JSON line.  `value` = interval cell-evals per second over the timed frames;
-`roofline` reports the tape-evaluation kernel against the FP32 VALU peak (its device time by the
-device's clock, from a level's first block to its last); `temporal_vs_full` compares the set inversion of
+`roofline` reports the tape-evaluation kernel against the FP32 VALU peak: the VALU instructions that
+the committed counter run of the workload saw, over the kernel's time in this run (by the device's
+clock, from a level's first block to its last), and apart from that the rate at which whole-tape
+operations are answered (`whole_tape`), most of them from decisions of a cell's parents, not run; `temporal_vs_full` compares the set inversion of
 the temporal frames with full re-evaluation (every frame from an empty octree), the quantity
 the reference publishes (~3x at 1024^3, delta 0.01); `cpu_baseline` times the oracle (the C
 restatement of the reference) on a bounded sample of the same workload.
@@ -62,21 +64,24 @@ def _profile_path(workload: str) -> str:
 
 
 def profiled_traffic(workload: str, engine: str):
-    """(HBM bytes per eval launch, summary path, average kernel us) from the committed rocprofv3
-    summary of this workload (timed frames only), if any."""
+    """(HBM bytes per eval launch, summary path, average kernel us, wave64 VALU instructions per eval
+    launch) from the committed rocprofv3 summary of this workload (timed frames only), if any."""
     path = _profile_path(workload)
     if engine != "compiled" or not os.path.exists(path):
-        return None, None, None
-    traffic = avg = None
+        return None, None, None, None
+    traffic = avg = valu = None
     for line in open(path):
         parts = line.split()
-        # "tsi_tape_eval_level timed <n> dispatches avg_us <us>" and
-        # "tsi_tape_eval_level hbm <n> <fetch KiB> <write KiB> <bytes per dispatch>"
+        # "tsi_tape_eval_level timed <n> dispatches avg_us <us>",
+        # "tsi_tape_eval_level hbm <n> <fetch KiB> <write KiB> <bytes per dispatch>" and
+        # "SQ_INSTS_VALU <instructions per dispatch>"
         if len(parts) >= 6 and parts[0] == "tsi_tape_eval_level" and parts[1] == "timed":
             avg = float(parts[5])
         if len(parts) >= 6 and parts[0] == "tsi_tape_eval_level" and parts[1] == "hbm":
             traffic = float(parts[5])
-    return traffic, os.path.relpath(path, ROOT), avg
+        if len(parts) == 2 and parts[0] == "SQ_INSTS_VALU":
+            valu = float(parts[1])
+    return traffic, os.path.relpath(path, ROOT), avg, valu
 
 
 def _csv_rows(path):
@@ -542,6 +547,20 @@ def make_state(T, w, tape, prune, engine):
                    prune={"on": True, "off": False, "exact": "exact"}[prune], engine=engine)
 
 
+def pruned_per_cell(st, warmup, steps):
+    """Records left out per evaluated cell over the timed frames of a run (after its warm-up)."""
+    st.reset()
+    pruned = cells = 0
+    for k in range(warmup + steps):
+        st.update(float(np.float32(k / 60.0)))
+        s = st.set_inversion().stats
+        st.enqueue_root()
+        if k >= warmup:
+            pruned += s["pruned_instr"]
+            cells += s["cell_evals"]
+    return pruned / max(cells, 1)
+
+
 # ---------------------------------------------------------------- batched and served forms
 
 # node capacity per session by octree depth (generous: a request that still exhausts its pool is
@@ -833,6 +852,8 @@ def main():
     prune = args.prune if args.prune != "auto" else "off"
     st = make_state(T, w, tape, prune, args.engine)
     info = st.tape_info()
+    # a chain's kernels (loops over segments that a cell's parents left undecided)
+    chain = info["engine"] == "compiled" and "kSkip = true" in T.kernel_source(tape, prune=False)[0]
     st.reset()
     frame = 0
 
@@ -915,12 +936,23 @@ def main():
                                           "full_cell_evals": f_cells}
     st.close()
 
+    launches = max(tot["launches"], 1)
     ops = tot["fwd_ops"] + tot["rev_ops"]
     kernel_s = tot["kernel_ms"] * 1e-3
-    achieved = ops / kernel_s / 1e12 if kernel_s > 0 else 0.0
-    launches = max(tot["launches"], 1)
-    traffic, traffic_src, prof_avg_us = profiled_traffic(args.workload, info["engine"])
-    # trace: SURVEY-style algorithmic bytes, 40 B per node visit + 20 B per pixel (colour + depth)
+    answered = ops / kernel_s / 1e12 if kernel_s > 0 else 0.0
+    traffic, traffic_src, prof_avg_us, valu = profiled_traffic(args.workload, info["engine"])
+    # what the VALU did: a wave64 instruction is 64 operations.  (The interpreter counts what it runs.)
+    achieved, achieved_from = answered, "operations counted by the kernels"
+    if info["engine"] == "compiled":
+        achieved = valu * 64 * launches / kernel_s / 1e12 if valu and kernel_s > 0 else None
+        achieved_from = f"SQ_INSTS_VALU x 64 per launch ({traffic_src}), over this run's time" if achieved else None
+    records_run = (len(tape) - 4) - tot["pruned"] / max(tot["cells"], 1)
+    if chain and prune == "off":
+        # with pruning refused a chain's kernels report the whole tape for every cell; the same kernels
+        # report the records run where it is allowed: the same frames again, untimed
+        with make_state(T, w, tape, "on", args.engine) as st2:
+            records_run = (len(tape) - 4) - pruned_per_cell(st2, args.warmup, args.steps)
+    # trace: algorithmic bytes, 40 B per node visit + 20 B per pixel (colour + depth)
     px = w["width"] * w["height"]
     trace_bytes = trace["visits"] * 40 + args.steps * px * 20
     trace_gbs = trace_bytes / (trace["ms"] * 1e-3) / 1e9 if trace["ms"] > 0 else 0.0
@@ -942,9 +974,9 @@ def main():
                    "lipschitz_corrected": w["lipschitz_corrected"], "swept_volume": w["swept_volume"],
                    "point_sample": w["point_sample"], "times": "t_k = k/60", "engine": info["engine"],
                    "trace": "synchronous" if args.sync_trace else "overlapped with the next set inversion",
-                   "prune": prune, "frames_in_flight": 1 if args.sync_trace else 2},
+                   "prune": prune, "skips_decided_segments": chain, "frames_in_flight": 1 if args.sync_trace else 2},
         "tape_compile_s": info["compile_ms"] / 1e3, "tape_compile_cached": bool(info["cache_hit"]),
-        "records_run_per_cell": (len(tape) - 4) - tot["pruned"] / max(tot["cells"], 1),
+        "records_run_per_cell": records_run,
         "set_inversion_ms_per_frame": tot["gpu_ms"] / args.steps,
         "cell_evals_per_frame": tot["cells"] / args.steps,
         "rev_evals_per_frame": tot["rev"] / args.steps,
@@ -953,22 +985,21 @@ def main():
                      "kernel": ("tsi_tape_eval_level (one launch per octree level: forward-only and reverse lists)"
                                 if info["engine"] == "compiled" else
                                 "k_eval (one launch per octree level: forward-only and reverse lists)"),
-                     "achieved": achieved, "peak": PEAK_VALU_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_VALU_TFLOPS,
-                     "frac_vs_unpacked_issue": achieved / PEAK_VALU_UNPACKED_TOPS,
+                     "achieved": achieved, "achieved_from": achieved_from, "peak": PEAK_VALU_TFLOPS, "unit": "TFLOP/s",
+                     "frac": achieved / PEAK_VALU_TFLOPS if achieved is not None else None,
+                     "frac_vs_unpacked_issue": achieved / PEAK_VALU_UNPACKED_TOPS if achieved is not None else None,
                      "peak_unpacked_issue": PEAK_VALU_UNPACKED_TOPS,
                      "traffic": traffic, "traffic_unit": "HBM bytes per launch", "traffic_source": traffic_src,
-                     # (of the full tape in every cell: records whose outcome a cell's parents decided are
-                     # counted, not run)
-                     "algorithmic_ops_per_launch": ops / launches,
-                     "ops_per_cell_eval": ops / max(tot["cells"], 1),
+                     "whole_tape": {"what": "operations of the full tape in every evaluated cell over the levels' time, "
+                                            "whether run or known from a cell's parents: not VALU work",
+                                    "tera_ops_per_s": answered, "ops_per_launch": ops / launches,
+                                    "ops_per_cell_eval": ops / max(tot["cells"], 1), "ops_per_frame": ops / args.steps},
                      # the levels' time by the device's clock (tsi_stats.eval_kernel_ms), over the timed frames
                      "avg_launch_us": tot["kernel_ms"] * 1e3 / launches,
                      # the same kernel's average over the timed frames of the committed rocprofv3 summary
                      "profile_avg_kernel_us": prof_avg_us,
                      "eval_ms_per_frame": tot["kernel_ms"] / args.steps,
-                     "eval_span_ms_per_frame": tot["eval_ms"] / args.steps,
-                     "ops_per_frame": ops / args.steps},
+                     "eval_span_ms_per_frame": tot["eval_ms"] / args.steps},
         "roofline_trace": {"bound": "hbm", "kernel": "k_trace / k_trace_quads (the form the runtime picks per frame)",
                            "achieved": trace_gbs, "peak": PEAK_HBM_GBS,
                            "unit": "GB/s", "frac": trace_gbs / PEAK_HBM_GBS,
