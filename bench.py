@@ -949,9 +949,11 @@ def main():
     records_run = (len(tape) - 4) - tot["pruned"] / max(tot["cells"], 1)
     if chain and prune == "off":
         # with pruning refused a chain's kernels report the whole tape for every cell; the same kernels
-        # report the records run where it is allowed: the same frames again, untimed
-        with make_state(T, w, tape, "on", args.engine) as st2:
-            records_run = (len(tape) - 4) - pruned_per_cell(st2, args.warmup, args.steps)
+        # report the records run where it is allowed: the same frames again, untimed (not in a profiled run)
+        records_run = None
+        if not args.no_full:
+            with make_state(T, w, tape, "on", args.engine) as st2:
+                records_run = (len(tape) - 4) - pruned_per_cell(st2, args.warmup, args.steps)
     # trace: algorithmic bytes, 40 B per node visit + 20 B per pixel (colour + depth)
     px = w["width"] * w["height"]
     trace_bytes = trace["visits"] * 40 + args.steps * px * 20
