@@ -257,7 +257,7 @@ typedef struct {
     uint32_t stack;               /* saved operand intervals per lane (reverse pass) */
     uint32_t slots;               /* interpreter register-file slots used */
     uint32_t prune_class;         /* 0 never pruned, 1 pruned up to ulp-level decisions, 2 exact */
-    uint32_t engine;              /* 0 interpreter, 1 compiled straight-line kernels */
+    uint32_t engine;              /* 0 interpreter, 1 compiled kernels */
     uint32_t cache_hit;           /* compiled kernels came from the code-object cache */
     uint32_t specialized;         /* the kernels assume every cell box inside [-5,5]^3 and every
                                      t-window inside [-2, 64] (rebuilt without it otherwise) */
@@ -269,14 +269,19 @@ int tsi_tape_info_get(tsi_ctx *ctx, tsi_tape_info *out);
 
 /* Compiles a tape's evaluation kernels into the code-object cache without a device or
  * context (no counterpart in the reference): a later tsi_upload_tape of the same tape with the
- * same pruning flags (TSI_FLAG_NO_PRUNE, TSI_FLAG_PRUNE_EXACT_ONLY) then only loads them.  Cache directory: $TSI_JIT_CACHE, else $XDG_CACHE_HOME/tsi-jit, else
- * ~/.cache/tsi-jit. */
+ * same pruning flags (TSI_FLAG_NO_PRUNE, TSI_FLAG_PRUNE_EXACT_ONLY) then only loads them.  Of a
+ * chain that may be pruned: its own kernels and, for contexts with prune_live_max > 0, those pruned
+ * by regions (compile_ms: both; cache_hit: both were there).  Cache directory: $TSI_JIT_CACHE, else
+ * $XDG_CACHE_HOME/tsi-jit, else ~/.cache/tsi-jit. */
 int tsi_precompile_tape(const tsi_gpu_instruction *tape, uint32_t n, uint32_t flags, tsi_tape_info *out);
 
-/* The source of the evaluation kernels tsi_precompile_tape / tsi_upload_tape would compile for a
- * tape under these flags, without compiling it (no counterpart in the reference, which interprets
- * the tape): writes min(cap - 1, length) characters and a NUL to out (may be NULL); *len receives
- * the length; *info (may be NULL) the lowering's figures (n, stack, slots, prune_class). */
+/* The source of the evaluation kernels that a tape is compiled to, without compiling it (no
+ * counterpart in the reference, which interprets the tape): with TSI_FLAG_NO_PRUNE a chain's loops
+ * or the straight-line kernels; without it, where the tape is pruned at all, the kernels pruned by
+ * regions (of a chain: those of a context with prune_live_max > 0; other contexts run its loops,
+ * whatever the pruning flags).  Writes min(cap - 1, length) characters and a NUL to out (may be NULL);
+ * *len receives the length; *info (may be NULL) the lowering's figures (n, stack, slots,
+ * prune_class). */
 int tsi_tape_kernel_source(const tsi_gpu_instruction *tape, uint32_t n, uint32_t flags, char *out, size_t cap,
                            size_t *len, tsi_tape_info *info);
 

@@ -44,7 +44,6 @@ struct JitChain {
     struct Class {
         uint32_t rep = 0;             // a segment of it
         std::vector<int> lit;         // per record of the segment: word of the table, -1 = the same in all
-        std::vector<char> ff, pz;     // per record: fix is the identity / the value is never negative, in all
     };
     std::vector<Segment> segs;        // [0]: the base (lo, o only); then upwards
     std::vector<Class> classes;

@@ -41,7 +41,10 @@ __global__ void k_frame_begin(KArgs a) { frame_begin(a, threadIdx.x, blockDim.x)
 
 // The speculative pass's node list (spec_gather, tsi_eval.h): one block.
 __global__ void __launch_bounds__(1024) k_spec_gather(KArgs a) { spec_gather(a, threadIdx.x, blockDim.x); }
-// every parent decided.  Groups with an entry lacking a record run the full program.
+
+// The interpreter's programs of a level, both lists (blockIdx.y): for each group of 8 entries the records
+// that some entry's liveness record keeps, forward and reverse, with each entry's decisions.  Groups with an
+// entry lacking a record run the full program.
 __global__ void __launch_bounds__(256) k_prune(KArgs a, int level) {
     const int which = int(blockIdx.y);
     Counters *cnt = a.cnt;
