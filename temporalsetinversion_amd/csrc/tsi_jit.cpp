@@ -235,8 +235,10 @@ constexpr float kBig = 1000000.0f;   // fix's bound (compute.wgsl:2534)
 
 struct HBound { float lo, hi; bool ok; };
 
-float hmin(float a, float b) { return __builtin_fminimum_numf(a, b); }
-float hmax(float a, float b) { return __builtin_fmaximum_numf(a, b); }
+// (comparisons: the host compiler's __builtin_fminimum_numf and __builtin_fmaximum_numf give the other
+// operand than the named one for values known at run time only; a NaN stays or makes the bound none)
+float hmin(float a, float b) { return a < b ? a : b; }
+float hmax(float a, float b) { return a > b ? a : b; }
 
 HBound hb(float lo, float hi) {
     const bool ok = lo == lo && hi == hi && lo >= -kBig && hi <= kBig;
