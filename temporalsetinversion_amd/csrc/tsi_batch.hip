@@ -348,7 +348,7 @@ int compile_batch(const tsi_gpu_instruction *const *tapes, const uint32_t *lens,
             fwd[i].resize(low[i].nfwd);
             rev[i].resize(low[i].nrev);
             stack_rows = std::max(stack_rows, low[i].stack + 1u);
-            const JitChain chain = jit_chain(copies[i].data(), lens[i], fwd[i], rev[i], low[i]);
+            const JitChain chain = jit_chain(copies[i].data(), lens[i], fwd[i], rev[i], low[i], &kBatchDomain);
             rec_words.push_back(chain.ok() ? chain.record_words : 0u);
             col_words.push_back(chain.ok() ? chain.col_words : 0u);
         }

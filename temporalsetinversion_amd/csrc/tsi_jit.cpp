@@ -346,10 +346,10 @@ uint32_t chain_min_segments() {
 }  // namespace
 
 JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
-                   const std::vector<RevIns> &rev, const Lowered &L) {
+                   const std::vector<RevIns> &rev, const Lowered &L, const JitDomain *domain) {
     JitChain C;
     const uint32_t min_segs = chain_min_segments();
-    if (min_segs == 0 || n < 24) return C;
+    if (min_segs == 0 || n < 24 || !domain) return C;
     auto side = [&](uint32_t j) { return side_of(tape[j]); };
     auto form = [&](uint32_t j) { return j < 4 ? uint32_t(F_COUNT) : uint32_t(fwd[j - 4].form); };
     auto left = [&](uint32_t j) { return larg_of(tape[j]); };
@@ -368,17 +368,21 @@ JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vecto
         if (side(j) == 0 || side(j) == 1) { deps[j] |= deps[left(j)]; if (used[j]) users[left(j)].push_back(j); }
         if (side(j) == 0 || side(j) == 2) { deps[j] |= deps[right(j)]; if (used[j]) users[right(j)].push_back(j); }
     }
-    // every form inclusion-monotone in binary32 (a sub-interval's value lies in the interval's), but
-    // for the transcendental ones, which get checks of their own
+    // Every form inclusion-monotone in binary32 (a sub-interval's value lies in the interval's), but for
+    // sines and cosines, which get checks of their own.  And no value of the domain's that fix would
+    // change: it clamps the two bounds apart, so an interval beyond +-1e6 comes out reversed ([2e6, 3e6] as
+    // [2e6, 1e6]), on which a sub-interval's value may lie outside; a cell inside it then decides
+    // differently.
     std::vector<uint32_t> trans;
+    const std::vector<char> ff = fix_free(tape, n, fwd, *domain);
     for (uint32_t j = 4; j < n; ++j) {
-        if (!used[j] || (side(j) == 0 && left(j) == right(j))) return C;
+        if (!used[j] || !ff[j] || (side(j) == 0 && left(j) == right(j))) return C;
         switch (form(j)) {
         case F_ADD_RR: case F_ADD_RL: case F_SUB_RR: case F_SUB_RL: case F_SUB_LR: case F_MUL_RR: case F_MUL_RL:
         case F_DIV_RL: case F_SQR: case F_SQRT: case F_MIN_RR: case F_MIN_RL: case F_MAX_RR: case F_MAX_RL: case F_NEG:
         case F_ABS: case F_RET: case F_FLOOR: case F_ZERO:
             break;
-        case F_SIN: case F_COS: case F_EXP: case F_LOG: trans.push_back(j); break;
+        case F_SIN: case F_COS: trans.push_back(j); break;
         default: return C;
         }
     }
@@ -847,23 +851,18 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         const int w = C.lit[j - CH.segs[C.rep].lo];
         return w < 0 ? lit(tape[j].literal) : "__uint_as_float(c_.v[" + std::to_string(w) + "])";
     };
-    // the forward expression of record j of class c (that of a global: c < 0)
+    // the forward expression of record j of class c (that of a global: c < 0); a chain's values need no fix
     auto chain_fwd = [&](int c, uint32_t j, const std::string &l, const std::string &r) {
         const uint32_t form = fwd[j - 4].form;
-        bool f = ff[j], z = form == F_SQRT && side_of(tape[j]) == 1 && pz[larg_of(tape[j])];
+        bool z = form == F_SQRT && side_of(tape[j]) == 1 && pz[larg_of(tape[j])];
         std::string lt = lit(tape[j].literal);
         if (c >= 0) {
             const uint32_t at = j - CH.segs[CH.classes[size_t(c)].rep].lo;
             for (const JitChain::Segment &S : CH.segs)
-                if (S.cls == uint32_t(c)) {
-                    f = f && ff[S.lo + at];
-                    z = z && pz[larg_of(tape[S.lo + at])];
-                }
+                if (S.cls == uint32_t(c)) z = z && pz[larg_of(tape[S.lo + at])];
             lt = chain_lit(uint32_t(c), j);
         }
-        const std::string e = z ? "SQRT_NN(" + l + ")"
-                                : "fwd_form_t<true>(" + std::to_string(form) + "u, " + l + ", " + r + ", " + lt + ")";
-        return std::make_pair(f ? e : "fixk(" + e + ", K)", f);
+        return z ? "SQRT_NN(" + l + ")" : "fwd_form_t<true>(" + std::to_string(form) + "u, " + l + ", " + r + ", " + lt + ")";
     };
     // The zero tests of a body's sensitivities and the ops counted with each: a sensitivity passed on
     // as it is (or negated) is zero where its source is, and the counts of such records add up.
@@ -875,7 +874,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
     };
     // one reverse rule: record j, sensitivity s (name), operand names a / b, the derivatives from the
     // operands' values; add(k, product, zero test or empty) receives the contributions
-    auto chain_rule = [&](int c, uint32_t j, const std::string &s, const std::string &a, const std::string &b, bool f_,
+    auto chain_rule = [&](int c, uint32_t j, const std::string &s, const std::string &a, const std::string &b,
                           uint64_t &static_ops, const std::function<void(bool, const std::string &, const std::string &)> &add) {
         const auto &g = tape[j];
         const uint32_t side = side_of(g), form = fwd[j - 4].form;
@@ -906,7 +905,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         } else {
             std::string rule = "rev_form_t<true>(" + std::to_string(form) + "u, " + (side == 0 || side == 1 ? a : b) + ", " +
                                (side == 0 ? b : "ZI") + ", " + lt + ")";
-            if (form == F_SQRT && side == 1 && f_) rule = "Iv2{sqrt_rr_of_value(v" + std::to_string(j) + "), ZI}";
+            if (form == F_SQRT && side == 1 && c >= 0) rule = "Iv2{sqrt_rr_of_value(v" + std::to_string(j) + "), ZI}";
             if (form == F_ABS)
                 rule = "Iv2{sel(" + kc + " == 3u, I(-1.0f, 1.0f), sel(" + kc + " == 2u, I_FROM(-1.0f), ONE)), ZI}";
             else if (rl)
@@ -917,9 +916,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
             // fix of the derivative: as in the straight-line pass (emit_reverse)
             auto d = [&](const char *x) {
                 const std::string e = "d" + J + "." + x;
-                const uint32_t other = x[0] == 'a' ? rarg_of(g) : larg_of(g);
-                if (code || (form == F_MUL_RR && other >= 4u)) return e;
-                if (domain && (form == F_MUL_RR || (form == F_SQR && f_))) return e;
+                if (code || form == F_MUL_RR || (form == F_SQR && c >= 0)) return e;
                 return "fixk(" + e + ", K)";
             };
             ca = "MUL_II(" + d("a") + ", " + s + ")";
@@ -981,14 +978,14 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         // ---- forward ----
         o += "template <bool PUSH>\n__device__ __noinline__ FwdOut tape_forward(Iv v0, Iv v1, Iv v2, Iv v3, float2 *stk_, uint32_t lane, "
              "const uint32_t *lrec, uint32_t cap, uint32_t *cols, RegionMask mask, bool act) {\n"
-             "    gfloat2 *stk = (gfloat2 *)stk_;\n    const Iv ZI = I_FROM(0.0f);\n    const FixK K = fix_consts();\n";
+             "    gfloat2 *stk = (gfloat2 *)stk_;\n    const Iv ZI = I_FROM(0.0f);\n";
         for (uint32_t k = 0; k + 1 < n; ++k) {
             if (k >= 4 && CH.seg[k] >= 0) break;
             if (k >= 4) {
                 const uint32_t side = side_of(tape[k]);
                 const std::string l = (side == 0 || side == 1) ? V(larg_of(tape[k])) : "ZI";
                 const std::string r = (side == 0 || side == 2) ? V(rarg_of(tape[k])) : "ZI";
-                o += "    const Iv " + V(k) + " = " + chain_fwd(-1, k, l, r).first + ";\n";
+                o += "    const Iv " + V(k) + " = " + chain_fwd(-1, k, l, r) + ";\n";
             }
             if (CH.row[k] >= 0) o += "    if (PUSH) " + row(uint32_t(CH.row[k])) + " = make_float2(" + V(k) + ".lo, " + V(k) + ".hi);\n";
         }
@@ -1044,7 +1041,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                 const uint32_t side = side_of(tape[j]);
                 const std::string l = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
                 const std::string r = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
-                o += "        const Iv " + V(j) + " = " + chain_fwd(int(c), j, l, r).first + ";\n";
+                o += "        const Iv " + V(j) + " = " + chain_fwd(int(c), j, l, r) + ";\n";
             }
             if (!base) {
                 const std::string l = nm(larg_of(tape[R.choice])), r = nm(rarg_of(tape[R.choice]));
@@ -1070,7 +1067,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
              "        if (cols) cols[(" + std::to_string(2 * X) + "u + w) * 64u] = np;\n"
              "        live = lane == w ? lw : live;\n    }\n"
              "    if (cols) cols[" + std::to_string((2 * X + W) * 64u) + "u] = tp;\n";
-        o += "    return FwdOut{" + chain_fwd(-1, n - 1, "cur", "ZI").first + ", cost, records, live, rows};\n}\n\n";
+        o += "    return FwdOut{" + chain_fwd(-1, n - 1, "cur", "ZI") + ", cost, records, live, rows};\n}\n\n";
         if (!rev_kernel) return;
         // ---- reverse ----
         o += "__device__ __noinline__ RevOut tape_reverse(const float2 *stk_, uint32_t lane, uint32_t live, uint32_t rows, bool act) {\n"
@@ -1090,7 +1087,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
         for (uint32_t j = 4; j < n; ++j)
             if (CH.seg[j] >= 0 && !single_use(rev[(n - 1) - j], side_of(tape[j]))) static_ops += rev[(n - 1) - j].cost;
         o += "    Iv s = ZI;\n    {\n";
-        chain_rule(-1, n - 1, "ONE", "ZI", "ZI", false, static_ops,
+        chain_rule(-1, n - 1, "ONE", "ZI", "ZI", static_ops,
                    [&](bool, const std::string &e, const std::string &) { o += "        s = " + e + ";\n"; });
         o += "    }\n    // segments decided for p in every cell pass the sensitivity on: their ops, where it is not zero\n"
              "    auto through = [&](uint32_t hi, uint32_t lo) { ops += s.lo == 0.0f && s.hi == 0.0f ? 0u : kThrough[hi] - kThrough[lo]; };\n"
@@ -1114,14 +1111,12 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
             const bool base = CH.classes[c].rep == 0;
             const auto nm = chain_names(c);
             o += "            case " + std::to_string(c) + "u: {\n";
-            std::vector<char> f(R.o - R.lo + 1, 0), live(n, 0);
+            std::vector<char> live(n, 0);
             for (uint32_t j = R.lo; j <= R.o; ++j) {
                 const uint32_t side = side_of(tape[j]);
                 const std::string l = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
                 const std::string r = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
-                const auto e = chain_fwd(int(c), j, l, r);
-                f[j - R.lo] = e.second;
-                o += "        const Iv " + V(j) + " = " + e.first + ";\n";
+                o += "        const Iv " + V(j) + " = " + chain_fwd(int(c), j, l, r) + ";\n";
                 if (j != R.o) o += "        Iv " + S(j) + " = ZI;\n";
             }
             if (!base) o += "        Iv sp = ZI;\n";
@@ -1138,7 +1133,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
                 const uint32_t side = side_of(tape[j]);
                 const std::string a = (side == 0 || side == 1) ? nm(larg_of(tape[j])) : "ZI";
                 const std::string b = (side == 0 || side == 2) ? nm(rarg_of(tape[j])) : "ZI";
-                chain_rule(int(c), j, j == R.o ? "s" : S(j), a, b, f[j - R.lo], static_ops,
+                chain_rule(int(c), j, j == R.o ? "s" : S(j), a, b, static_ops,
                            [&](bool first, const std::string &e, const std::string &z) {
                                const uint32_t k = first ? larg_of(tape[j]) : rarg_of(tape[j]);
                                const bool isp = !base && k == R.p;
@@ -1165,7 +1160,7 @@ std::string jit_source(const tsi_gpu_instruction *tape, uint32_t n, const std::v
             const uint32_t side = side_of(tape[j]);
             const std::string a = (side == 0 || side == 1) ? (CH.row[larg_of(tape[j])] >= 0 ? V(larg_of(tape[j])) : "ZI") : "ZI";
             const std::string b = (side == 0 || side == 2) ? (CH.row[rarg_of(tape[j])] >= 0 ? V(rarg_of(tape[j])) : "ZI") : "ZI";
-            chain_rule(-1, j, S(j), a, b, false, static_ops,
+            chain_rule(-1, j, S(j), a, b, static_ops,
                        [&](bool first, const std::string &e, const std::string &z) {
                            const uint32_t k = first ? larg_of(tape[j]) : rarg_of(tape[j]);
                            std::string v = "ADD_II(" + e + ", " + S(k) + ")";
@@ -1867,7 +1862,7 @@ std::string module_body(const std::string &src) {
 
 std::string jit_source_level(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
                              const std::vector<RevIns> &rev, const Lowered &L, bool prune, const JitDomain *domain) {
-    const JitChain chain = prune ? JitChain() : jit_chain(tape, n, fwd, rev, L);
+    const JitChain chain = prune ? JitChain() : jit_chain(tape, n, fwd, rev, L, domain);
     const std::string f = jit_source(tape, n, fwd, rev, L, false, prune, domain, true, 0, &chain);
     const std::string r = jit_source(tape, n, fwd, rev, L, true, prune, domain, true, 0, &chain);
     std::string o = "// generated by tsi_jit.cpp: straight-line evaluation of one tape, both lists of a level\n";
@@ -1907,7 +1902,7 @@ std::string jit_source_batch(const std::vector<BatchTape> &tapes, const JitDomai
         // (with 64: 611 against 643 frames/s batched, served p50 2.01 against 1.80 ms)
         const bool skip = batch_skip();
         const uint32_t group = batch_region_records();
-        const JitChain chain = jit_chain(t.tape, t.n, *t.fwd, *t.rev, *t.low);
+        const JitChain chain = jit_chain(t.tape, t.n, *t.fwd, *t.rev, *t.low, domain);
         const std::string f = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, false, false, domain, skip, group, &chain);
         const std::string r = jit_source(t.tape, t.n, *t.fwd, *t.rev, *t.low, true, false, domain, skip, group, &chain);
         o += "namespace tb" + std::to_string(i) + " {\nnamespace jf {   // forward-only list\n" + module_body(f);

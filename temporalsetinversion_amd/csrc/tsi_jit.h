@@ -49,7 +49,7 @@ struct JitChain {
     std::vector<Class> classes;
     std::vector<int> seg;             // per record: its segment, -1 = global (and the final RET)
     std::vector<int> row;             // per record: its saved-operand row (globals read by rules or segments)
-    std::vector<uint32_t> x_records;  // sin / cos / exp / log of the cell's position: not monotone to the ulp,
+    std::vector<uint32_t> x_records;  // sin / cos of the cell's position: not monotone to the ulp,
                                       // so a cell checks that its values lie inside its parent's
     bool exact_t = false;             // some depend on t alone: the t-windows must be equal
     bool finite = false;              // no sensitivity can overflow (see jit_chain)
@@ -58,8 +58,6 @@ struct JitChain {
     uint32_t words = 0, record_words = 0, col_words = 0;
     bool ok() const { return !segs.empty(); }
 };
-JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
-                   const std::vector<RevIns> &rev, const Lowered &L);
 
 // The domain a tape's kernels may be specialised for: every cell box inside `box` (lo xyz, hi
 // xyz), every t-window inside [t0, t1].  fix_free marks the records whose value no cell in it can
@@ -67,6 +65,11 @@ JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vecto
 struct JitDomain { float box[6]; float t0, t1; };
 std::vector<char> fix_free(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
                            const JitDomain &d);
+
+// The chain of a tape whose cells stay in `domain` (none without one: what a cell's parents decided holds
+// in the cell only where no value is clamped, see jit_chain).
+JitChain jit_chain(const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
+                   const std::vector<RevIns> &rev, const Lowered &L, const JitDomain *domain);
 
 // HIP source of the code of one list for one tape: the forward-only frontier list, or
 // (rev_kernel) forward with saved operands, then reverse; with a kernel of its own

@@ -167,7 +167,8 @@ struct tsi_ctx {
     uint32_t last_tslot = 0;   // the slot of the last trace issued: the frame read back
     // the domain the loaded tape kernels are specialised for (they leave out fix where it is the
     // identity there), the root box of the last reset and the t-windows seen since
-    bool jit_specialized = false;
+    bool jit_specialized = false;               // for jit_domain
+    JitDomain jit_domain{};
     float root_box[6] = {-5.0f, -5.0f, -5.0f, 5.0f, 5.0f, 5.0f};
     float t_seen_lo = 1.0f, t_seen_hi = 0.0f;   // empty
 };
@@ -369,15 +370,15 @@ void release_jit(tsi_ctx *c) {
 // Compiles (or finds cached) the tape's two level kernels and loads them on this device.
 // The root box of the reference (main.rs) and a t-range around the frame loop's times (about a
 // minute of frames at 1/60): the tape kernels are compiled for it, and recompiled without that
-// assumption if a frame leaves it.
+// assumption (a chain's for a wider domain) if a frame leaves it.
 const JitDomain kDefaultDomain{{-5.0f, -5.0f, -5.0f, 5.0f, 5.0f, 5.0f}, -2.0f, 64.0f};
 
 // The generated module addresses no stack row, liveness-record word or choice column beyond what
 // alloc_prune and tsi_upload_tape allocate (a module that would is refused, not run).
 int check_module(const std::string &src, const tsi_gpu_instruction *tape, uint32_t n, const std::vector<FwdIns> &fwd,
-                 const std::vector<RevIns> &rev, const Lowered &L, std::string &log) {
+                 const std::vector<RevIns> &rev, const Lowered &L, const JitDomain *domain, std::string &log) {
     const JitLayout Y = jit_layout(fwd, L, true);
-    const JitChain chain = jit_chain(tape, n, fwd, rev, L);
+    const JitChain chain = jit_chain(tape, n, fwd, rev, L, domain);
     const std::string bad =
         jit_check_bounds(src, L.stack + 1u, Y.record_words, Y.mode_words, chain.record_words, chain.col_words);
     if (bad.empty()) return TSI_OK;
@@ -396,7 +397,7 @@ int load_jit(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n, const std:
     int rc = TSI_OK;
     try {
         src = jit_source_level(tape, n, fwd, rev, L, c->prune, domain);
-        rc = check_module(src, tape, n, fwd, rev, L, log);
+        rc = check_module(src, tape, n, fwd, rev, L, domain, log);
         if (rc == TSI_OK) rc = jit_compile(src, c->prune, code, log, hit, ms);
     } catch (const std::runtime_error &) {   // the generator cannot lay out this tape
         return TSI_E_JIT;
@@ -417,6 +418,7 @@ int load_jit(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n, const std:
         return TSI_E_HIP;
     }
     c->jit_specialized = domain != nullptr;
+    if (domain) c->jit_domain = *domain;
     c->info.specialized = domain ? 1u : 0u;
     c->info.fix_kept = n - 4u;
     if (domain) {
@@ -728,7 +730,7 @@ int tsi_upload_tape(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n) {
     release_prune(c);
     JitChain chain;
     try {
-        if (!(c->p.flags & TSI_FLAG_INTERPRET)) chain = jit_chain(tape, n, fwd, rev, L);
+        if (!(c->p.flags & TSI_FLAG_INTERPRET)) chain = jit_chain(tape, n, fwd, rev, L, &kDefaultDomain);
     } catch (...) {
         return TSI_E_OOM;
     }
@@ -786,34 +788,62 @@ int tsi_enqueue_root(tsi_ctx *c) {
 
 namespace {
 
+bool in_domain(const tsi_ctx *c, const JitDomain &d) {
+    bool inside = c->t_seen_lo >= d.t0 && c->t_seen_hi <= d.t1;
+    for (int k = 0; k < 3; ++k)
+        inside = inside && c->root_box[k] >= d.box[k] && c->root_box[3 + k] <= d.box[3 + k] &&
+                 c->root_box[k] <= c->root_box[3 + k];
+    return inside;
+}
+
+// A domain with the root box and the times seen: times up to a power of four times the default's, so that an
+// animation that goes on rebuilds rarely.
+JitDomain wider_domain(const tsi_ctx *c) {
+    JitDomain d = kDefaultDomain;
+    for (int k = 0; k < 3; ++k) {
+        d.box[k] = std::fmin(d.box[k], c->root_box[k]);
+        d.box[3 + k] = std::fmax(d.box[3 + k], c->root_box[3 + k]);
+    }
+    while (d.t0 > c->t_seen_lo && d.t0 > -1e6f) d.t0 *= 4.0f;
+    while (d.t1 < c->t_seen_hi && d.t1 < 1e6f) d.t1 *= 4.0f;
+    return d;
+}
+
 // Every cell box lies in the root box and every t-window in the span of the frames' times since
 // the reset (each swept window reaching swept_window below its frame's time): when these leave
-// the domain the kernels were specialised for, the kernels are rebuilt without the assumption.
+// the domain the kernels were specialised for, the kernels are rebuilt without the assumption;
+// those of a chain, which need one, for a wider domain if the tape is a chain there.
 int keep_domain(tsi_ctx *c) {
     const float t = c->u.time;
-    const float lo = c->p.swept_volume ? t - c->p.swept_window : t;
+    const float from = c->p.swept_volume ? t - c->p.swept_window : t;
+    const float lo = from <= t ? from : t, hi = from <= t ? t : from;
     if (c->t_seen_lo > c->t_seen_hi) {
         c->t_seen_lo = lo;
-        c->t_seen_hi = t;
+        c->t_seen_hi = hi;
     } else {
         c->t_seen_lo = std::fmin(c->t_seen_lo, lo);
-        c->t_seen_hi = std::fmax(c->t_seen_hi, t);
+        c->t_seen_hi = std::fmax(c->t_seen_hi, hi);
     }
-    if (!c->jit_specialized) return TSI_OK;
-    const JitDomain &d = kDefaultDomain;
-    bool inside = c->t_seen_lo >= d.t0 && c->t_seen_hi <= d.t1;
-    for (int k = 0; k < 3; ++k) inside = inside && c->root_box[k] >= d.box[k] && c->root_box[3 + k] <= d.box[3 + k];
-    if (inside) return TSI_OK;
+    if (!c->jit_specialized || in_domain(c, c->jit_domain)) return TSI_OK;
     HIP_OK(hipStreamSynchronize(c->stream));   // frames in flight use the loaded kernels
     for (auto &t : c->tslot) HIP_OK(hipStreamSynchronize(t.stream));
     std::vector<FwdIns> fwd;
     std::vector<RevIns> rev;
     Lowered L;
-    int rc = lower(c->tape.data(), uint32_t(c->tape.size()), fwd, rev, L);
-    if (rc) return rc;
-    fwd.resize(L.nfwd);
-    rev.resize(L.nrev);
-    return load_jit(c, c->tape.data(), uint32_t(c->tape.size()), fwd, rev, L, nullptr);
+    const uint32_t n = uint32_t(c->tape.size());
+    const JitDomain wider = wider_domain(c);
+    bool chain = false;
+    try {
+        const int rc = lower(c->tape.data(), n, fwd, rev, L);
+        if (rc) return rc;
+        fwd.resize(L.nfwd);
+        rev.resize(L.nrev);
+        chain = !c->prune && in_domain(c, wider) && jit_chain(c->tape.data(), n, fwd, rev, L, &wider).ok();
+    } catch (...) {
+        return TSI_E_OOM;
+    }
+    if (!chain && c->chain) release_prune(c);   // a chain's records
+    return load_jit(c, c->tape.data(), n, fwd, rev, L, chain ? &wider : nullptr);
 }
 
 }  // namespace
@@ -1162,12 +1192,12 @@ int tsi_precompile_tape(const tsi_gpu_instruction *tape, uint32_t n, uint32_t fl
             const std::vector<char> ff = fix_free(tape, n, fwd, kDefaultDomain);
             for (uint32_t j = 4; j < n; ++j) info.fix_kept -= ff[j] ? 1u : 0u;
             // a chain's kernels, and the pruned module that prune_live_max selects
-            const bool both = prune && chain_wanted(flags, 0, L, jit_chain(tape, n, fwd, rev, L));
+            const bool both = prune && chain_wanted(flags, 0, L, jit_chain(tape, n, fwd, rev, L, &kDefaultDomain));
             info.cache_hit = 1;
             for (int k = both ? 0 : 1; k < 2 && rc == TSI_OK; ++k) {
                 const bool pruned = prune && k == 1;
                 src = jit_source_level(tape, n, fwd, rev, L, pruned, &kDefaultDomain);
-                rc = check_module(src, tape, n, fwd, rev, L, log);
+                rc = check_module(src, tape, n, fwd, rev, L, &kDefaultDomain, log);
                 if (rc == TSI_OK) rc = jit_compile(src, pruned, code, log, hit, ms);
                 info.compile_ms += ms;
                 info.cache_hit = info.cache_hit && hit;
