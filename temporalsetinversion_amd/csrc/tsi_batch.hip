@@ -589,7 +589,8 @@ int tsi_batch_submit(tsi_batch *b, const tsi_frame_req *reqs, uint32_t n) {
         const Session &s = b->sessions[r.session];
         // the kernels' domain: t-windows inside [-2, 64]
         const float lo = s.p.swept_volume ? r.time - s.p.swept_window : r.time;
-        if (!(lo >= kBatchDomain.t0 && r.time <= kBatchDomain.t1)) return TSI_E_ARG;
+        if (!(std::fmin(lo, r.time) >= kBatchDomain.t0 && std::fmax(lo, r.time) <= kBatchDomain.t1 && r.time == r.time))
+            return TSI_E_ARG;
         if (size_t(r.width) * r.height > s.px_cap) return TSI_E_ARG;
         levels = std::max(levels, s.p.localsubdiv);
     }

@@ -105,3 +105,23 @@ def test_root_boxes_that_leave_the_domain():
     boxes = [(-5, -5, -5, 5, 5, 5), (-7, -1, -1, 1, 1, 1), (-1, -1, -1, 1, 1, 1), (1, -1, -1, -1, 1, 1), (-3e3, -1, -1, 3e3, 1, 1)]
     got = _compare(tape, [0.0, 0.1, 0.2, 0.25, 0.3], boxes)
     assert [i["specialized"] for _, _, i in got] == [1, 1, 1, 0, 0]
+
+
+@pytest.mark.gpu
+def test_batched_windows_that_leave_the_domain():
+    """A swept window reaches from the frame's time to swept_window before it; one of negative length, after it."""
+    from temporalsetinversion_amd.batch import Batch
+    tapes = [T.tape_from_ll(x) for x in scenes.batch_test_sets()["one"]]
+    with Batch(tapes, arena_bytes=64 << 20, max_sessions=2) as b:
+        kw = dict(tape=0, localsubdiv=4, voxel_capacity=1 << 16, max_width=16, max_height=16, swept_volume=True)
+        before, after = b.open(swept_window=10.0, **kw), b.open(swept_window=-10.0, **kw)
+        for sid, t, inside in ((before, 64.0, True), (before, 64.1, False), (before, 7.9, False), (before, 8.0, True),
+                               (after, 54.0, True), (after, 54.1, False), (after, -2.0, True), (after, -2.1, False),
+                               (before, float("nan"), False)):
+            if inside:
+                (r,), _, _ = b.run([(sid, t, 0, 0, None)])
+                assert r["status"] == 0
+            else:
+                with pytest.raises(T.TsiError) as e:
+                    b.run([(sid, t, 0, 0, None)])
+                assert e.value.code == -6                 # TSI_E_ARG
