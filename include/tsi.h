@@ -260,7 +260,8 @@ typedef struct {
     uint32_t engine;              /* 0 interpreter, 1 compiled kernels */
     uint32_t cache_hit;           /* compiled kernels came from the code-object cache */
     uint32_t specialized;         /* the kernels assume every cell box inside [-5,5]^3 and every
-                                     t-window inside [-2, 64] (rebuilt without it otherwise) */
+                                     t-window inside [-2, 64] (rebuilt without it otherwise; a
+                                     chain's for a wider domain while it is a chain there) */
     uint32_t fix_kept;            /* records whose fix is evaluated (the rest provably never clamp) */
     double compile_ms;            /* hiprtc compile (or cache lookup) wall time */
     char log[1024];               /* compiler log of a failed compile (truncated) */

@@ -698,6 +698,8 @@ int tsi_upload_tape(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n) {
     }
     if (rc != TSI_OK) return rc;
     HIP_OK(hipStreamSynchronize(c->stream));
+    // from here on the previous tape's buffers go: until the new one's are all there, the context has none
+    c->have_tape = false;
     dfree(c->fprog);
     dfree(c->rprog);
     // zero padding records: the interpreter fetches program records ahead of execution
@@ -742,10 +744,7 @@ int tsi_upload_tape(tsi_ctx *c, const tsi_gpu_instruction *tape, uint32_t n) {
     c->info.slots = L.slots;
     c->info.prune_class = uint32_t(L.prune_class);
     if (!(c->p.flags & TSI_FLAG_INTERPRET)) {
-        if ((rc = load_jit(c, tape, n, fwd, rev, L, &kDefaultDomain))) {
-            c->have_tape = false;
-            return rc;
-        }
+        if ((rc = load_jit(c, tape, n, fwd, rev, L, &kDefaultDomain))) return rc;
         c->info.engine = 1;
         if (use_chain) {
             alloc_chain(c, chain);
@@ -843,7 +842,9 @@ int keep_domain(tsi_ctx *c) {
         return TSI_E_OOM;
     }
     if (!chain && c->chain) release_prune(c);   // a chain's records
-    return load_jit(c, c->tape.data(), n, fwd, rev, L, chain ? &wider : nullptr);
+    const int rc = load_jit(c, c->tape.data(), n, fwd, rev, L, chain ? &wider : nullptr);
+    if (rc) c->have_tape = false;   // (its kernels are gone, and the interpreter's buffers were never there)
+    return rc;
 }
 
 }  // namespace

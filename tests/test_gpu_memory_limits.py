@@ -1,10 +1,10 @@
 """Records of chain tapes only save work: where device memory is nearly spent they give way to what a batch's
 or a context's calls need, and the results are the same without them."""
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
-import torch
 
 import temporalsetinversion_amd as T
 from temporalsetinversion_amd import scenes
@@ -16,22 +16,40 @@ MIB = 1 << 20
 VIEW = T.look_at_inverse((2.2, 1.7, 2.6))
 
 
+def _free_now():
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert T.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0   # (of the runtime that the library is bound to)
+    return free.value
+
+
 def _free():
     """Free device memory, once it has not changed for a second (the driver clears what is given back first)."""
-    torch.cuda.empty_cache()
-    seen = [torch.cuda.mem_get_info()[0]]
-    while len(seen) < 6 or len(set(seen[-6:])) > 1:
+    seen = [_free_now()]
+    while (len(seen) < 6 or len(set(seen[-6:])) > 1) and len(seen) < 100:
         time.sleep(0.2)
-        seen.append(torch.cuda.mem_get_info()[0])
+        seen.append(_free_now())
     return seen[-1]
 
 
-def _hold_all_but(rest):
-    """Allocations that leave at most `rest` bytes and 8 MiB free (in a list that the caller clears)."""
-    held = []
-    while (extra := _free() - rest) > 8 * MIB:
-        held.append(torch.empty(extra - 4 * MIB, dtype=torch.uint8, device="cuda"))
-    return held
+class _HoldAllBut:
+    """Allocations that leave at most `rest` bytes and 8 MiB free."""
+
+    def __init__(self, rest):
+        self.held = []
+        for _ in range(20):
+            extra = _free() - rest
+            if extra <= 8 * MIB:
+                break
+            p = C.c_void_p()
+            assert T.lib().hipMalloc(C.byref(p), C.c_size_t(extra - 4 * MIB)) == 0
+            self.held.append(p)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        for p in self.held:
+            T.lib().hipFree(p)
 
 
 def _state(**kw):
@@ -85,13 +103,9 @@ def test_frame_that_needs_the_records_memory(sizes, overlap):
     print(f"{records >> 20} MiB of records, {room >> 20} free, a frame of {WIDTH}x{height}", flush=True)
     with _state() as st:
         want = _frames(st, overlap, height)
-    held = _hold_all_but(base + room)
-    try:
+    with _HoldAllBut(base + room):
         with _state(prune_capacity=ENTRIES) as st:
             got = _frames(st, overlap, height)
-    finally:
-        held.clear()
-        torch.cuda.empty_cache()
     assert got == want
 
 
